@@ -277,18 +277,35 @@ void ideal_workspace(const mf_config *cfg, i64 n, i64 m, i64 p, i64 *xbytes, i64
     *wbytes = align256((p * cfg->cols + 31) / 32 * G * 8);
 }
 
+bool plain_read(const mf_config *cfg) {
+    return !cfg->has_vnoise && !(cfg->has_read && cfg->read_mode != MF_READ_SHARED);
+}
+// Reads that k_noisy_block (noisy_block.hip) takes: 64-row reads with more input slices than
+// k_noisy's registers hold, and 128-row reads, where the converters' arguments stay by whole
+// counts (linear converters, programming noise and stuck-at faults alone).
+bool block_read(const mf_config *cfg) {
+    return (cfg->read_rows == 64 && cfg->n_in > 5) || cfg->read_rows == 128;
+}
+bool whole_counts(const mf_config *cfg) {
+    return !cfg->has_vnoise && !cfg->has_read && !cfg->has_nonlinear && !cfg->has_drift;
+}
+
 // Whether every conductance term k1[w] * (g - L) fits fp16 with margin.  The
 // sampled normals are sqrt(-2 ln u) cos(2 pi v) with u >= 2^-25, so |z| < 5.9;
 // programming and shared read noise multiply g by at most exp(5.9 sigma) each,
 // drift by the drift factor, and stuck-at faults set L or H.
-bool fp16_terms_fit(const mf_config *cfg) {
+double largest_delta(const mf_config *cfg) {
     const double zmax = 5.9;
     double high = cfg->f_high;
     if (cfg->has_write) high *= std::exp(zmax * double(cfg->f_write));
     if (cfg->has_read) high *= std::exp(zmax * double(cfg->f_read));
     if (cfg->has_drift && cfg->f_drift > 1.0f) high *= double(cfg->f_drift);
     const double low = cfg->f_low;
-    const double span = std::max(high - low, low);   // |g - L| for g in [0, high]
+    return std::max(high - low, low);   // |g - L| for g in [0, high]
+}
+
+bool fp16_terms_fit(const mf_config *cfg) {
+    const double span = largest_delta(cfg);
     for (int w = 0; w < cfg->n_w; ++w) {
         const double k1 = double(float(cfg->d_voltage * double(cfg->w_mask[w]) * cfg->d_inv_unit));
         if (!(k1 * span < 16384.0)) return false;
@@ -320,11 +337,18 @@ bool build_noisy_plan(const mf_config *cfg, i64 m, i64 p, NoisyPlan *plan, int *
         for (int a = 0; a < cfg->n_in; ++a)
             if (cfg->in_mask[a] > 15) { *why = "output-mode read noise with input digits above 15"; return false; }
     }
-    if ((cfg->read_rows != 32 && cfg->read_rows != 64) || cfg->rows % cfg->read_rows) {
-        *why = "rows_per_read must be 32 or 64 and divide the array rows";
+    if ((cfg->read_rows != 32 && cfg->read_rows != 64 && cfg->read_rows != 128) ||
+        cfg->rows % cfg->read_rows) {
+        *why = "rows_per_read must be 32, 64 or 128 and divide the array rows";
         return false;
     }
-    if (cfg->read_rows == 64 && cfg->n_in > 5) { *why = "more than 5 input slices at 64-row reads"; return false; }
+    // Elsewhere an argument may lie anywhere between two counts, and the general read's order
+    // of FP32 sums decides which way the closest ones round: those reads keep it.
+    if (block_read(cfg) && !whole_counts(cfg)) {
+        *why = "more than 5 input slices at 64-row reads, or 128-row reads, with read noise, "
+               "drift or nonlinear converters";
+        return false;
+    }
     if (cfg->n_in > 8 || cfg->n_w > 8) { *why = "too many slices"; return false; }
     const i64 G = m * cfg->reads;
     if (G >= 4096) { *why = "more than 4095 reads per output"; return false; }
@@ -368,7 +392,20 @@ bool build_noisy_plan(const mf_config *cfg, i64 m, i64 p, NoisyPlan *plan, int *
             const int f = int(plan->fa[a] * plan->fw[w]);
             plan->f24[a][w] = u32(int(u32(f) << 8) >> 8);
         }
-    for (int w = 0; w < cfg->n_w; ++w) plan->top_magic[w] = 12582912.0f + plan->top[w];
+    for (int w = 0; w < cfg->n_w; ++w) {
+        plan->magic[w] = 12582912.0f;
+        plan->top_magic[w] = 12582912.0f + plan->top[w];
+        if (!block_read(cfg)) continue;
+        // Terms as large as fp16 takes (below 2^14): the power of two is exact in k1 and in
+        // the converter's constants.  It is an even power, so that the exponent of
+        // the rounding constant keeps a clear low bit, the top one of the 24 that are added.
+        double scale = 1.0;
+        while (double(plan->k1[w]) * largest_delta(cfg) * scale * 4.0 < 16384.0 && scale < 4096.0)
+            scale *= 4.0;
+        plan->k1[w] *= float(scale);
+        plan->magic[w] *= float(scale);
+        plan->top_magic[w] *= float(scale);
+    }
     *ks = cfg->read_rows / 16;
     return true;
 }
@@ -393,6 +430,47 @@ i64 noisy_terms_bytes(const mf_config *cfg, i64 m, i64 p) {
     return (p * cfg->cols + 63) / 64 * 2 * noisy_block_bytes(cfg, m);
 }
 
+// Whether a split noisy read runs k_noisy_pairs (one wave per weight slice, 32 vectors):
+// batches of at most 32 vectors, where the four-wave tile (64 vectors, the slices one
+// after another) would leave half its waves idle; plain and S-curve reads (no voltage,
+// slice_pair or output-mode noise).
+bool noisy_small_tile(const mf_config *cfg, i64 n) { return n <= 32 && plain_read(cfg); }
+
+// The same for a read of k_noisy_block's, which keeps a wave on all pairs of slices: a wave per
+// weight slice is faster up to 12 such waves per SIMD (default Config, 1024 x 1024 weights: 64
+// vectors, 8 waves, 23 against 30 us; 128 vectors, 16 waves, 40 against 37).
+bool pairs_read(const mf_config *cfg, i64 n, i64 m, i64 p) {
+    if (noisy_small_tile(cfg, n)) return true;
+    const i64 tiles = (p * cfg->cols + 31) / 32 * ((n + 31) / 32);
+    return block_read(cfg) && tiles * m * cfg->reads * cfg->n_w <= 12 * 1024;
+}
+
+// Waves per workgroup of k_noisy_block: 32 columns each, four where there are as many.
+int block_waves(i64 cols) { return cols > 96 ? 4 : int((cols + 31) / 32); }
+
+// Read chunks of k_noisy_block.  A tile's read (32 x 32 outputs of one read, one wave) takes one
+// unit of a SIMD's time where another wave fills its gaps and 1.6 units alone, so a chunk of s
+// reads takes s * max(1.6, waves per SIMD).  Splitting writes and reads back 8 bytes per output
+// and read: 2e-4 units per tile for eight by eight slices of 64 rows (10 us), more for less work.
+i64 block_split(const mf_config *cfg, i64 n, i64 G, i64 cols) {
+    constexpr i64 SIMDS = 1024;
+    const i64 tiles = (cols + 31) / 32 * ((n + 31) / 32);
+    const double traffic = 2e-4 * double(tiles) * double(G) * 256.0 /
+                           (double(cfg->n_in) * cfg->n_w * (cfg->read_rows / 16));
+    i64 best = 1;
+    double least = 0.0;
+    for (i64 z = 1; z <= G; ++z) {
+        const double waves = double((tiles * z + SIMDS - 1) / SIMDS);
+        const double cost =
+            double((G + z - 1) / z) * std::max(1.6, waves) + (z > 1 ? traffic : 0.0);
+        if (z == 1 || cost < least) {
+            least = cost;
+            best = z;
+        }
+    }
+    return best;
+}
+
 // Read chunks of a split read (1: not split).  `requested` (the variant's
 // split field) overrides the automatic choice: 1 never splits, s >= 2 splits
 // into s chunks (at most one per read).
@@ -401,6 +479,8 @@ i64 noisy_split(const mf_config *cfg, i64 n, i64 m, i64 p, int requested = 0) {
     i64 z;
     if (requested > 0) {
         z = requested;
+    } else if (block_read(cfg)) {
+        z = pairs_read(cfg, n, m, p) ? G : block_split(cfg, n, G, p * cfg->cols);
     } else {
         const i64 blocks = (p * cfg->cols + 63) / 64 * ((n + 63) / 64);
         if (G < 2 || blocks >= NOISY_SPLIT_BELOW) return 1;
@@ -432,16 +512,6 @@ i64 noisy_voltage_bytes(const mf_config *cfg, i64 n, i64 m) {
     return cfg->has_vnoise ? align256(voltage_terms(cfg) * i64(cfg->n_in) * vectors * m *
                                       cfg->rows * 2)
                            : 0;
-}
-
-// Whether a split noisy read runs k_noisy_pairs (one wave per weight slice, 32 vectors):
-// batches of at most 32 vectors, where the four-wave tile (64 vectors, the slices one
-// after another) would leave half its waves idle; plain and S-curve reads (no voltage,
-// slice_pair or output-mode noise).
-bool noisy_small_tile(const mf_config *cfg, i64 n) {
-    const bool per_read_noise = cfg->has_vnoise ||
-                                (cfg->has_read && cfg->read_mode != MF_READ_SHARED);
-    return n <= 32 && !per_read_noise;
 }
 
 // Fields of the `variant` word (include/memfast_hip.h).
@@ -512,8 +582,11 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
         } else if (ks == 2) {
             hipLaunchKernelGGL(k_split_conductances<2>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
                                packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
-        } else {
+        } else if (ks == 4) {
             hipLaunchKernelGGL(k_split_conductances<4>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+                               packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
+        } else {
+            hipLaunchKernelGGL(k_split_conductances<8>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
                                packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         }
         NoisyArgs args{};
@@ -548,12 +621,16 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
         }
         const bool nl = cfg->has_nonlinear != 0;
         const bool slice = plan.planes > 1 && !plan.out_noise;
-        // A split read of at most 32 vectors runs k_noisy_pairs: one read per workgroup,
-        // one wave per weight slice.
-        const bool pairs = use_split && noisy_small_tile(cfg, n);
+        // A small split read runs k_noisy_pairs: one read per workgroup, one wave per weight
+        // slice.
+        const bool pairs = use_split && pairs_read(cfg, n, m, p);
+        const bool wide_block = block_read(cfg) && !pairs;
+        const int waves = block_waves(cols);
         const dim3 grid = pairs ? dim3{unsigned(CB), unsigned((n + 31) / 32), unsigned(g_run)}
-                                : dim3{unsigned((n + 63) / 64), unsigned(CB / 2), gz};
-        const dim3 block{pairs ? unsigned(64 * cfg->n_w) : 256u};
+                          : wide_block ? dim3{unsigned((n + 31) / 32),
+                                              unsigned((cols + 32 * waves - 1) / (32 * waves)), gz}
+                                       : dim3{unsigned((n + 63) / 64), unsigned(CB / 2), gz};
+        const dim3 block{pairs ? unsigned(64 * cfg->n_w) : wide_block ? unsigned(64 * waves) : 256u};
         if (pairs) {
             args.g_step = 1;
             args.restored = 1;   // the values (float(T) * xs) * ws; consumers only sum them
@@ -581,9 +658,18 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
         else if (slice) MF_NOISY_LAUNCH2(KS, NA, false, true, false)                          \
         else MF_NOISY_LAUNCH2(KS, NA, false, false, false)                                    \
     }
-        if (ks == 4) MF_NOISY_LAUNCH(4, 5)
+#define MF_BLOCK_LAUNCH(KS)                                                                     \
+    if (pairs) hipLaunchKernelGGL((k_noisy_pairs<KS, 8, false>), grid, block, 0, s, plan, args); \
+    else hipLaunchKernelGGL(k_noisy_block<KS>, grid, block, unsigned(cfg->n_in * KS * 1024), s,   \
+                            plan, args)
+        if (block_read(cfg)) {
+            if (ks == 8) { MF_BLOCK_LAUNCH(8); }
+            else { MF_BLOCK_LAUNCH(4); }
+        }
+        else if (ks == 4) MF_NOISY_LAUNCH(4, 5)
         else if (cfg->n_in <= 5) MF_NOISY_LAUNCH(2, 5)
         else MF_NOISY_LAUNCH(2, 8)
+#undef MF_BLOCK_LAUNCH
 #undef MF_NOISY_LAUNCH
 #undef MF_NOISY_LAUNCH2
 #undef MF_NOISY_LAUNCH1
@@ -594,7 +680,7 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
     }
     // With split_totals the caller restores and sums a split read's totals [n, G, ncols]
     // itself (null when the read wrote `out`).
-    const bool restored = use_split && noisy_small_tile(cfg, n);   // k_noisy_pairs restored
+    const bool restored = use_split && pairs_read(cfg, n, m, p);   // k_noisy_pairs restored
     if (split_totals) *split_totals = use_split ? partial : nullptr;
     if (split_restored) *split_restored = restored;
     if (use_split && !split_totals)
@@ -1769,7 +1855,10 @@ int mf_mm_static(const mf_config *cfg, const uint8_t *q, const float *xscale, in
                                  "conductance terms"
                                : "one 64-column chunk of noisy conductance terms";
     }
-    if (need > MF_STATIC_SCRATCH_BYTES)
+    // A block read beyond the scratch whose conductances need no sampling runs on the general
+    // kernel, which takes none.
+    const bool general = block_read(cfg) && !needs_conductances(cfg);
+    if (need > MF_STATIC_SCRATCH_BYTES && !general)
         return fail(MF_E_RESOURCE,
                     "mf_mm_static needs %lld bytes of scratch for the %s; its static scratch "
                     "holds %lld (MF_STATIC_SCRATCH_BYTES)",
@@ -2294,7 +2383,7 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
     const bool ks4 = cfg->read_rows == 64;
     const bool output_noise = cfg->has_read && cfg->read_mode == MF_READ_OUTPUT;
     const void *fn = nullptr;
-    int threads = 256;
+    int threads = 256, dynamic_lds = 0;
     if (kernel_id == 1) {
         // 32-row reads: 32 or (tile field 1) 64 vectors per wave; 64-row reads: KS 2.
         if (ks4) fn = reinterpret_cast<const void *>(&k_ideal<1, 2>);
@@ -2323,6 +2412,11 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
         const int mode = output_noise ? (cfg->has_vnoise ? 3 : 2) : (cfg->has_vnoise ? 1 : 0);
         const bool slice = cfg->has_read && cfg->read_mode == MF_READ_SLICE_PAIR;
         fn = table[which][mode][slice ? 1 : 0][nl ? 1 : 0];
+        if (block_read(cfg)) {
+            fn = ks4 ? reinterpret_cast<const void *>(&k_noisy_block<4>)
+                     : reinterpret_cast<const void *>(&k_noisy_block<8>);
+            dynamic_lds = cfg->n_in * (ks4 ? 4 : 8) * 1024;
+        }
         if (n > 0 && noisy_small_tile(cfg, n) && variant_split(variant) != 1) {
             // A split read of at most 32 vectors (the automatic split applies below 512
             // four-wave blocks, 32768 output columns): k_noisy_pairs, one wave per weight
@@ -2335,7 +2429,11 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                 {reinterpret_cast<const void *>(&k_noisy_pairs<4, 5, false>),
                  reinterpret_cast<const void *>(&k_noisy_pairs<4, 5, true>)}};
             fn = pairs[which][nl ? 1 : 0];
+            if (block_read(cfg))
+                fn = ks4 ? reinterpret_cast<const void *>(&k_noisy_pairs<4, 8, false>)
+                         : reinterpret_cast<const void *>(&k_noisy_pairs<8, 8, false>);
             threads = 64 * cfg->n_w;
+            dynamic_lds = 0;
         }
     } else if (kernel_id == 3) {
         // The LDS tier: the schedule's (tier field 1-3), else launch_noisy_wide's automatic one.
@@ -2377,11 +2475,11 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
     if (e != hipSuccess) return fail(MF_E_HIP, "hipFuncGetAttributes: %s", hipGetErrorString(e));
     memset(out, 0, sizeof(*out));
     out->threads = threads;
-    out->shared_bytes = int32_t(attr.sharedSizeBytes);
+    out->shared_bytes = int32_t(attr.sharedSizeBytes) + dynamic_lds;
     out->registers = attr.numRegs;
     out->local_bytes = int32_t(attr.localSizeBytes);
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, threads, 0) == hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, threads, size_t(dynamic_lds)) == hipSuccess)
         out->max_blocks_per_cu = blocks;
     if (blocks == 0) return fail(MF_E_RESOURCE, "zero resident blocks");
     return MF_OK;

@@ -169,7 +169,10 @@ struct NoisyPlan {
     u32 in_mask4[8];   // input slice mask replicated into four bytes
     u32 bias;          // -0x400000 * sum(fa*fw) modulo 2^32
     u32 f24[8][8];     // fa*fw as the 24-bit signed operand of v_mad_i32_i24, per (a, w)
-    float top_magic[8];  // 1.5 * 2^23 + adc_max[w] (exact in FP32)
+    // Rounding constant and upper limit of the converter, 1.5 * 2^23 and that plus adc_max[w]
+    // (exact in FP32), times the terms' scale: k_noisy_block's terms carry a power of two S_w
+    // in k1[w].
+    float magic[8], top_magic[8];
 };
 
 struct NoisyArgs {
@@ -202,6 +205,10 @@ __global__ void k_noisy(const NoisyPlan plan, const NoisyArgs args);
 // vectors x 32 columns and one read (grid: column blocks, vector blocks, reads); writes
 // slice totals [n, G, ldo], or with args.restored the restored (float(T) * xs) * ws
 // (plain and S-curve reads).
+// The read of digits in LDS (noisy_block.hip): block = up to 4 waves on the same 32 vectors,
+// 32 columns per wave; n_in * KS KiB of dynamic LDS.
+template <int KS>
+__global__ void k_noisy_block(const NoisyPlan plan, const NoisyArgs args);
 template <int KS, int NA, bool NONLINEAR>
 __global__ void k_noisy_pairs(const NoisyPlan plan, const NoisyArgs args);
 // Input operands of a read with voltage variation (memfast/reference.py:77-82): per

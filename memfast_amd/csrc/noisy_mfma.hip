@@ -34,13 +34,9 @@
 // writes one plane of terms per input slice and a pair loads its plane.
 #include <cfloat>
 
-#include "mf_kernels.h"
+#include "mf_noisy.h"
 
 namespace mf {
-
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v4fn __attribute__((ext_vector_type(4)));
 
 template <int KS>
 __global__ __launch_bounds__(256) void k_split_conductances(const mf_config cfg, const u8 *packed_t,
@@ -126,31 +122,9 @@ template __global__ void k_split_conductances<2>(const mf_config, const u8 *, co
 template __global__ void k_split_conductances<4>(const mf_config, const u8 *, const float *, i64,
                                                  i64, i64, u32, u64, i64, i64, const NoisyPlan,
                                                  uint4 *);
-
-// Buffer resource over [base, base + bytes): loads past the end return zero.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t noisy_buffer(const void *base, i64 bytes) {
-    const int records = bytes > 0x7FFFFFFF ? 0x7FFFFFFF : int(bytes < 0 ? 0 : bytes);
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), short(0), records,
-                                             0x00020000);
-}
-
-// Eight input digits (bytes of `word`, slice (shift, mask)) as eight fp16.  Each digit d
-// (at most 8 bits) becomes the low byte of fp16 0x64dd = 1024 + d: one v_perm places two
-// digits beside two 0x64 bytes, and one packed fp16 subtraction of 1024 leaves d exactly
-// (the same fp16 values as a conversion).  Six instructions per four digits.
-__device__ __forceinline__ v8h digits_f16(uint2 word, int shift, u32 mask4) {
-    typedef _Float16 v2f16 __attribute__((ext_vector_type(2)));
-    const v2f16 base = {_Float16(1024.0f), _Float16(1024.0f)};
-    const u32 lo = (word.x >> shift) & mask4, hi = (word.y >> shift) & mask4;
-    // Byte pool of v_perm(src0, src1, sel): src1 bytes 0-3 (0x64), src0 bytes 4-7.
-    const u32 k64 = 0x64646464u;
-    const u32 w[4] = {__builtin_amdgcn_perm(lo, k64, 0x00050004u), __builtin_amdgcn_perm(lo, k64, 0x00070006u),
-                      __builtin_amdgcn_perm(hi, k64, 0x00050004u), __builtin_amdgcn_perm(hi, k64, 0x00070006u)};
-    u32 o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(u32, __builtin_bit_cast(v2f16, w[i]) - base);
-    return __builtin_bit_cast(v8h, make_uint4(o[0], o[1], o[2], o[3]));
-}
+template __global__ void k_split_conductances<8>(const mf_config, const u8 *, const float *, i64,
+                                                 i64, i64, u32, u64, i64, i64, const NoisyPlan,
+                                                 uint4 *);
 
 // Eight consecutive input codes of one vector: bytes (narrow) or 32-bit words (wide).
 __device__ __forceinline__ void codes8(const u8 *q, u32 (&c)[8]) {
@@ -657,8 +631,9 @@ __device__ __forceinline__ void noisy_read(const NoisyPlan &plan, const NoisyArg
 // S-curve reads (terms event-independent or shared read noise).
 template <int KS, int NA, bool NONLINEAR>
 __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const NoisyArgs args) {
-    const float MAGIC = 12582912.0f;   // 1.5 * 2^23
     constexpr int P = 16 * KS;
+    // Configurations of k_noisy_block (scaled terms) sum the low terms first, as it does.
+    constexpr bool LOW_FIRST = KS * NA > 20;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // this wave's weight slice
@@ -687,7 +662,8 @@ __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const
                                __builtin_amdgcn_raw_buffer_load_b32(qbuf, q_off + ks * 16 + 4, 0, 0));
     // LDS: first the digits of every input slice (wave w builds slices w, w + W, ..), then
     // the waves' total words.
-    __shared__ u32 shared_words[8 * 16 * 64];
+    constexpr int DIGIT_WORDS = NA * KS * 64 * 4, PLANE_WORDS = 8 * 16 * 64;
+    __shared__ u32 shared_words[DIGIT_WORDS > PLANE_WORDS ? DIGIT_WORDS : PLANE_WORDS];
     uint4 *sdigits = reinterpret_cast<uint4 *>(shared_words);   // [a][ks][64 lanes]
     for (int a = w; a < A; a += W)
 #pragma unroll
@@ -711,9 +687,9 @@ __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const
     u32 Ti[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) Ti[r] = 0u;
-    const float top = plan.top_magic[w], alpha = plan.alpha[w];
-    // The MFMA order of noisy_read (terms outer, row blocks inner), so the totals are its
-    // totals bit for bit.  Unrolled over the input slices (at most NA), so that a slice's
+    const float magic = plan.magic[w], top = plan.top_magic[w], alpha = plan.alpha[w];
+    // The MFMA order of noisy_read or k_noisy_block (terms outer, row blocks inner), so the
+    // totals are its totals bit for bit.  Unrolled over the input slices (at most NA), so that a slice's
     // MFMAs can issue while the previous slice's currents are converted.
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
@@ -724,15 +700,17 @@ __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const
             digits[ks] = __builtin_bit_cast(v8h, sdigits[(a * KS + ks) * 64 + lane]);
         v16f I = {};
 #pragma unroll
-        for (int term = 0; term < NOISY_TERMS; ++term)
+        for (int i = 0; i < NOISY_TERMS; ++i) {
+            const int term = LOW_FIRST ? NOISY_TERMS - 1 - i : i;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
                 I = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[term][ks], digits[ks], I, 0, 0, 0);
+        }
         const u32 f24 = u32(int(plan.f24[a][w] << 8) >> 8);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            float y = (NONLINEAR ? scurve(I[r], alpha) : I[r]) + MAGIC;
-            y = __builtin_amdgcn_fmed3f(y, MAGIC, top);
+            float y = (NONLINEAR ? scurve(I[r], alpha) : I[r]) + magic;
+            y = __builtin_amdgcn_fmed3f(y, magic, top);
             const int low = int(__float_as_uint(y) << 8) >> 8;
             Ti[r] += u32(low) * f24;
         }
@@ -762,6 +740,8 @@ __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const
     }
 }
 
+template __global__ void k_noisy_pairs<4, 8, false>(const NoisyPlan, const NoisyArgs);
+template __global__ void k_noisy_pairs<8, 8, false>(const NoisyPlan, const NoisyArgs);
 #define MF_PAIRS_INST(KS, NA)                                                                  \
     template __global__ void k_noisy_pairs<KS, NA, false>(const NoisyPlan, const NoisyArgs);  \
     template __global__ void k_noisy_pairs<KS, NA, true>(const NoisyPlan, const NoisyArgs);

@@ -818,6 +818,12 @@ def variant_word(tile=0, split=0, tier=0):
     return tile | split << SPLIT_SHIFT | tier << TIER_SHIFT
 
 
+def block_read(config):
+    """Whether a noisy read of ``config`` is one of k_noisy_block's (noisy_block.hip): 64-row
+    reads with more than five input slices, and 128-row reads."""
+    return (config.read_rows == 64 and len(config.input_layout) > 5) or config.read_rows == 128
+
+
 def terms_event_independent(config):
     """Whether the noisy read's sampled conductances are the same on every read event."""
     return not config.nonidealities.read_variation

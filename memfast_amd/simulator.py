@@ -412,9 +412,10 @@ class Simulator:
         budget or its kernel would spill registers."""
         c = self.config
         n, arrays, _ = q.shape
-        if tuning.workspace_need(c, n, arrays, matrix.p, schedule) > self.workspace_bytes:
+        budget = self.workspace_bytes
+        if tuning.workspace_need(c, n, arrays, matrix.p, schedule, budget) > budget:
             raise hip.ResourceError("workspace budget")
-        kernel = tuning.read_kernel(c, n, arrays, matrix.p)
+        kernel = tuning.read_kernel(c, n, arrays, matrix.p, budget)
         with torch.cuda.device(self.device):
             resource = hip.program(c, schedule["vectors"], schedule["columns"],
                                    self.device.index).resources(
@@ -706,7 +707,8 @@ class AnalogMatrix(nn.Module):
         if stable:
             output = self._execute_stable(q, xscale, packed, event)
         else:
-            kernel = hip.mm_kernel(config, q.shape[0], q.shape[1], self.p)
+            budget = (self.simulator.workspace_bytes if self.simulator.mode == "tuned" else None)
+            kernel = tuning.read_kernel(config, q.shape[0], q.shape[1], self.p, budget)
             codes_t = self._column_codes() if config.wide or kernel else None
             status = hip.status_word(q.device) if status is None else status
             if not defer and self._output_bounded(q.shape[1]):

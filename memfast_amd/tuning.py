@@ -50,9 +50,17 @@ def schedule_variant(schedule):
                             schedule.get("tier", 0))
 
 
-def read_kernel(config, n, arrays, partitions):
-    """The read kernel (0-3) ``hip.mm`` launches for n vectors through m x p arrays."""
-    return hip.mm_kernel(config, n, arrays, partitions)
+def read_kernel(config, n, arrays, partitions, budget=None):
+    """The read kernel (0-3) ``hip.mm`` launches for n vectors through m x p arrays.
+
+    A block read (``hip.block_read``) whose scratch exceeds ``budget`` bytes goes to the
+    general kernel where that needs no scratch of its own."""
+    kernel = hip.mm_kernel(config, n, arrays, partitions)
+    if (budget is not None and kernel == 2 and hip.block_read(config)
+            and not hip.needs_conductances(config)
+            and hip.mm_workspace_bytes(config, n, arrays, partitions, 0) > budget):
+        return 0
+    return kernel
 
 
 def schedule_grid(config, n, partitions, arrays=None):
@@ -73,11 +81,11 @@ def schedule_grid(config, n, partitions, arrays=None):
     return [base]
 
 
-def workspace_need(config, n, arrays, partitions, schedule):
+def workspace_need(config, n, arrays, partitions, schedule, budget=None):
     """Device bytes a read under ``schedule`` allocates besides its inputs and output: the MFMA
     kernels' scratch (mf_mm_workspace for the schedule's variant) or, for the general kernel
     with device noise, the restored conductance tensor."""
-    kernel = read_kernel(config, n, arrays, partitions)
+    kernel = read_kernel(config, n, arrays, partitions, budget)
     if kernel:
         return hip.mm_workspace_bytes(config, n, arrays, partitions, schedule_variant(schedule))
     if not hip.needs_conductances(config):

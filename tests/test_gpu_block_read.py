@@ -1,0 +1,110 @@
+"""The noisy read whose digits live in LDS (k_noisy_block, csrc/noisy_block.hip): 64-row reads
+with six to eight input slices and 128-row reads, linear converters, programming noise and faults.
+
+Sizes sit at the edges of its tiles: 32 vectors and 32 or 64 columns per wave, four waves per
+workgroup, cascades of 16 and 256 reads, small batches on k_noisy_pairs.
+"""
+
+import pytest
+import torch
+
+from memfast_amd import Config, Nonidealities, Simulator, hip
+from oracle import oracle
+from parity import check_product
+
+pytestmark = pytest.mark.gpu
+
+WRITE = dict(write_variation=0.02)
+CASES = {
+    # The default configuration: 64x64 arrays, one-bit slices of eight-bit codes.
+    "default": (dict(), WRITE),
+    "int4_faults": (dict(weight_bits=4), WRITE | dict(stuck_at_low=0.01, stuck_at_high=0.01)),
+    # Six and seven input slices, several weight slice widths, arrays of two reads.
+    "six_slices": (dict(input_slice=(1, 1, 1, 1, 2, 2), weight_slice=(1, 1, 2, 4), adc_bits=8,
+                        array_size=(128, 64), rows_per_read=64), WRITE),
+    "seven_slices": (dict(activation_bits=7, adc_bits=5, array_size=(64, 32)), WRITE),
+    # 128-row reads of one- and two-bit slices, with array columns 32 and 128.
+    "rows128": (dict(array_size=(128, 128), adc_bits=8), WRITE),
+    "rows128_sliced": (dict(input_slice=(1, 1, 2, 2, 2), weight_slice=(1, 1, 2, 2, 2),
+                            array_size=(256, 32), rows_per_read=128, adc_bits=8), WRITE),
+    "rows128_ideal": (dict(array_size=(128, 64), adc_bits=7), dict(write_variation=0.0)),
+}
+
+
+def case(name):
+    kwargs, effects = CASES[name]
+    return Config(**kwargs, nonidealities=Nonidealities(**effects))
+
+
+def programmed(cfg, n, k, o, device, seed):
+    gen = torch.Generator().manual_seed(seed)
+    a, b = torch.randn(n, k, generator=gen), torch.randn(k, o, generator=gen)
+    q, xs = hip.input_tiles(a.to(device), cfg)
+    packed, packed_t, ws = hip.weight_tiles(b.T.to(device), cfg)
+    return a, b, q, xs, packed, packed_t, ws.reshape(-1, packed.shape[1] * cfg.array_size[1])
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_totals_with_injected_conductances(hip_device, name):
+    """Slice totals equal the oracle's on the same conductances, except converter flips (the
+    budget of 1e-4 of the codes)."""
+    cfg = case(name)
+    a, b, q, _, packed, packed_t, _ = programmed(cfg, 70, 200, 100, hip_device, 3)
+    p = packed.shape[1]
+    assert hip.block_read(cfg) and hip.mm_kernel(cfg, 70, q.shape[1], p) == 2
+    raw, _, _ = oracle.restored(packed.cpu(), cfg, 4242, 3, 0, p)
+    expected = oracle.partial(q.cpu(), packed.cpu(), cfg, 4242, 3, 0, p, conductance=raw)
+    got = hip.mm_totals(q, packed_t, cfg, 4242, 3, conductance=raw.to(hip_device)).cpu()
+    diff = got.double() - expected.double()
+    codes = diff.numel() * len(cfg.input_layout) * len(cfg.weight_layout)
+    print("[block read]", name, "totals differing", int((diff != 0).sum()), "codes", codes,
+          flush=True)
+    assert int((diff != 0).sum()) <= max(1, 1e-4 * codes)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("n,k,o", [(1, 100, 32), (33, 64, 30), (32, 500, 300), (97, 300, 260)])
+def test_product_and_schedules(hip_device, name, n, k, o):
+    """The product is the oracle's under the flip accounting, and every read split (automatic,
+    none, two and seven chunks) gives the same output bit for bit."""
+    cfg = case(name)
+    a, b, q, xs, packed, packed_t, ws = programmed(cfg, n, k, o, hip_device, 5)
+    outputs = [hip.mm(q, xs, packed, packed_t, ws, cfg, 77, 1, variant=hip.variant_word(split=z),
+                      out_cols=o, k_rows=k)[:, :o].clone() for z in (0, 1, 2, 7)]
+    for output in outputs[1:]:
+        assert torch.equal(output.view(torch.int32), outputs[0].view(torch.int32))
+    got = Simulator(cfg, device=hip_device).mm(a.to(hip_device), b.to(hip_device))
+    check_product(cfg, got, a, b, hip_device, label=f"block read {name}")
+
+
+def test_reads_between_counts_keep_the_general_kernel():
+    """Read noise, drift, nonlinear converters and voltage noise put converter arguments
+    anywhere between two counts."""
+    for effects in (dict(read_variation=0.01), dict(adc_nonlinearity=0.1), dict(voltage_variation=0.01),
+                    dict(drift_coefficient=0.05, drift_time=100.0)):
+        cfg = Config(nonidealities=Nonidealities(**(WRITE | effects)))
+        assert hip.mm_kernel(cfg, 100, 4, 4) == 0, effects
+
+
+@pytest.mark.parametrize("name,reads", [("default", 300), ("rows128", 270), ("rows128_sliced", 17)])
+def test_read_order_levels(hip_device, name, reads):
+    """The fused cascade over more than 16 and 256 reads equals the split read's epilogue."""
+    cfg = case(name)
+    k = reads * cfg.read_rows - 5
+    _, _, q, xs, packed, packed_t, ws = programmed(cfg, 40, k, 70, hip_device, 6)
+    fused, split = (hip.mm(q, xs, packed, packed_t, ws, cfg, 9, 0, out_cols=70, k_rows=k,
+                           variant=hip.variant_word(split=z))[:, :70] for z in (1, 4))
+    assert torch.equal(fused.view(torch.int32), split.view(torch.int32))
+
+
+def test_tuned_read_without_samples_beyond_its_budget(hip_device, tmp_path):
+    """Ideal devices need no sampled conductances: where the block read's terms exceed a tuned
+    simulator's workspace budget, the general kernel reads the same counts."""
+    cfg = case("rows128_ideal")
+    gen = torch.Generator().manual_seed(8)
+    a, b = torch.randn(40, 500, generator=gen), torch.randn(500, 200, generator=gen)
+    tuned = Simulator(cfg, device=hip_device, mode="tuned", cache_dir=tmp_path, workspace_mb=0.01)
+    got = tuned.mm(a.to(hip_device), b.to(hip_device))
+    expected = Simulator(cfg, device=hip_device).mm(a.to(hip_device), b.to(hip_device))
+    assert torch.equal(got.view(torch.int32), expected.view(torch.int32))
+    assert tuned.report()["selections"][0]["selected"] is not None
