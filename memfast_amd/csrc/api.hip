@@ -155,6 +155,15 @@ bool all_cascade_columns(int C, i64 p) {
     return true;
 }
 
+// Largest |slice total|: the ADC clamps every count.
+double totals_bound(const mf_config *cfg) {
+    double fa = 0.0, fw = 0.0;
+    for (int a = 0; a < cfg->n_in; ++a) fa += std::fabs(double(cfg->in_factor[a]));
+    for (int w = 0; w < cfg->n_w; ++w)
+        fw += std::fabs(double(cfg->w_factor[w])) * double(cfg->adc_max[w]);
+    return fa * fw;
+}
+
 int byte_mask(int shift, int mask, bool sign_slice) {
     int m = (mask << shift) & 0xFF;
     if (sign_slice) m |= (0xFF << shift) & 0xFF;
@@ -924,6 +933,68 @@ int launch_general(const mf_config *cfg, const GeneralArgs &args, int out_kind, 
     return check_launch("general read");
 }
 
+// FP32 currents run on FP32 MFMA (k_general_mfma32, the same bits) for narrow codes without
+// output-mode read noise (or slice_pair noise with voltage variation, which spills): reads of at most 128 rows, cascade columns, totals in 32 bits, and
+// products of voltage and conductance far from FP32's subnormals.  `p`: tiles of the matrix.
+static bool fp32_mfma_ok(const mf_config *cfg, i64 m, i64 p) {
+    return !cfg->wide && !cfg->precise && !(cfg->has_read && cfg->read_mode == MF_READ_OUTPUT) &&
+           !(cfg->has_vnoise && restore_planes(cfg) > 1) && cfg->read_rows <= 128 && cfg->n_in <= 8 && cfg->n_w <= 8 && m * cfg->reads < 4096 &&
+           all_cascade_columns(cfg->cols, p) && totals_bound(cfg) < 2147483647.0 &&
+           double(cfg->f_low) * double(cfg->f_voltage) > 1e-25 && largest_delta(cfg) < 1e18;
+}
+
+// Read chunks of a fused read (grid z; 1: not split): the number that takes the fewest rounds of
+// reads over the blocks a CU holds (eight waves of these registers, 160 KiB of LDS), within
+// 256 MiB of totals.  Default Config with read noise, 600x900 inputs, 500 columns: 1.21 ms
+// unsplit, 0.82 ms split; 4x1500, 700 columns: 0.90 and 0.23 ms.
+static i64 mfma32_split(const mf_config *cfg, i64 n, i64 m, i64 p) {
+    const i64 G = m * cfg->reads, ncols = p * cfg->cols;
+    if (n * G * ncols * 4 > (i64(256) << 20)) return 1;
+    const int rows = cfg->read_rows <= 64 ? 64 : 128, waves = mfma32_waves(rows, cfg->n_w);
+    const i64 lds = mfma32_lds(rows, cfg->n_in, waves);
+    const i64 per_cu = std::max<i64>(1, std::min<i64>(8 / waves, (160 << 10) / lds));
+    const i64 blocks = (n + 31) / 32 * ((ncols + 31) / 32), slots = 256 * per_cu;
+    i64 best = 1, least = (blocks + slots - 1) / slots * G;
+    for (i64 z = 2; z <= G; ++z) {
+        const i64 cost = (blocks * z + slots - 1) / slots * ((G + z - 1) / z);
+        // (a chunk's totals are written and read back: only for a clear gain)
+        if (cost * 10 < least * 9) {
+            least = cost;
+            best = z;
+        }
+    }
+    return best;
+}
+
+static i64 mfma32_scratch(const mf_config *cfg, i64 n, i64 m, i64 p) {
+    if (!fp32_mfma_ok(cfg, m, p) || mfma32_split(cfg, n, m, p) < 2) return 0;
+    return align256(n * m * cfg->reads * p * cfg->cols * 4);
+}
+
+// Launches it and returns true, or returns false where the grid or the LDS does not fit.
+static bool launch_general_mfma32(const mf_config *cfg, GeneralArgs args, int out_kind,
+                                  hipStream_t s, i64 split = 1) {
+    const i64 gx = (args.n + 31) / 32, gy = (args.width * cfg->cols + 31) / 32;
+    args.g_step = (args.g_run + split - 1) / split;
+    const i64 gz = (args.g_run + args.g_step - 1) / args.g_step;
+    if (gy > 65535 || gz > 65535 || gx * gy > 0x7FFFFFFF) return false;
+    const dim3 grid{unsigned(gx), unsigned(gy), unsigned(gz)};
+    const bool slice = args.planes > 1, vn = cfg->has_vnoise != 0;
+    const int rows = cfg->read_rows <= 64 ? 64 : 128, waves = mfma32_waves(rows, cfg->n_w);
+#define MF_MFMA32_LAUNCH(ROWS, SLICE, VNOISE)                                                    \
+    hipLaunchKernelGGL((k_general_mfma32<ROWS, SLICE, VNOISE>), grid, dim3(64 * waves),          \
+                       unsigned(mfma32_lds(ROWS, cfg->n_in, waves)), s, *cfg, args, out_kind)
+#define MF_MFMA32_LAUNCH2(ROWS)                                                                  \
+    if (slice) MF_MFMA32_LAUNCH(ROWS, true, false);                                         \
+    else if (vn) MF_MFMA32_LAUNCH(ROWS, false, true);                                            \
+    else MF_MFMA32_LAUNCH(ROWS, false, false)
+    if (rows == 64) { MF_MFMA32_LAUNCH2(64); }
+    else { MF_MFMA32_LAUNCH2(128); }
+#undef MF_MFMA32_LAUNCH2
+#undef MF_MFMA32_LAUNCH
+    return true;
+}
+
 // Precise currents run on FP64 MFMA (k_general_mfma64) unless voltage variation or
 // output-mode read noise needs the general kernel.
 static bool precise_mfma_ok(const mf_config *cfg) {
@@ -954,10 +1025,29 @@ static int launch_general_mfma64(const mf_config *cfg, const GeneralArgs &args, 
     return check_launch("precise MFMA read");
 }
 
-// The general read (fused or to totals): FP32 currents on k_general, precise ones on FP64
-// MFMA where that applies and no per-pair codes are asked for, else k_general in FP64.
+// The general read (fused or to totals) on FP32 or (precise currents) FP64 MFMA where that
+// applies and no per-pair codes are asked for, else on k_general.
 static int launch_general_read(const mf_config *cfg, const GeneralArgs &args, int out_kind,
-                               hipStream_t s) {
+                               hipStream_t s, void *workspace = nullptr, i64 bytes = 0) {
+    const i64 scratch = out_kind == OUT_FUSED && workspace ? mfma32_scratch(cfg, args.n, args.m, args.p) : 0;
+    if (scratch > 0 && scratch <= bytes) {
+        // Chunks of reads write totals; the epilogue restores and sums them in torch's order.
+        GeneralArgs part = args;
+        part.out = workspace;
+        if (launch_general_mfma32(cfg, part, OUT_TOTALS, s, mfma32_split(cfg, args.n, args.m, args.p))) {
+            const i64 ncols = args.p * cfg->cols, G = args.m * cfg->reads;
+            hipLaunchKernelGGL(k_restore_sum_f32, dim3(grid_for(args.n * ncols)), dim3(256), 0, s,
+                               static_cast<const float *>(workspace), args.n, G, args.g_run, ncols,
+                               ncols, static_cast<const float *>(args.xscale),
+                               static_cast<const float *>(args.wscale), args.ldws,
+                               static_cast<float *>(args.out), args.ldo, args.lp_cascade, 0,
+                               args.status);
+            return check_launch("general MFMA read");
+        }
+    }
+    if (!args.codes && fp32_mfma_ok(cfg, args.m, args.p) &&
+        launch_general_mfma32(cfg, args, out_kind, s))
+        return check_launch("general MFMA read");
     if (!cfg->precise) return launch_general<float>(cfg, args, out_kind, s);
     return precise_mfma_ok(cfg) && !args.codes ? launch_general_mfma64(cfg, args, out_kind, s)
                                                : launch_general<double>(cfg, args, out_kind, s);
@@ -1409,6 +1499,7 @@ int mf_partial(const mf_config *cfg, const uint8_t *q, int64_t n, int64_t m, con
     args.event = event;
     args.planes = g ? restore_planes(cfg) : 1;
     const i64 G = m * cfg->reads;
+    args.g_run = G;
     args.lp_cascade = level_power(G);
     args.lp_interleaved = level_power(G / 4);
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1479,7 +1570,7 @@ int mf_mm_workspace(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32
         const i64 blocks = std::max<i64>(2, (p * cfg->cols + 31) / 32);
         *bytes = wide_prefix_bytes(n, m, cfg) + blocks * wide_block_bytes(cfg, m);
     } else {
-        *bytes = 0;
+        *bytes = mfma32_scratch(cfg, n, m, p);
     }
     return MF_OK;
 }
@@ -1639,11 +1730,13 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
     args.seed = seed;
     args.event = event;
     args.planes = g ? restore_planes(cfg) : 1;
+    args.g_run = g_run;
     args.lp_cascade = level_power(G);
     args.lp_interleaved = level_power(G / 4);
     std::pair<hipEvent_t, hipEvent_t> timing{nullptr, nullptr};
     if (profiling() && (timing = profile_pair()).first) hipEventRecord(timing.first, s);
-    const int launched = launch_general_read(cfg, args, OUT_FUSED, s);
+    // (the conductances g are the caller's: the workspace holds the split read's totals)
+    const int launched = launch_general_read(cfg, args, OUT_FUSED, s, workspace, workspace_bytes);
     if (timing.first) {
         hipEventRecord(timing.second, s);
         profile_push(timing);
@@ -1873,9 +1966,11 @@ int mf_mm_static(const mf_config *cfg, const uint8_t *q, const float *xscale, in
     variant &= ~MF_MM_REUSE_TERMS;
     const bool was_off = g_profile_off;
     g_profile_off = true;
+    // The general kernel takes none of the scratch: its reads on several streams may overlap.
+    const bool scratchless = need == 0 || need > MF_STATIC_SCRATCH_BYTES;
     const int launched = mf_mm(cfg, q, xscale, n, m, packed, packed_t, wscale, p, out_cols,
-                               k_rows, g, seed, event, out, ldo, ptr, MF_STATIC_SCRATCH_BYTES,
-                               variant, status, stream);
+                               k_rows, g, seed, event, out, ldo, scratchless ? nullptr : ptr,
+                               scratchless ? 0 : MF_STATIC_SCRATCH_BYTES, variant, status, stream);
     g_profile_off = was_off;
     return launched;
 }
@@ -2253,6 +2348,7 @@ int mf_partial_wide(const mf_config *cfg, const uint32_t *q, int64_t n, int64_t 
     args.event = event;
     args.planes = g ? restore_planes(cfg) : 1;
     const i64 G = m * cfg->reads;
+    args.g_run = G;
     args.lp_cascade = level_power(G);
     args.lp_interleaved = level_power(G / 4);
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2309,6 +2405,7 @@ int mf_mm_wide(const mf_config *cfg, const uint32_t *q, const double *xscale, in
     args.event = event;
     args.planes = g ? restore_planes(cfg) : 1;
     const i64 G = m * cfg->reads;
+    args.g_run = G;
     args.lp_cascade = level_power(G);
     args.lp_interleaved = level_power(G / 4);
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2467,6 +2564,18 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                          : reinterpret_cast<const void *>(&k_general<float, 8, false, WIDE>)))
         fn = cfg->wide ? MF_GENERAL_FN(true) : MF_GENERAL_FN(false);
 #undef MF_GENERAL_FN
+        if (fp32_mfma_ok(cfg, 1, 2)) {
+            const bool sl = restore_planes(cfg) > 1, vn = cfg->has_vnoise != 0;
+#define MF_MFMA32_FN(ROWS)                                                                       \
+    (sl ? reinterpret_cast<const void *>(&k_general_mfma32<ROWS, true, false>)                   \
+     : vn ? reinterpret_cast<const void *>(&k_general_mfma32<ROWS, false, true>)                 \
+          : reinterpret_cast<const void *>(&k_general_mfma32<ROWS, false, false>))
+            fn = cfg->read_rows <= 64 ? MF_MFMA32_FN(64) : MF_MFMA32_FN(128);
+#undef MF_MFMA32_FN
+            const int rows = cfg->read_rows <= 64 ? 64 : 128, waves = mfma32_waves(rows, cfg->n_w);
+            threads = 64 * waves;
+            dynamic_lds = mfma32_lds(rows, cfg->n_in, waves);
+        }
     } else {
         return fail(MF_E_INVALID, "unknown read kernel %d", kernel_id);
     }

@@ -1,5 +1,6 @@
 // General sliced array read on gfx950: every non-wide configuration, every
-// device effect.  Used for noisy devices and as the parity entry point.
+// device effect.  Used for noisy devices and as the parity entry point (k_general; on FP32 and
+// FP64 MFMA, k_general_mfma32 and k_general_mfma64 below, where those apply).
 //
 // Model (memfast/reference.py:63-117, memfast/kernels.cu:71-202): for each
 // read group g = i*Gr + j, input slice a and weight slice w,
@@ -266,6 +267,285 @@ __global__ __launch_bounds__(256) void k_general(const mf_config cfg, const Gene
             atomicOr(args.status, u32(MF_STATUS_OUTPUT));
     }
 }
+
+// The same read on FP32 MFMA, bit for bit (no output-mode read noise, and not slice_pair read
+// noise together with voltage variation):
+// v_mfma_f32_32x32x2_f32 adds its two rows one after the other, each as one fused multiply-add
+// (204,800 sums of 64 rows over magnitudes from 1e-18 to 1e3 equal fmaf's in every bit), so a
+// chain of it is k_general's ascending-row sum.  SLICE: slice_pair planes of conductances.
+//
+// Block: 32 vectors x 32 columns, a wave per weight slice (two from five slices on where two
+// blocks then fit a CU: one's staging and converters run under the other's sums, 13.8 against
+// 14.9 ms at 2048^3).  Per read the block stages the voltages of every input slice in LDS in operand order (a
+// lane's float4 is four steps of two rows; its digit's voltage comes from a small table, computed
+// once); a wave loads its slice's conductances from global memory eight rows ahead and holds
+// the currents of four input slices at a time, 16 registers each (eight at a time spilled).
+// After the converters the waves' totals meet in LDS, and each restores and sums the outputs
+// r = wave, wave + waves, ..
+// Why: k_general spends an LDS read per two FMAs and reaches 4.2 TFMA/s.  Bound: FP32 MFMA
+// (69 TFMA/s measured back to back on this card), with the converters (5 VALU instructions per
+// output and pair, 11 with the S-curve) partly under it.  Default Config, 2048^3, read noise and
+// S-curve: 13.5 ms (41 TFMA/s), 134 ms on k_general; 600x900 inputs and 500 columns with
+// slice_pair noise: 1.1 ms against 22.5.
+typedef float v16fg __attribute__((ext_vector_type(16)));
+
+template <int ROWS, bool SLICE, bool VNOISE>
+__global__ __launch_bounds__(ROWS == 64 ? 256 : 512, 2) void k_general_mfma32(const mf_config cfg,
+                                                           const GeneralArgs args, int out_kind) {
+    constexpr int GROUPS = ROWS / 8;              // eight rows (four steps) per group
+    constexpr int NA = MFMA32_SLICES;
+    const float MAGIC = 12582912.0f;              // 1.5 * 2^23
+    constexpr int PLANES = SLICE ? NA : 1;
+    extern __shared__ __align__(16) float lds32[];
+    float *table = lds32;                         // voltage of (slice, digit)
+    float4 *volt = reinterpret_cast<float4 *>(lds32 + MFMA32_TABLE);   // [slice][group][64]
+    int *planes = reinterpret_cast<int *>(lds32 + MFMA32_TABLE);       // [waves][16][64], reused
+    const int waves = int(blockDim.x >> 6);
+    // Levels 0 and 1 of the cascade over reads, [16][64] each: the wave that sums output r.
+    float *acc0 = lds32 + mfma32_lds(ROWS, cfg.n_in, waves) / 4 - 2048, *acc1 = acc0 + 1024;
+    const u8 *q_codes = static_cast<const u8 *>(args.q);
+    const u8 *packed = static_cast<const u8 *>(args.packed);
+    const float *xscale = static_cast<const float *>(args.xscale);
+    const float *wscale = static_cast<const float *>(args.wscale);
+    const float *cond = static_cast<const float *>(args.g);
+    float *out = static_cast<float *>(args.out);
+
+    const int R = cfg.rows, C = cfg.cols, P = cfg.read_rows, Gr = cfg.reads;
+    const int A = cfg.n_in, W = cfg.n_w;
+    const i64 m = args.m;
+    const int G = int(m * Gr);
+    const i64 ncols = args.width * C;
+    const i64 kp = m * R;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = lane & 31, h = lane >> 5;
+    u32 vtile, ctile;
+    xcd_tile(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x, gridDim.y, vtile, ctile);
+    const i64 v0 = i64(vtile) * 32, c0 = i64(ctile) * 32;
+    const i64 vec = v0 + l;              // this lane's vector: staging, and of every output
+    const bool vec_live = vec < args.n;
+    const u8 *q_row = q_codes + (vec_live ? vec : v0) * kp;
+    // This lane's column of the conductance operand (the last one past the matrix: those
+    // outputs are not written).
+    const i64 col = c0 + l < ncols ? c0 + l : ncols - 1;
+    const i64 col_t = col / C;
+    const int col_c = int(col - col_t * C);
+    const u64 read_seed = event_seed(args.seed, args.event);
+    const float low = cfg.f_low;
+    const float drift = drift_of<float>(cfg);
+    const i64 plane_stride = m * args.width * W * R * C;
+
+    // Voltages of every digit, as k_general forms them.
+    for (int a = 0, base = 0; a < A; base += cfg.in_mask[a] + 1, ++a)
+        for (int d = threadIdx.x; d <= cfg.in_mask[a]; d += blockDim.x)
+            table[base + d] = float(d) / float(cfg.in_mask[a]) * cfg.f_voltage;
+
+    // This lane's four codes (row parity h) of group sg of read g, and with them the voltages.
+    auto four_codes = [&](int g, int sg) -> u32 {
+        const int i = g / Gr, row0 = (g - i * Gr) * P;
+        const int len = (R - row0) < P ? (R - row0) : P;
+        const u8 *src = q_row + i64(i) * R + row0;
+        u32 four = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int rr = sg * 8 + 2 * j + h;
+            const u32 code = src[rr < len ? rr : len - 1];
+            four |= (rr < len && vec_live ? code : 0u) << (8 * j);
+        }
+        return four;
+    };
+    auto stage = [&](int i, int row0, int sg, u32 four) {
+        int base = 0;
+        for (int a = 0; a < A; ++a) {
+            const u32 mask = u32(cfg.in_mask[a]);
+            float4 *dst = &volt[(a * GROUPS + sg) * 64 + lane];
+            if constexpr (VNOISE) {
+                // One sample at a time (not unrolled): four would spill registers.
+#pragma unroll 1
+                for (int j = 0; j < 4; ++j) {
+                    const float v = table[base + ((four >> (8 * j + cfg.in_shift[a])) & mask)];
+                    // (a row past the read has digit 0: no voltage to vary)
+                    const i64 r = row0 + sg * 8 + 2 * j + h;
+                    const u64 address = u64(((vec * m + i) * A + a) * R + r);
+                    const float z = normal(address, read_seed, 40u, cfg.f_two_pi);
+                    reinterpret_cast<float *>(dst)[j] = v * (1.0f + cfg.f_vnoise * z);
+                }
+            } else {
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    v[j] = table[base + ((four >> (8 * j + cfg.in_shift[a])) & mask)];
+                *dst = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            base += int(mask) + 1;
+        }
+    };
+    // Group it*waves + wave of a read is this wave's; the first few are fetched a read ahead.
+    constexpr int AHEAD = GROUPS / 4;
+    u32 codes[AHEAD];
+    auto fetch = [&](int g) {
+#pragma unroll
+        for (int it = 0; it < AHEAD; ++it)
+            if (it * waves + wave < GROUPS) codes[it] = four_codes(g, it * waves + wave);
+    };
+
+    for (int r = wave; r < 16; r += waves) acc0[r * 64 + lane] = acc1[r * 64 + lane] = 0.0f;
+
+    // Reads of this block (a read split across blocks writes totals).
+    const int g0 = int(blockIdx.z * args.g_step);
+    const int g1 = int(g0 + args.g_step < args.g_run ? g0 + args.g_step : args.g_run);
+    if (g0 < g1) fetch(g0);
+    for (int g = g0; g < g1; ++g) {
+        const int i = g / Gr, row0 = (g - i * Gr) * P;
+        const int len = (R - row0) < P ? (R - row0) : P;
+        const int groups = (len + 7) / 8;
+        __syncthreads();   // the table, and every use of the last read's totals
+#pragma unroll
+        for (int it = 0; it < AHEAD; ++it)
+            if (it * waves + wave < groups) stage(i, row0, it * waves + wave, codes[it]);
+        for (int sg = AHEAD * waves + wave; sg < groups; sg += waves)
+            stage(i, row0, sg, four_codes(g, sg));
+        __syncthreads();
+        if (g + 1 < g1) fetch(g + 1);   // in flight under this read's sums
+
+        // Totals modulo 2^32: every converter adds fa*fw*(0x400000 + code), see below.
+        u32 Ti[16];
+        u32 bias = 0u;
+        for (int w = wave; w < W; w += waves)
+            for (int a = 0; a < A; ++a)
+                bias -= u32(int(cfg.in_factor[a] * cfg.w_factor[w])) * 0x400000u;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) Ti[r] = bias;
+        for (int w = wave; w < W; w += waves) {
+            const int w_mask = cfg.w_mask[w], w_shift = cfg.w_shift[w];
+            // Conductances of the rows of group sg (plane: slice_pair's input slice), `low` past
+            // the read.
+            const float *const cond_read =
+                cond + (((i * args.width + col_t) * W + w) * R + row0) * C + col_c;
+            const u8 *const code_read = packed + ((i * args.p + args.begin + col_t) * R + row0) * C + col_c;
+            auto load = [&](float (&e)[4], int sg, int plane) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int rr = sg * 8 + 2 * j + h;
+                    const int at = (rr < len ? rr : len - 1) * C;
+                    float value;
+                    if (cond) {
+                        value = cond_read[plane * plane_stride + at];
+                    } else {
+                        const u32 digit = (u32(code_read[at]) >> w_shift) & u32(w_mask);
+                        value = nominal_level<float>(cfg, int(digit), w_mask) * drift;
+                    }
+                    e[j] = rr < len ? value : low;
+                }
+            };
+            const float top = MAGIC + float(cfg.adc_max[w]), alpha = cfg.f_alpha_over_max[w];
+            for (int a0 = 0; a0 < A; a0 += NA) {
+                v16fg sum[NA];
+#pragma unroll
+                for (int a = 0; a < NA; ++a) sum[a] = v16fg{};
+                float next[PLANES][4];
+#pragma unroll
+                for (int pl = 0; pl < PLANES; ++pl) load(next[pl], 0, SLICE && a0 + pl < A ? a0 + pl : 0);
+                for (int sg = 0; sg < groups; ++sg) {
+                    float eff[PLANES][4];
+#pragma unroll
+                    for (int pl = 0; pl < PLANES; ++pl)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) eff[pl][j] = next[pl][j] - low;
+                    const int ahead = sg + 1 < groups ? sg + 1 : sg;
+#pragma unroll
+                    for (int pl = 0; pl < PLANES; ++pl)
+                        load(next[pl], ahead, SLICE && a0 + pl < A ? a0 + pl : 0);
+                    // (slices past A read stale LDS and their sums are not used)
+                    float4 v[NA];
+#pragma unroll
+                    for (int a = 0; a < NA; ++a) v[a] = volt[((a0 + a) * GROUPS + sg) * 64 + lane];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int a = 0; a < NA; ++a) {
+                            const float x = j == 0 ? v[a].x : j == 1 ? v[a].y : j == 2 ? v[a].z : v[a].w;
+                            sum[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(eff[SLICE ? a : 0][j], x,
+                                                                          sum[a], 0, 0, 0);
+                        }
+                }
+                // Converters and signed shift-add with k_general's roundings (currents are finite
+                // here): the add to 1.5 * 2^23 rounds half-even, med3 clamps in that domain, and
+                // its low 24 bits are 0x400000 + code.
+#pragma unroll
+                for (int a = 0; a < NA; ++a) {
+                    if (a0 + a < A) {
+                        const float scale = float(cfg.in_mask[a0 + a] * w_mask);
+                        const int factor = int(cfg.in_factor[a0 + a] * cfg.w_factor[w]);
+                        const u32 f24 = u32(int(u32(factor) << 8) >> 8);   // for v_mad_i32_i24
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            float z = sum[a][r] * scale;
+                            z = z * cfg.f_inv_unit;
+                            if (cfg.has_nonlinear) z = scurve(z, alpha);
+                            const float y = __builtin_amdgcn_fmed3f(z + MAGIC, MAGIC, top);
+                            Ti[r] += u32(int(__float_as_uint(y) << 8) >> 8) * f24;
+                        }
+                    }
+                }
+            }
+        }
+        // The waves' totals: each writes its plane, then adds outputs r = wave, wave + waves, ..
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) planes[(wave * 16 + r) * 64 + lane] = int(Ti[r]);
+        __syncthreads();
+        const float xs = xscale && vec_live ? xscale[vec * G + g] : 0.0f;
+        const int count = g + 1;
+        for (int r = wave; r < 16; r += waves) {
+            const i64 c = c0 + (r >> 2) * 8 + h * 4 + (r & 3);
+            int total = 0;
+            for (int k = 0; k < waves; ++k) total += planes[(k * 16 + r) * 64 + lane];
+            if (c >= ncols || !vec_live) continue;
+            if (out_kind == OUT_TOTALS) {
+                out[(vec * G + g) * ncols + c] = float(total);
+                continue;
+            }
+            float value = float(total) * xs;
+            value = value * wscale[g * args.ldws + args.begin * C + c];
+            float &s0 = acc0[r * 64 + lane], &s1 = acc1[r * 64 + lane];
+            s0 = s0 + value;
+            if ((count & 15) == 0) {
+                s1 = s1 + s0;
+                s0 = 0.0f;
+                if ((count & 255) == 0) {
+                    // Level 2 of the cascade lives in `out` (more than 255 reads).
+                    float *dst = out + vec * args.ldo + args.begin * C + c;
+                    *dst = count == 256 ? s1 : *dst + s1;
+                    s1 = 0.0f;
+                }
+            }
+        }
+    }
+    if (out_kind != OUT_FUSED) return;
+    bool finite = true;
+    for (int r = wave; r < 16; r += waves) {
+        const i64 c = c0 + (r >> 2) * 8 + h * 4 + (r & 3);
+        if (c >= ncols || !vec_live) continue;
+        float *dst = out + vec * args.ldo + args.begin * C + c;
+        float value = acc0[r * 64 + lane] + acc1[r * 64 + lane];
+        if (g1 >= 256) value = value + *dst;
+        *dst = value;
+        finite = finite && fabsf(value) <= FLT_MAX;
+    }
+    if (!finite && args.status) atomicOr(args.status, u32(MF_STATUS_OUTPUT));
+}
+
+#define MF_MFMA32_INST(ROWS, SLICE, VNOISE)                                                      \
+    template __global__ void k_general_mfma32<ROWS, SLICE, VNOISE>(const mf_config,              \
+                                                                   const GeneralArgs, int);
+MF_MFMA32_INST(64, false, false)
+MF_MFMA32_INST(64, false, true)
+MF_MFMA32_INST(64, true, false)
+MF_MFMA32_INST(128, false, false)
+MF_MFMA32_INST(128, false, true)
+MF_MFMA32_INST(128, true, false)
+#undef MF_MFMA32_INST
 
 // FP64 MFMA read for precise currents (memfast/config.py:215-224: FP64 conductances and
 // currents), every device effect but voltage variation and output-mode read noise.

@@ -21,6 +21,8 @@ struct GeneralArgs {
     int32_t *codes;       // optional [n, G, A, W, width*C]
     u32 *status;          // optional: MF_STATUS_OUTPUT for a non-finite fused output
     i64 n, m, p, begin, width, ldo, ldws;
+    i64 g_run;            // reads executed: [0, g_run) (the rest is zero padding)
+    i64 g_step;           // k_general_mfma32: reads per blockIdx.z
     u32 seed;
     u64 event;
     int planes;
@@ -33,6 +35,22 @@ __global__ void k_general(const mf_config cfg, const GeneralArgs args, int out_k
 // noise), fused or to totals as k_general.
 template <bool WIDE, bool STAGED>
 __global__ void k_general_mfma64(const mf_config cfg, const GeneralArgs args, int out_kind);
+// k_general's FP32 read on FP32 MFMA, bit for bit (narrow codes, no output-mode read noise):
+// mfma32_waves() waves a block, one or two weight slices each, reads of at most ROWS rows;
+// dynamic LDS of mfma32_lds() bytes: the voltage table, the voltages or the waves' totals, the
+// cascade's sums.
+template <int ROWS, bool SLICE, bool VNOISE>
+__global__ void k_general_mfma32(const mf_config cfg, const GeneralArgs args, int out_kind);
+constexpr int MFMA32_SLICES = 4;    // input slices whose currents a wave holds at a time
+constexpr int MFMA32_TABLE = 256;   // (slice, digit) voltages: at most 2 + 128 of 8-bit codes
+constexpr int mfma32_waves(int rows, int n_w) {
+    return rows == 64 && n_w > 4 ? (n_w + 1) / 2 : n_w;
+}
+__host__ __device__ constexpr int mfma32_lds(int rows, int n_in, int waves) {
+    const int slices = (n_in + MFMA32_SLICES - 1) / MFMA32_SLICES * MFMA32_SLICES;
+    const int volts = slices * (rows / 8) * 1024, totals = waves * 4096;
+    return MFMA32_TABLE * 4 + (volts > totals ? volts : totals) + 8192;
+}
 constexpr int MFMA64_STAGED_MAX_W = 8;   // weight slices of the LDS-staged variant
 
 // ---- ideal MFMA read (ideal_mfma.hip) -------------------------------------

@@ -830,7 +830,8 @@ def terms_event_independent(config):
 
 
 def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=None, out=None,
-       variant=0, status=None, workspace=None, reuse_terms=False, out_cols=None, k_rows=None):
+       variant=0, status=None, workspace=None, reuse_terms=False, out_cols=None, k_rows=None,
+       split_budget=None):
     """Fused read + scale restore: [N, p*C] FP32, summed over reads in torch's order.
 
     Wide configurations: ``packed_t`` is the uint32 kernel copy of the codes
@@ -840,7 +841,8 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
     a previous call of this program sampled (honoured when they do not depend
     on the read event).  ``out_cols``/``k_rows`` (default: all) are the logical
     output columns and input rows; the MFMA kernels leave columns past
-    ``out_cols`` unwritten and skip reads wholly past row ``k_rows``.
+    ``out_cols`` unwritten and skip reads wholly past row ``k_rows``.  ``split_budget``
+    (optional) bounds the bytes of totals that a general read may be split through.
     """
     supported(config)
     require_device(q)
@@ -873,7 +875,10 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
         if reuse_terms and kernel == 2:
             variant |= REUSE_TERMS
     else:
-        workspace = None
+        # The general kernel's: totals of a read split across blocks, where that helps.
+        size = mm_workspace_bytes(config, n, m, p, 0) if mm_kernel(config, n, m, p) == 0 else 0
+        fits = size and (split_budget is None or size <= split_budget)
+        workspace = torch.empty(size, dtype=torch.uint8, device=q.device) if fits else None
     # Converted operands stay referenced until the launch is queued (a freed
     # temporary could be handed to the next conversion by the caching allocator).
     q, xscale = q.contiguous(), xscale.contiguous()

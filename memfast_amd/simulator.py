@@ -721,9 +721,12 @@ class AnalogMatrix(nn.Module):
             if kernel == 2 and hip.terms_event_independent(config):
                 workspace, reuse, source = self._terms_workspace(q.shape[0], q.shape[1], q.device,
                                                                  codes_t, variant)
+            # A tuned read's totals stay within the budget its schedule was admitted under.
+            left = (None if budget is None else budget - tuning.workspace_need(
+                config, q.shape[0], q.shape[1], self.p, schedule, budget))
             output = hip.mm(q, xscale, packed, codes_t, self.weight_scale.reshape(-1, columns),
                             config, self.seed, event, variant=variant, status=status,
-                            workspace=workspace, reuse_terms=reuse,
+                            workspace=workspace, reuse_terms=reuse, split_budget=left,
                             out_cols=self.out_features, k_rows=self.in_features)
             if source is not None:
                 self._terms_source = source
