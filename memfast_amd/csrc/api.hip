@@ -82,6 +82,8 @@ int check_launch(const char *what) {
     return MF_OK;
 }
 
+bool aligned(const void *p, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; }
+
 unsigned grid_for(i64 total, int block = 256) {
     i64 blocks = (total + block - 1) / block;
     if (blocks < 1) blocks = 1;
@@ -1317,6 +1319,20 @@ int mf_quantize_inputs(const mf_config *cfg, const float *x, int64_t n, int64_t 
             hipLaunchKernelGGL(k_row_groups_wave<16>, grid, dim3(256), 0, s, x, n, k, ld, ncg, kp,
                                -upper, upper, mask, q, scale, status, u32(MF_STATUS_INPUT), reads);
         return check_launch("input quantization");
+    } else if (gr == 1 && gc >= 64 && n * ncg <= 0x7FFFFFFF) {
+        // Groups of other lengths: a wave each up to 1024 columns, else a workgroup.
+        const ReadTable reads{direct ? nullptr : xscale, m * Gr, R, P, Gr};
+        const unsigned groups = unsigned(n * ncg);
+#define MF_ROW_BLOCK(T, VEC)                                                                     \
+    hipLaunchKernelGGL((k_row_groups_block<T, VEC>), dim3((groups + 256 / T - 1) / (256 / T)),     \
+                       dim3(256), 0, s, x, n, k, ld, gc, ncg, kp, -upper, upper, mask, q, scale,  \
+                       status, u32(MF_STATUS_INPUT), reads)
+        if (gc <= 1024 && vec) MF_ROW_BLOCK(64, true);
+        else if (gc <= 1024) MF_ROW_BLOCK(64, false);
+        else if (vec) MF_ROW_BLOCK(256, true);
+        else MF_ROW_BLOCK(256, false);
+#undef MF_ROW_BLOCK
+        return check_launch("input quantization");
     } else if (gr == 1 && gc <= 1024) {
         if (vec)
             hipLaunchKernelGGL(k_row_groups<true>, dim3(grid_for(n * ncg)), dim3(256), 0, s, x, n, k,
@@ -1367,6 +1383,31 @@ int mf_quantize_weights(const mf_config *cfg, const float *b, int64_t k, int64_t
     const bool reg_group = gr == 8 || gr == 16 || gr == 32 || gr == 64;
     const bool tiled = (gr == 16 || gr == 32) && cfg->cols % 64 == 0 && R % (4 * gr) == 0 &&
                        kp % 16 == 0;
+    // Whole columns of more than 64 rows: maxima of chunks of rows (kept in `packed`, whose codes
+    // are written last), scales, codes.  Shorter ones stay with the kernels that hold a group.
+    const i64 chunk_rows = std::max<i64>(16, (k + m * Gr - 1) / (m * Gr));
+    const i64 chunks = (k + chunk_rows - 1) / chunk_rows;
+    if (gc == 1 && nrg == 1 && gr > 64 && kp % 16 == 0 && cfg->cols % 64 == 0 &&
+        chunks * o * 4 <= kp * op && chunks <= 65535 && (kp + 127) / 128 <= 65535 &&
+        aligned(packed, 16) && aligned(packed_t, 16)) {
+        float *peaks = reinterpret_cast<float *>(packed);
+        const bool vec = o % 4 == 0 && ld % 4 == 0 && aligned(b, 16);
+        if (vec)
+            hipLaunchKernelGGL(k_column_peaks<4>, dim3(unsigned((o + 255) / 256), unsigned(chunks)),
+                               dim3(256), 0, s, b, k, o, ld, chunk_rows, peaks, status,
+                               u32(MF_STATUS_WEIGHT));
+        else
+            hipLaunchKernelGGL(k_column_peaks<1>, dim3(unsigned((o + 63) / 64), unsigned(chunks)),
+                               dim3(256), 0, s, b, k, o, ld, chunk_rows, peaks, status,
+                               u32(MF_STATUS_WEIGHT));
+        hipLaunchKernelGGL(k_column_scales, dim3(unsigned(op / 64)), dim3(256), 0, s, peaks, chunks,
+                           o, op, m * Gr, upper, scale, wscale);
+        hipLaunchKernelGGL((k_col_groups_tile<32, true>),
+                           dim3(unsigned(op / 64), unsigned((kp + 127) / 128)), dim3(256), 0, s, b,
+                           k, o, ld, R, C, m, p, lower, upper, mask, packed, packed_t, scale, gr,
+                           status, u32(MF_STATUS_WEIGHT));
+        return check_launch("weight quantization");
+    }
     if (gc == 1 && tiled && kp / (4 * gr) <= 65535) {
         const dim3 grid{unsigned(op / 64), unsigned(kp / (4 * gr)), 1u};
         if (gr == 16)

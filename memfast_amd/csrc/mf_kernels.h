@@ -367,6 +367,15 @@ template <int V>
 __global__ void k_row_groups_wave(const float *x, i64 n, i64 k, i64 ld, i64 ncg, i64 kp,
                                   float lower, float upper, u32 mask, u8 *q, float *scale,
                                   u32 *status, u32 flag, const ReadTable reads);
+template <int T, bool VEC>
+__global__ void k_row_groups_block(const float *x, i64 n, i64 k, i64 ld, i64 gc, i64 ncg, i64 kp,
+                                   float lower, float upper, u32 mask, u8 *q, float *scale,
+                                   u32 *status, u32 flag, const ReadTable reads);
+template <int V>
+__global__ void k_column_peaks(const float *b, i64 k, i64 o, i64 ld, i64 rows, float *peaks,
+                               u32 *status, u32 flag);
+__global__ void k_column_scales(const float *peaks, i64 chunks, i64 o, i64 op, i64 G, float upper,
+                                float *scale, float *wscale);
 template <int GR, bool WORD>
 __global__ void k_col_groups_reg(const float *b, i64 k, i64 o, i64 ld, int R, int C, i64 m,
                                  i64 p, float lower, float upper, u32 mask, u8 *packed,

@@ -276,6 +276,157 @@ template __global__ void k_row_groups_wave<16>(const float *, i64, i64, i64, i64
                                                float, u32, u8 *, float *, u32 *, u32,
                                                const ReadTable);
 
+// Row groups of any length: T threads per group (a wave, or a workgroup of 256), a pass for the
+// peak and one for the codes; a group of a few KiB stays in cache for the second.  VEC as in
+// k_row_groups, `reads` as in k_row_groups_wave.  784 columns, 128 rows: 6.2 us (launch and two
+// dependent passes), where one thread per group (k_row_groups) took 107; 1000 x 1500: 6.1 us in
+// one launch, where the group maximum, scale, code and scale-table passes took 20 in five.
+template <int T, bool VEC>
+__global__ __launch_bounds__(256) void k_row_groups_block(const float *x, i64 n, i64 k, i64 ld,
+                                                          i64 gc, i64 ncg, i64 kp, float lower,
+                                                          float upper, u32 mask, u8 *q,
+                                                          float *scale, u32 *status, u32 flag,
+                                                          const ReadTable reads) {
+    __shared__ float peaks[4];
+    constexpr int STEP = VEC ? 4 : 1;
+    const int member = threadIdx.x % T, lane = threadIdx.x & 63;
+    const i64 grp = i64(blockIdx.x) * (256 / T) + threadIdx.x / T;
+    const bool live = grp < n * ncg;   // whole waves (T == 64) or the whole block
+    const i64 row = live ? grp / ncg : 0, j = live ? grp - row * ncg : 0;
+    const i64 c0 = j * gc, c1 = live ? ((c0 + gc) < k ? (c0 + gc) : k) : c0;
+    const float *src = x + row * ld;
+    float peak = 0.0f;
+    bool finite = true;
+    for (i64 c = c0 + member * STEP; c < c1; c += T * STEP) {
+        float v[STEP];
+        if constexpr (VEC) {
+            const float4 f = *reinterpret_cast<const float4 *>(src + c);
+            v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        } else {
+            v[0] = src[c];
+        }
+#pragma unroll
+        for (int e = 0; e < STEP; ++e) {
+            const float a = fabsf(v[e]);
+            finite = finite && a <= FLT_MAX;
+            peak = fmaxf(peak, a);
+        }
+    }
+    for (int off = 1; off < 64; off <<= 1) peak = fmaxf(peak, __shfl_xor(peak, off, 64));
+    if constexpr (T == 256) {
+        if (lane == 0) peaks[threadIdx.x >> 6] = peak;
+        __syncthreads();
+        peak = fmaxf(fmaxf(peaks[0], peaks[1]), fmaxf(peaks[2], peaks[3]));
+    }
+    if (!finite && status) atomicOr(status, flag);
+    if (!live) return;
+    const float s = group_scale(peak, upper);
+    if (member == 0) scale[grp] = s;
+    if (reads.xscale) {
+        for (i64 rd = member; rd < reads.G; rd += T) {
+            i64 first = (rd / reads.Gr) * reads.R + (rd % reads.Gr) * reads.P;
+            first = first < k ? first : k - 1;
+            if (first >= c0 && first < c0 + gc) reads.xscale[row * reads.G + rd] = s;
+        }
+    }
+    u8 *dst = q + row * kp;
+    for (i64 c = c0 + member * STEP; c < c1; c += T * STEP) {
+        if constexpr (VEC) {
+            const float4 f = *reinterpret_cast<const float4 *>(src + c);
+            *reinterpret_cast<u32 *>(dst + c) =
+                u32(quantize_code(f.x, s, lower, upper, mask)) |
+                u32(quantize_code(f.y, s, lower, upper, mask)) << 8 |
+                u32(quantize_code(f.z, s, lower, upper, mask)) << 16 |
+                u32(quantize_code(f.w, s, lower, upper, mask)) << 24;
+        } else {
+            dst[c] = quantize_code(src[c], s, lower, upper, mask);
+        }
+    }
+    if (j == ncg - 1)
+        for (i64 c = k + member * STEP; c < kp; c += T * STEP) {
+            if constexpr (VEC) *reinterpret_cast<u32 *>(dst + c) = 0u;
+            else dst[c] = 0;
+        }
+}
+#define MF_ROW_BLOCK_INST(T, VEC)                                                                \
+    template __global__ void k_row_groups_block<T, VEC>(const float *, i64, i64, i64, i64, i64,  \
+                                                        i64, float, float, u32, u8 *, float *,   \
+                                                        u32 *, u32, const ReadTable);
+MF_ROW_BLOCK_INST(64, false)
+MF_ROW_BLOCK_INST(64, true)
+MF_ROW_BLOCK_INST(256, false)
+MF_ROW_BLOCK_INST(256, true)
+#undef MF_ROW_BLOCK_INST
+
+// Whole columns as weight groups (the default: one scale per output channel).  k_column_peaks:
+// max |b| of each column over one chunk of rows, peaks[chunk][o] (no atomics, nothing to clear);
+// V adjacent columns per lane.  k_column_scales then takes a column's maximum over the chunks,
+// and writes its group scale and its column of the per-read scale table (padded columns repeat
+// the last logical one, as k_weight_scales does).  Three launches with the codes' LDS tile, 21 us
+// for 1500 x 700; clearing, group maxima, scales, 256-row columns of codes (k_col_codes: six
+// workgroups) and the table took 100 in five.
+template <int V>
+__global__ __launch_bounds__(256) void k_column_peaks(const float *b, i64 k, i64 o, i64 ld,
+                                                      i64 rows, float *peaks, u32 *status,
+                                                      u32 flag) {
+    __shared__ float part[4][64 * V];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const i64 c = (i64(blockIdx.x) * 64 + lane) * V;
+    const i64 r0 = i64(blockIdx.y) * rows, r1 = (r0 + rows) < k ? (r0 + rows) : k;
+    float peak[V];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < V; ++e) peak[e] = 0.0f;
+    if (c < o) {   // o is a multiple of V
+#pragma unroll 4
+        for (i64 r = r0 + wave; r < r1; r += 4) {
+            float v[V];
+            if constexpr (V == 4) {
+                const float4 f = *reinterpret_cast<const float4 *>(b + r * ld + c);
+                v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+            } else {
+                v[0] = b[r * ld + c];
+            }
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const float a = fabsf(v[e]);
+                finite = finite && a <= FLT_MAX;
+                peak[e] = fmaxf(peak[e], a);
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) part[wave][lane * V + e] = peak[e];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * V; i += 256) {
+        const i64 col = i64(blockIdx.x) * 64 * V + i;
+        if (col < o)
+            peaks[i64(blockIdx.y) * o + col] =
+                fmaxf(fmaxf(part[0][i], part[1][i]), fmaxf(part[2][i], part[3][i]));
+    }
+    if (!finite && status) atomicOr(status, flag);
+}
+template __global__ void k_column_peaks<1>(const float *, i64, i64, i64, i64, float *, u32 *, u32);
+template __global__ void k_column_peaks<4>(const float *, i64, i64, i64, i64, float *, u32 *, u32);
+
+__global__ __launch_bounds__(256) void k_column_scales(const float *peaks, i64 chunks, i64 o,
+                                                       i64 op, i64 G, float upper, float *scale,
+                                                       float *wscale) {
+    __shared__ float part[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const i64 col = i64(blockIdx.x) * 64 + lane;
+    const i64 from = col < o ? col : o - 1;
+    float peak = 0.0f;
+    for (i64 i = wave; i < chunks; i += 4) peak = fmaxf(peak, peaks[i * o + from]);
+    part[wave][lane] = peak;
+    __syncthreads();
+    peak = fmaxf(fmaxf(part[0][lane], part[1][lane]), fmaxf(part[2][lane], part[3][lane]));
+    const float s = group_scale(peak, upper);
+    if (wave == 0 && col < o) scale[col] = s;
+    if (col < op)
+        for (i64 g = wave; g < G; g += 4) wscale[g * op + col] = s;
+}
+
 // Column groups of GR rows held in registers: thread = (physical column, one
 // row group), so every lane issues its GR coalesced loads at once.  Writes the
 // scale grid, packed [m, p, R, C] (bytes, coalesced across lanes) and the
@@ -347,8 +498,8 @@ __device__ __forceinline__ uint64_t proven_slots(const SlotTests &tests, const i
 // holds its group's GR values in registers (coalesced 256-byte row loads),
 // writes its codes into the tile, and the workgroup then stores the tile as
 // 64-byte row segments of packed [m, p, R, C] and 4*GR-byte column runs of
-// packed_t [p*C, m*R], 16 bytes per store.  Requires C % 64 == 0, R % (4*GR)
-// == 0 (row segments stay inside one array tile) and kp % 16 == 0.
+// packed_t [p*C, m*R], 16 bytes per store.  Requires C % 64 == 0 and kp % 16 == 0, and
+// without GIVEN R % (4*GR) == 0 (a group stays inside one array tile).
 // GIVEN: the group scales [ceil(k/gr), o] are already in `scale` (any gr, from
 // a separate group-maximum pass); each row takes its group's scale.
 // With `digits` (GR == 32 == rows per read), each wave also reduces its read's
