@@ -687,7 +687,8 @@ __global__ __launch_bounds__(512) void k_noisy_pairs(const NoisyPlan plan, const
     u32 Ti[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) Ti[r] = 0u;
-    const float magic = plan.magic[w], top = plan.top_magic[w], alpha = plan.alpha[w];
+    const float magic = LOW_FIRST ? plan.magic[w] : 12582912.0f;   // else unscaled: 1.5 * 2^23
+    const float top = plan.top_magic[w], alpha = plan.alpha[w];
     // The MFMA order of noisy_read or k_noisy_block (terms outer, row blocks inner), so the
     // totals are its totals bit for bit.  Unrolled over the input slices (at most NA), so that a slice's
     // MFMAs can issue while the previous slice's currents are converted.
