@@ -587,17 +587,18 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
     for (i64 c_begin = 0; c_begin < ocols; c_begin += max_cb * 32) {
         const i64 cols = (ocols - c_begin) < max_cb * 32 ? (ocols - c_begin) : max_cb * 32;
         const i64 CB = (cols + 63) / 64 * 2;
-        const i64 threads = i64(cfg->n_w) * CB * G * ks * 64;
+        const dim3 units(unsigned(CB), unsigned(std::min<i64>((G * ks + 3) / 4, 65535)),
+                         unsigned(cfg->n_w));
         if (reuse) {
             // terms already in place
         } else if (ks == 2) {
-            hipLaunchKernelGGL(k_split_conductances<2>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+            hipLaunchKernelGGL(k_split_conductances<2>, units, dim3(256), 0, s, *cfg,
                                packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         } else if (ks == 4) {
-            hipLaunchKernelGGL(k_split_conductances<4>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+            hipLaunchKernelGGL(k_split_conductances<4>, units, dim3(256), 0, s, *cfg,
                                packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         } else {
-            hipLaunchKernelGGL(k_split_conductances<8>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+            hipLaunchKernelGGL(k_split_conductances<8>, units, dim3(256), 0, s, *cfg,
                                packed_t, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         }
         NoisyArgs args{};
@@ -836,12 +837,12 @@ int launch_noisy_wide(const mf_config *cfg, const NoisyWidePlan &plan, int ks,
     for (i64 c_begin = 0; c_begin < ncols; c_begin += max_cb * 32) {
         const i64 cols = (ncols - c_begin) < max_cb * 32 ? (ncols - c_begin) : max_cb * 32;
         const i64 CB = (cols + 31) / 32;
-        const i64 threads = CB * G * cfg->n_w * ks * 64;
+        const dim3 units(unsigned(CB), unsigned((G * ks + 3) / 4), unsigned(cfg->n_w));
         if (ks == 2)
-            hipLaunchKernelGGL(k_split_wide<2>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+            hipLaunchKernelGGL(k_split_wide<2>, units, dim3(256), 0, s, *cfg,
                                packed, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         else
-            hipLaunchKernelGGL(k_split_wide<4>, dim3(grid_for(threads)), dim3(256), 0, s, *cfg,
+            hipLaunchKernelGGL(k_split_wide<4>, units, dim3(256), 0, s, *cfg,
                                packed, g, m, p, ncols, seed, event, c_begin, CB, plan, gs);
         NoisyWideArgs args{};
         args.q16 = q16;

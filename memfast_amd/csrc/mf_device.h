@@ -65,6 +65,17 @@ __device__ __forceinline__ float normal_fast(u64 address, u64 seed, u32 stream) 
     return box_muller(uniform(address, seed, stream), uniform(address, seed, stream + 1u));
 }
 
+// normal_fast() at addresses below 2^32: the folds of both streams depend on the wave-uniform
+// seed alone, so they stay in scalar registers and a sample hashes twice instead of four times.
+struct LowNormal {
+    u32 fold_u, fold_v;
+    __device__ __forceinline__ LowNormal(u64 seed, u32 stream)
+        : fold_u(uniform_fold(0u, seed, stream)), fold_v(uniform_fold(0u, seed, stream + 1u)) {}
+    __device__ __forceinline__ float operator()(u32 address) const {
+        return box_muller(uniform_finish(address, fold_u), uniform_finish(address, fold_v));
+    }
+};
+
 // exp(x) for the noise exponents as exp2(x * log2(e)) on v_exp_f32: within 1 ulp of
 // exp(x) for |x| <= 0.5 and 4 ulp for |x| <= 4 (measured over 2^24 points).
 __device__ __forceinline__ float exp_small(float x) {

@@ -78,4 +78,54 @@ __device__ __forceinline__ Phys cell_conductance(const mf_config &cfg, u32 code,
     return raw;
 }
 
+// cell_conductance<float> at cells below 2^32 (LowNormal): the same samples.
+struct LowCells {
+    LowNormal write, read;
+    u32 fault_fold;
+    __device__ __forceinline__ LowCells(u32 seed, u64 read_seed)
+        : write(seed, 10u), read(read_seed, 20u), fault_fold(uniform_fold(0u, seed, 30u)) {}
+    __device__ __forceinline__ float operator()(const mf_config &cfg, u32 code, int w,
+                                                u32 cell) const {
+        const int mask = cfg.w_mask[w];
+        const int digit = int((code >> cfg.w_shift[w]) & u32(mask));
+        float raw = nominal_level<float>(cfg, digit, mask);
+        if (cfg.has_write) raw = raw * exp_small(cfg.f_write * write(cell));
+        raw = raw * cfg.f_drift;
+        if (cfg.has_saf) {
+            const float u = uniform_finish(cell, fault_fold);
+            if (u < cfg.f_saf_low) raw = cfg.f_low;
+            else if (u < cfg.f_saf_band) raw = cfg.f_high;
+        }
+        if (cfg.read_mode == MF_READ_SHARED && cfg.has_read)
+            raw = raw * exp_small(cfg.f_read * read(cell));
+        return raw;
+    }
+};
+
+// Conductances of eight cells of one column, `stride` apart.  `low`: wave-uniform, every
+// address is below 2^32 (a matrix of up to 4.3e9 cells and slices).
+__device__ __forceinline__ void cell_column(const mf_config &cfg, const u32 (&codes)[8], int w,
+                                            u64 cell, int stride, u32 seed, u64 read_seed, bool low,
+                                            float (&level)[8]) {
+    if (low) {
+        const LowCells cells(seed, read_seed);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) level[j] = cells(cfg, codes[j], w, u32(cell) + u32(j * stride));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            level[j] = cell_conductance<float>(cfg, codes[j], w, cell + u64(j) * stride, seed,
+                                               read_seed);
+    }
+}
+
+// One fp16 pair (hi, lo) of x, added to packed operands as element j of eight.
+__device__ __forceinline__ void put_terms(float x, int j, u32 (&hi4)[4], u32 (&lo4)[4]) {
+    const _Float16 hi = static_cast<_Float16>(x);   // round to nearest even
+    const _Float16 lo = static_cast<_Float16>(x - static_cast<float>(hi));
+    const int shift = 16 * (j & 1);
+    hi4[j >> 1] |= u32(__builtin_bit_cast(unsigned short, hi)) << shift;
+    lo4[j >> 1] |= u32(__builtin_bit_cast(unsigned short, lo)) << shift;
+}
+
 }  // namespace mf

@@ -122,6 +122,8 @@ __global__ void k_codes16(const u32 *q, i64 count, uint16_t *q16) {
         q16[i] = uint16_t(q[i]);
 }
 
+// Grid: 32-column blocks, four (read, 16-row step) units per block (one a wave), weight slices,
+// as k_split_conductances.  4096 x 4096 cells of three slices: 141 us, 226 before.
 template <int KS>
 __global__ __launch_bounds__(256) void k_split_wide(const mf_config cfg, const u32 *packed,
                                                     const float *g_in, i64 m, i64 p, i64 ncols,
@@ -129,56 +131,61 @@ __global__ __launch_bounds__(256) void k_split_wide(const mf_config cfg, const u
                                                     const NoisyWidePlan plan, uint4 *gs) {
     constexpr int P = 16 * KS;
     const int R = cfg.rows, C = cfg.cols, W = cfg.n_w;
-    const i64 G = m * R / P;
-    const i64 total = CB * G * W * plan.planes * KS * 64;
+    const int G = int(m * R / P);
+    const int lane = threadIdx.x & 63;
+    const int unit = __builtin_amdgcn_readfirstlane(int(blockIdx.y) * 4 + int(threadIdx.x >> 6));
+    const int g = unit / KS, ks = unit % KS;
+    if (g >= G) return;
+    const i64 cb = blockIdx.x;
+    const int w = blockIdx.z;
     const u64 read_seed = event_seed(seed, event);
-    for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-         t += i64(gridDim.x) * blockDim.x) {
-        i64 rest = t;
-        const int lane = int(rest & 63); rest >>= 6;
-        const int ks = int(rest % KS); rest /= KS;
-        const int vw = int(rest % (W * plan.planes)); rest /= W * plan.planes;
-        const int plane = vw / W, w = vw - plane * W;   // planes outermost: [plane][w]
-        const i64 g = rest % G;
-        const i64 cb = rest / G;
-        const int lr = lane & 31, h = lane >> 5;
-        const i64 c = c_begin + cb * 32 + lr;
-        const i64 k0 = g * P + ks * 16 + h * 8;
-        u32 terms[2][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-        if (c < ncols) {
-            const i64 i = k0 / R, r0 = k0 - i * R;
-            const i64 tt = c / C, cc = c - tt * C;
+    const int lr = lane & 31, h = lane >> 5;
+    const i64 c = c_begin + cb * 32 + lr;
+    const bool live = c < ncols;
+    const int per_array = R / P, i = g / per_array;
+    const int r0 = (g - i * per_array) * P + ks * 16 + h * 8;   // row in the array
+    float level[8] = {};
+    u64 cell = 0;
+    if (live) {
+        const u32 tt = u32(c) / u32(C), cc = u32(c) - tt * u32(C);
+        const i64 tile = i64(i) * p + tt;
+        cell = u64((tile * W + w) * R + r0) * u64(C) + cc;
+        if (g_in) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) level[j] = g_in[cell + u64(j) * C];
+        } else {
+            const u32 *src = packed + (tile * R + r0) * C + cc;
+            u32 codes[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) codes[j] = src[j * C];
+            cell_column(cfg, codes, w, cell, C, seed, read_seed,
+                        m * p * W * R * C <= (i64(1) << 32), level);
+        }
+    }
+    // slice_pair read noise (memfast/reference.py:86-90): a read factor per (cell, input slice),
+    // one plane of terms per input slice, planes outermost.
+    const bool low = m * p * W * R * C * cfg.n_in <= (i64(1) << 32);
+    const LowNormal pair_noise(read_seed, 20u);
+    for (int plane = 0; plane < plan.planes; ++plane) {
+        u32 hi4[4] = {0u, 0u, 0u, 0u}, lo4[4] = {0u, 0u, 0u, 0u};
+        if (live) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const i64 r = r0 + j;
-                const u64 cell = u64((((i * p + tt) * W + w) * R + r) * C + cc);
-                float level;
-                if (g_in) {
-                    level = g_in[cell];
-                } else {
-                    const u32 code = packed[((i * p + tt) * R + r) * C + cc];
-                    level = cell_conductance<float>(cfg, code, w, cell, seed, read_seed);
+                float g_read = level[j];
+                if (plan.planes > 1) {
+                    const u64 address = (cell + u64(j) * C) * u64(cfg.n_in) + u64(plane);
+                    const float z = low ? pair_noise(u32(address))
+                                        : normal_fast(address, read_seed, 20u);
+                    g_read = g_read * exp_small(cfg.f_read * z);
                 }
-                // slice_pair read noise (memfast/reference.py:86-90): a read factor per
-                // (cell, input slice), one plane of terms per input slice.
-                if (plan.planes > 1)
-                    level = level * exp_small(cfg.f_read *
-                                              normal_fast(cell * u64(cfg.n_in) + u64(plane),
-                                                          read_seed, 20u));
-                const float delta = (level - cfg.f_low) * plan.k1[w];   // ADC counts per digit
-                const _Float16 hi = static_cast<_Float16>(delta);        // round to nearest even
-                const _Float16 lo = static_cast<_Float16>(delta - static_cast<float>(hi));
-                const int shift = 16 * (j & 1);
-                terms[0][j >> 1] |= u32(__builtin_bit_cast(unsigned short, hi)) << shift;
-                terms[1][j >> 1] |= u32(__builtin_bit_cast(unsigned short, lo)) << shift;
+                put_terms((g_read - cfg.f_low) * plan.k1[w], j, hi4, lo4);   // ADC counts per digit
             }
         }
+        const i64 vw = i64(plane) * W + w;
         uint4 *dst = gs + ((((cb * G + g) * W * plan.planes + vw) * NOISY_TERMS) * KS + ks) * 64 +
                      lane;
-#pragma unroll
-        for (int term = 0; term < NOISY_TERMS; ++term)
-            dst[term * KS * 64] = make_uint4(terms[term][0], terms[term][1], terms[term][2],
-                                             terms[term][3]);
+        dst[0] = make_uint4(hi4[0], hi4[1], hi4[2], hi4[3]);
+        dst[KS * 64] = make_uint4(lo4[0], lo4[1], lo4[2], lo4[3]);
     }
 }
 
