@@ -799,6 +799,54 @@ bool wide_extent_ok(i64 n, i64 m, const mf_config *cfg) {
     return 64 * kp <= 0x7FFFFFFF && (n + 127) / 128 <= 65535;
 }
 
+i64 wide_small_bytes(const mf_config *cfg, i64 n, i64 m, i64 p) {
+    return align256(n * m * cfg->reads * p * cfg->cols * 4);
+}
+
+// Batches that k_wide_small reads: no per-vector or per-slice noise (a tuned schedule's LDS tier
+// asks for k_noisy_wide), totals that fit where the terms would be, and where its time is the
+// lesser.  Both sample every cell once (2.8 ps per cell and weight slice).  Beside that, per read
+// and pair of slices, k_wide_small takes 0.33 ps per column and vector of its blocks of 32, and its
+// sum 1 ps per read, column and vector; k_noisy_wide takes 0.27 us per round of 768 workgroups (128
+// vectors by 32 columns, three per CU) and 0.17 us per workgroup on a CU, however few of its vectors
+// are used.  Nine by three slices, 64-row reads, both with their sampling or sum: 4096 x 4096 at 32
+// vectors 0.23 against 0.87 ms, at 128 0.47 / 0.90, at 190 0.63 / 0.91; 4096 x 11008 at 4 vectors
+// 0.55 / 1.30, at 128 1.27 / 1.38, at 190 1.72 / 1.76; 1024 x 1024 at 128 0.05 / 0.20.
+bool wide_small(const mf_config *cfg, i64 n, i64 m, i64 p, int tier_request) {
+    const i64 reads = m * cfg->reads, ncols = p * cfg->cols, blocks = (ncols + 31) / 32;
+    if (cfg->has_vnoise || wide_term_planes(cfg) > 1 || tier_request != 0 || n > 65535 ||
+        reads > 65535 || wide_small_bytes(cfg, n, m, p) > blocks * wide_block_bytes(cfg, m))
+        return false;
+    const i64 groups = blocks * ((n + 127) / 128);
+    const double pairs = double(cfg->n_in) * cfg->n_w;
+    const double small = double((n + 31) / 32 * 32) * double(ncols) * (0.33e-6 + 1e-6 / pairs);
+    const double large = 0.27 * double((groups + 767) / 768) + 0.17 * double((groups + 255) / 256);
+    return small < large;
+}
+
+int launch_wide_small(const mf_config *cfg, const NoisyWidePlan &plan, int ks, const u32 *q,
+                      const double *xscale, i64 n, i64 m, const u32 *packed, const double *wscale,
+                      i64 p, u32 seed, u64 event, double *out, i64 ldo, int *totals, u32 *status,
+                      hipStream_t s) {
+    const i64 ncols = p * cfg->cols, G = m * cfg->reads;
+    const dim3 grid{unsigned((ncols + 31) / 32), unsigned(G), 1u}, block{unsigned(64 * cfg->n_w)};
+#define MF_SMALL_LAUNCH(KS, NL)                                                                  \
+    hipLaunchKernelGGL((k_wide_small<KS, NL>), grid, block, 0, s, *cfg, packed, m, p, seed,        \
+                       event, plan, q, n, ncols, totals)
+    if (ks == 4) {
+        if (cfg->has_nonlinear) MF_SMALL_LAUNCH(4, true);
+        else MF_SMALL_LAUNCH(4, false);
+    } else {
+        if (cfg->has_nonlinear) MF_SMALL_LAUNCH(2, true);
+        else MF_SMALL_LAUNCH(2, false);
+    }
+#undef MF_SMALL_LAUNCH
+    hipLaunchKernelGGL(k_restore_sum_wide, dim3(unsigned((ncols + 255) / 256), unsigned(n)),
+                       dim3(256), 0, s, totals, n, int(G), ncols, xscale, wscale, ncols, out, ldo,
+                       status);
+    return check_launch("small wide MFMA read");
+}
+
 // Repack codes to 16 bits, split conductances and run k_noisy_wide over column
 // chunks that fit the workspace.  g: optional injected conductances.
 int launch_noisy_wide(const mf_config *cfg, const NoisyWidePlan &plan, int ks,
@@ -1610,6 +1658,7 @@ int mf_mm_workspace(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32
         // At least the two 32-column blocks the wide read's chunking needs, even for
         // outputs narrower than 64 columns.
         const i64 blocks = std::max<i64>(2, (p * cfg->cols + 31) / 32);
+        // (k_wide_small's totals need no more: wide_small)
         *bytes = wide_prefix_bytes(n, m, cfg) + blocks * wide_block_bytes(cfg, m);
     } else {
         *bytes = mfma32_scratch(cfg, n, m, p);
@@ -2410,16 +2459,22 @@ int mf_mm_wide(const mf_config *cfg, const uint32_t *q, const double *xscale, in
     NoisyWidePlan wplan;
     int ks = 0;
     const char *why = "";
+    // (a workspace of terms that does not hold a small read's totals runs k_noisy_wide)
+    const bool small = wide_small(cfg, n, m, p, variant_tier(variant)) &&
+                       workspace_bytes >= wide_small_bytes(cfg, n, m, p);
     if (!g && workspace && (reinterpret_cast<uintptr_t>(workspace) % 256) == 0 &&
         wide_extent_ok(n, m, cfg) && build_noisy_wide_plan(cfg, m, p, &wplan, &ks, &why) &&
-        workspace_bytes >= wide_prefix_bytes(n, m, cfg) + 2 * wide_block_bytes(cfg, m)) {
+        (small || workspace_bytes >= wide_prefix_bytes(n, m, cfg) + 2 * wide_block_bytes(cfg, m))) {
         hipStream_t s = static_cast<hipStream_t>(stream);
         std::pair<hipEvent_t, hipEvent_t> timing{nullptr, nullptr};
         if (profiling() && (timing = profile_pair()).first) hipEventRecord(timing.first, s);
-        const int launched = launch_noisy_wide(cfg, wplan, ks, q, xscale, n, m, packed,
-                                               wscale, p, nullptr, seed, event, out, ldo,
-                                               workspace, workspace_bytes, 0, status, s,
-                                               variant_tier(variant));
+        const int launched =
+            small
+                ? launch_wide_small(cfg, wplan, ks, q, xscale, n, m, packed, wscale, p, seed, event,
+                                    out, ldo, static_cast<int *>(workspace), status, s)
+                : launch_noisy_wide(cfg, wplan, ks, q, xscale, n, m, packed, wscale, p, nullptr,
+                                    seed, event, out, ldo, workspace, workspace_bytes, 0, status, s,
+                                    variant_tier(variant));
         if (timing.first) {
             hipEventRecord(timing.second, s);
             profile_push(timing);
@@ -2593,6 +2648,14 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                   : tier == 1 ? MF_WIDE_FN(2, WIDE_FRAGS_SMALL) : MF_WIDE_FN(2, WIDE_FRAGS_TINY);
 #undef MF_WIDE_FN
 #undef MF_WIDE_FN2
+        // (the matrix is not known here: one of 64 x 64 arrays)
+        if (n > 0 && wide_small(cfg, n, 64, 64, variant_tier(variant))) {
+            fn = ks4 ? (nl ? reinterpret_cast<const void *>(&k_wide_small<4, true>)
+                           : reinterpret_cast<const void *>(&k_wide_small<4, false>))
+                     : (nl ? reinterpret_cast<const void *>(&k_wide_small<2, true>)
+                           : reinterpret_cast<const void *>(&k_wide_small<2, false>));
+            threads = 64 * cfg->n_w;
+        }
     } else if (kernel_id == 0) {
 #define MF_GENERAL_FN(WIDE)                                                                      \
     (cfg->precise                                                                                \

@@ -281,6 +281,15 @@ template <int KS>
 __global__ void k_split_wide(const mf_config cfg, const u32 *packed, const float *g_in, i64 m,
                              i64 p, i64 ncols, u32 seed, u64 event, i64 c_begin, i64 CB,
                              const NoisyWidePlan plan, uint4 *gs);
+// The wide read of small batches, conductances sampled in place: integer totals [n, G, ncols]
+// (grid: 32-column blocks, reads; one wave per weight slice), and their FP64 restore and sum.
+template <int KS, bool NONLINEAR>
+__global__ void k_wide_small(const mf_config cfg, const u32 *packed, i64 m, i64 p, u32 seed,
+                             u64 event, const NoisyWidePlan plan, const u32 *q, i64 n, i64 ncols,
+                             int *totals);
+__global__ void k_restore_sum_wide(const int *totals, i64 n, int G, i64 ncols, const double *xscale,
+                                   const double *wscale, i64 ldws, double *out, i64 ldo,
+                                   u32 *status);
 // LDS capacity of the wide read: fragments (1 KiB) per read and buffer.  24:
 // two buffers in 48 KiB (three blocks per CU); 36: 72 KiB (two blocks per CU);
 // 72: 144 KiB (one block per CU).

@@ -194,6 +194,152 @@ template __global__ void k_split_wide<2>(const mf_config, const u32 *, const flo
 template __global__ void k_split_wide<4>(const mf_config, const u32 *, const float *, i64, i64,
                                          i64, u32, u64, i64, i64, const NoisyWidePlan, uint4 *);
 
+// The read of small batches: conductances are sampled where they are used and never reach
+// memory.  Workgroup = one 32-column block and one read, one wave per weight slice: each wave
+// samples its slice's terms into registers, in k_split_wide's order, then walks the batch in
+// tiles of 32 vectors (digits from the 32-bit codes, k_noisy_wide's MFMA order and converter);
+// the waves' totals meet in LDS and go out as 32-bit integers [n, G, ldo], which k_restore_sum_wide
+// restores and sums.  Shared read noise or none, digit operands.
+// Why: at 4 tokens a 4096 -> 11008 projection wrote and read back 540 MB of terms (583 us of
+// sampling and stores) for a read that used 4 of its 128 vector lanes in 344 serial workgroups
+// (913 us); now 529 us and 13 us for the sum.  Bound: the sampling's VALU work (two hashed normals
+// per cell with programming and read noise, about 130 issue slots).
+template <int KS, bool NONLINEAR>
+__global__ __launch_bounds__(512) void k_wide_small(const mf_config cfg, const u32 *packed, i64 m,
+                                                    i64 p, u32 seed, u64 event,
+                                                    const NoisyWidePlan plan, const u32 *q, i64 n,
+                                                    i64 ncols, int *totals) {
+    constexpr int P = 16 * KS;
+    __shared__ u32 planes[WIDE_MFMA_MAX_W][16][64];
+    const float MAGIC = 12582912.0f;   // 1.5 * 2^23
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 31, h = lane >> 5;
+    const int R = cfg.rows, C = cfg.cols, W = cfg.n_w, A = plan.n_in;
+    const int g = blockIdx.y, Gr = cfg.reads, G = int(m) * Gr;
+    const i64 kp = m * R;
+    const int i = g / Gr, row0 = (g - i * Gr) * P;
+    const i64 col_tile = i64(blockIdx.x) * 32;
+    const u64 read_seed = event_seed(seed, event);
+
+    // Terms of (column lr, rows ks*16 + h*8 + j) of weight slice w.
+    v8h_w F[NOISY_TERMS][KS];
+    {
+        const i64 c = col_tile + lr < ncols ? col_tile + lr : ncols - 1;   // (not written past it)
+        const u32 tt = u32(c) / u32(C), cc = u32(c) - tt * u32(C);
+        const i64 tile = (i64(i) * p + tt) * R + row0;    // first cell row of this read
+        const u32 *codes = packed + tile * C + cc;
+        const u64 cell0 = u64(((i64(i) * p + tt) * W + w) * R + row0) * u64(C) + cc;
+        const bool low = m * p * W * R * C <= (i64(1) << 32);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int at = (ks * 16 + h * 8) * C;
+            u32 hi4[4] = {0u, 0u, 0u, 0u}, lo4[4] = {0u, 0u, 0u, 0u};
+            u32 code[8];
+            float level[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) code[j] = codes[at + j * C];
+            cell_column(cfg, code, w, cell0 + u32(at), C, seed, read_seed, low, level);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                put_terms((level[j] - cfg.f_low) * plan.k1[w], j, hi4, lo4);   // ADC counts
+            F[0][ks] = __builtin_bit_cast(v8h_w, make_uint4(hi4[0], hi4[1], hi4[2], hi4[3]));
+            F[1][ks] = __builtin_bit_cast(v8h_w, make_uint4(lo4[0], lo4[1], lo4[2], lo4[3]));
+        }
+    }
+    const float top = MAGIC + plan.top[w], alpha = plan.alpha[w];
+    const u32 magic16 = 0x64006400u;   // fp16 1024 in both halves (digits_magic)
+    for (i64 v0 = 0; v0 < n; v0 += 32) {
+        const i64 v = v0 + lr;
+        const u32 *row = q + (v < n ? v : n - 1) * kp + i64(i) * R + row0;
+        uint4 qc[KS];   // eight 16-bit codes each
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const u32 *src = row + ks * 16 + h * 8;
+            // Low halves of two codes each.
+            qc[ks] = make_uint4(__builtin_amdgcn_perm(src[1], src[0], 0x05040100u),
+                                __builtin_amdgcn_perm(src[3], src[2], 0x05040100u),
+                                __builtin_amdgcn_perm(src[5], src[4], 0x05040100u),
+                                __builtin_amdgcn_perm(src[7], src[6], 0x05040100u));
+        }
+        u32 T[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) T[r] = 0u;
+        for (int a = 0; a < A; ++a) {
+            v16f_w I = {};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const v8h_w B = digits_magic(qc[ks], plan.in_shift[a], plan.in_mask2[a], magic16);
+#pragma unroll
+                for (int term = 0; term < NOISY_TERMS; ++term)
+                    I = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[term][ks], B, I, 0, 0, 0);
+            }
+            const int f = plan.fa[a] * plan.fw[w];   // |fa*fw| < 2^23
+            const u32 f24 = u32(int(u32(f) << 8) >> 8);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float y = (NONLINEAR ? scurve(I[r], alpha) : I[r]) + MAGIC;
+                y = __builtin_amdgcn_fmed3f(y, MAGIC, top);
+                T[r] += u32(int(__float_as_uint(y) << 8) >> 8) * f24;
+            }
+        }
+        __syncthreads();   // the previous tile's totals are read
+#pragma unroll
+        for (int r = 0; r < 16; ++r) planes[w][r][lane] = T[r];
+        __syncthreads();
+        for (int r = w; r < 16; r += W) {
+            u32 total = plan.bias;
+            for (int k = 0; k < W; ++k) total += planes[k][r][lane];
+            const i64 c = col_tile + (r >> 2) * 8 + h * 4 + (r & 3);
+            if (v < n && c < ncols) totals[(v * G + g) * ncols + c] = int(total);
+        }
+    }
+}
+
+template __global__ void k_wide_small<2, false>(const mf_config, const u32 *, i64, i64, u32, u64,
+                                                const NoisyWidePlan, const u32 *, i64, i64, int *);
+template __global__ void k_wide_small<2, true>(const mf_config, const u32 *, i64, i64, u32, u64,
+                                               const NoisyWidePlan, const u32 *, i64, i64, int *);
+template __global__ void k_wide_small<4, false>(const mf_config, const u32 *, i64, i64, u32, u64,
+                                                const NoisyWidePlan, const u32 *, i64, i64, int *);
+template __global__ void k_wide_small<4, true>(const mf_config, const u32 *, i64, i64, u32, u64,
+                                               const NoisyWidePlan, const u32 *, i64, i64, int *);
+
+// Restored totals summed over reads as k_noisy_wide sums them (FP64 cascade, fewer than 256
+// reads).  A batch of reads is loaded before its values enter the sum.
+__global__ __launch_bounds__(256) void k_restore_sum_wide(const int *totals, i64 n, int G, i64 ncols,
+                                                          const double *xscale,
+                                                          const double *wscale, i64 ldws,
+                                                          double *out, i64 ldo, u32 *status) {
+    constexpr int BATCH = 8;
+    const i64 c = i64(blockIdx.x) * blockDim.x + threadIdx.x;
+    const i64 v = blockIdx.y;
+    if (c >= ncols) return;
+    double acc0 = 0.0, acc1 = 0.0;
+    for (int g0 = 0; g0 < G; g0 += BATCH) {
+        int t[BATCH];
+        double ws[BATCH];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+            const int g = g0 + j < G ? g0 + j : G - 1;   // past the end: unused
+            t[j] = totals[(v * G + g) * ncols + c];
+            ws[j] = wscale[i64(g) * ldws + c];
+        }
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+            if (g0 + j >= G) break;
+            acc0 = acc0 + restore_fast(t[j], xscale[v * G + g0 + j], ws[j]);
+            if (((g0 + j + 1) & 15) == 0) {
+                acc1 = g0 + j + 1 == 16 ? acc0 : acc1 + acc0;
+                acc0 = 0.0;
+            }
+        }
+    }
+    const double s = acc0 + (G >= 16 ? acc1 : 0.0);
+    out[v * ldo + c] = s;
+    if (!(fabs(s) <= DBL_MAX) && status) atomicOr(status, u32(MF_STATUS_OUTPUT));
+}
+
 template <int KS, bool NONLINEAR, int FRMAX, bool VNOISE, bool SLICE>
 __global__ __launch_bounds__(256, wide_blocks_per_cu(FRMAX, NONLINEAR)) void k_noisy_wide(
     const NoisyWidePlan plan,
