@@ -1243,10 +1243,18 @@ int mf_conv_input_tiles(const mf_config *cfg, const float *x, const mf_conv_geom
     const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)((kp + CONV_CHUNK_COLS - 1) / CONV_CHUNK_COLS));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int vec = kp % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
+    // The tap table: 32-bit byte offsets where the images of 64 rows lie within 2 GiB.
+    const i64 images = 63 / (g.out_height * g.out_width) + 2;
+    const bool far = std::min(images, g.n) * g.channels * g.height * g.width > 0x1FFFFFFF;
+    const i64 kk = i64(g.kh) * g.kw;
+    const u32 lds = u32((std::min<i64>(kk, CONV_CHUNK_COLS) + 1) * 64 * (far ? 8 : 4));
+    // A block takes several chunks of columns where there are rows enough for 4096 blocks (its tap
+    // table serves them all): 200704 patches of 576 columns 86 us; 90 with one block per 64 rows.
+    const dim3 loops(grid.x, std::min(grid.y, (4095 + grid.x) / grid.x));
     if (fixed_scale) {
-        hipLaunchKernelGGL(k_conv_codes, grid, dim3(256), 0, s, x, g, K, kp, fixed_scale, i64(1),
-                           i64(0), i64(1), -upper, upper, mask, q, vec, status,
-                           u32(MF_STATUS_INPUT));
+        hipLaunchKernelGGL((far ? k_conv_codes<u64, true> : k_conv_codes<u32, true>), loops,
+                           dim3(256), lds, s, x, g, K, kp, fixed_scale, i64(1), i64(0), i64(1),
+                           -upper, upper, mask, q, vec, status, u32(MF_STATUS_INPUT));
         hipLaunchKernelGGL(k_input_scales, dim3(grid_for(rows * m * Gr)), dim3(256), 0, s, rows, K,
                            m * Gr, R, P, Gr, fixed_scale, i64(1), i64(1), K, 1, xscale);
         return check_launch("conv input tiles");
@@ -1257,12 +1265,13 @@ int mf_conv_input_tiles(const mf_config *cfg, const float *x, const mf_conv_geom
     gc = gc < K ? gc : K;
     const i64 nrg = (rows + gr - 1) / gr, ncg = (K + gc - 1) / gc;
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(nrg * ncg)), dim3(256), 0, s, work, nrg * ncg, 0u);
-    hipLaunchKernelGGL(k_conv_group_max, dim3(unsigned((rows + 255) / 256)), dim3(256), 0, s, x, g,
-                       K, gr, gc, ncg, work, status, u32(MF_STATUS_INPUT));
+    hipLaunchKernelGGL((far ? k_conv_group_max<u64> : k_conv_group_max<u32>), grid, dim3(256), lds,
+                       s, x, g, K, gr, gc, ncg, work, status, u32(MF_STATUS_INPUT));
     hipLaunchKernelGGL(k_group_scale, dim3(grid_for(nrg * ncg)), dim3(256), 0, s, work, nrg * ncg,
                        upper, scale);
-    hipLaunchKernelGGL(k_conv_codes, grid, dim3(256), 0, s, x, g, K, kp, scale, gr, gc, ncg, -upper,
-                       upper, mask, q, vec, status, u32(MF_STATUS_INPUT));
+    hipLaunchKernelGGL((far ? k_conv_codes<u64, false> : k_conv_codes<u32, false>), loops,
+                       dim3(256), lds, s, x, g, K, kp, scale, gr, gc, ncg, -upper, upper, mask, q, vec, status,
+                       u32(MF_STATUS_INPUT));
     hipLaunchKernelGGL(k_input_scales, dim3(grid_for(rows * m * Gr)), dim3(256), 0, s, rows, K,
                        m * Gr, R, P, Gr, scale, gr, gc, ncg, 0, xscale);
     return check_launch("conv input tiles");

@@ -922,185 +922,311 @@ template __global__ void k_input_codes4<i64>(const float *, i64, i64, i64, i64, 
 // outside the image.  Lanes own consecutive patch rows, so for one k a wave reads
 // neighbouring pixels of one image row (coalesced); k is uniform across the wave and
 // its (c, i, j) decomposition advances incrementally in scalar registers.
-struct ConvLane {
-    i64 pixel;    // offset of x[b, c0, ih0, iw0] (may point outside the image)
-    int ih0, iw0;
-};
+// A block's 64 rows (one a lane) and the taps of CONV_CHUNK columns: `table` [taps + 1][64] holds
+// where tap (i, j) lies from the block's first image and channel on, NONE outside its image or past
+// the rows.  The taps of a kernel of up to CONV_CHUNK in order, else one per column from tap
+// `first` on; the last entry is the tap of columns past the patch.
+// Off u32: byte offsets of a buffer of less than 2 GiB, where NONE is past the end and loads zero;
+// u64: elements.
+template <typename Off>
+struct ConvTile {
+    static constexpr bool BUFFER = sizeof(Off) == 4;
+    static constexpr Off NONE = BUFFER ? Off(0x80000000u) : ~Off(0);
+    const float *base;   // the block's first image, the group's first channel
+    __amdgpu_buffer_rsrc_t buffer;
+    Off *table;
+    i64 hw;
+    int kk, taps;
 
-__device__ __forceinline__ ConvLane conv_lane(const mf_conv_geometry &g, u32 row) {
-    const u32 wo = u32(g.out_width), L = u32(g.out_height) * wo;
-    const u32 b = row / L, l = row - b * L;
-    const u32 oh = l / wo, ow = l - oh * wo;
-    ConvLane lane;
-    lane.ih0 = int(oh) * g.sh - g.ph;
-    lane.iw0 = int(ow) * g.sw - g.pw;
-    lane.pixel = (i64(b) * g.channels + g.c0) * g.height * g.width + i64(lane.ih0) * g.width +
-                 lane.iw0;
-    return lane;
-}
-
-// Position (c, i, j) of column k in the patch and its offset from the patch origin.
-struct ConvTap {
-    int c, i, j;
-    i64 delta;   // c*H*W + i*dh*W + j*dw
-    int di, dj;  // i*dh, j*dw
-
-    __device__ __forceinline__ void start(const mf_conv_geometry &g, int k) {
-        const int kk = g.kh * g.kw;
-        c = k / kk;
-        const int rem = k - c * kk;
-        i = rem / g.kw;
-        j = rem - i * g.kw;
-        di = i * g.dh;
-        dj = j * g.dw;
-        delta = i64(c) * g.height * g.width + i64(di) * g.width + dj;
+    __device__ __forceinline__ ConvTile(const float *x, const mf_conv_geometry &g, u32 r0,
+                                        Off *table_)
+        : table(table_), hw(i64(g.height) * g.width), kk(g.kh * g.kw) {
+        taps = kk < CONV_CHUNK_COLS ? kk : CONV_CHUNK_COLS;
+        const u32 image = r0 / u32(g.out_height * g.out_width);
+        base = x + (i64(image) * g.channels + g.c0) * hw;
+        const i64 bytes = ((g.n - image) * g.channels - g.c0) * hw * 4;
+        buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), short(0),
+                                                   bytes > 0x7FFFFFFF ? 0x7FFFFFFF : int(bytes),
+                                                   0x00020000);
     }
-    __device__ __forceinline__ void next(const mf_conv_geometry &g) {
-        if (++j < g.kw) {
-            dj += g.dw;
-            delta += g.dw;
-            return;
+    __device__ __forceinline__ void fill(const mf_conv_geometry &g, u32 r0, u32 row, bool live,
+                                         int first) {
+        const u32 wo = u32(g.out_width), L = u32(g.out_height) * wo;
+        const u32 image = row / L, l = row - image * L;
+        const u32 oh = l / wo, ow = l - oh * wo;
+        const int ih0 = int(oh) * g.sh - g.ph, iw0 = int(ow) * g.sw - g.pw;
+        const i64 at = i64(image - r0 / L) * g.channels * hw;
+        for (int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t <= taps; t += 4) {
+            const int tap = (first + t) % kk, i = tap / g.kw, j = tap - i * g.kw;
+            const u32 ih = u32(ih0 + i * g.dh), iw = u32(iw0 + j * g.dw);
+            const bool in = live && t < taps && ih < u32(g.height) && iw < u32(g.width);
+            const i64 element = at + i64(ih) * g.width + iw;
+            table[t * 64 + (threadIdx.x & 63)] = in ? Off(BUFFER ? element * 4 : element) : NONE;
         }
-        j = 0;
-        delta -= i64(dj);
-        dj = 0;
-        if (++i < g.kh) {
-            di += g.dh;
-            delta += i64(g.dh) * g.width;
-            return;
-        }
-        i = 0;
-        delta += i64(g.height - di) * g.width;
-        di = 0;
-        ++c;
     }
 };
 
-__device__ __forceinline__ float conv_load(const float *x, const mf_conv_geometry &g,
-                                           const ConvLane &lane, bool live, const ConvTap &t) {
-    const u32 ih = u32(lane.ih0 + t.di), iw = u32(lane.iw0 + t.dj);
-    return live && ih < u32(g.height) && iw < u32(g.width) ? x[lane.pixel + t.delta] : 0.0f;
-}
+// Walks a wave's columns from k0 on, N at a time (offsets from the table first, so that the loads
+// are in flight together).  Columns are counted in scalar registers.
+template <typename Off>
+struct ConvWalk {
+    const ConvTile<Off> &tile;
+    const Off *table;
+    Off channel, step;   // the current column's channel from the group's first, and one channel
+    int left;            // columns of the patch from the current one on
+    int tap, slot;
 
-// Codes q [rows, kp] (zero past K) for a tile of 64 rows x CONV_CHUNK columns per
-// block, with a fixed per-column scale (gc == 0) or per-(gr rows, gc columns) group
-// scales [ceil(rows/gr), ncg].  Each wave quantizes CONV_CHUNK/4 columns of the 64
-// rows into LDS; the block then writes whole row segments.
+    __device__ __forceinline__ ConvWalk(const ConvTile<Off> &tile_, i64 K, i64 kc, i64 k0)
+        : tile(tile_), table(tile_.table + (threadIdx.x & 63)),
+          step(Off(tile_.hw) * (ConvTile<Off>::BUFFER ? 4 : 1)), left(int(K - k0)) {
+        const int c = __builtin_amdgcn_readfirstlane(int(k0) / tile.kk);
+        tap = int(k0) - c * tile.kk;
+        slot = int(k0 - kc);
+        channel = Off(c) * step;
+    }
+    __device__ __forceinline__ float load(Off off, Off from) const {
+        if constexpr (ConvTile<Off>::BUFFER) {
+            return __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(tile.buffer, int(off), int(from), 0));
+        } else {
+            const float v = tile.base[off != ConvTile<Off>::NONE ? from + off : 0];
+            return off != ConvTile<Off>::NONE ? v : 0.0f;
+        }
+    }
+    template <int N>
+    __device__ __forceinline__ void values(float (&v)[N]) {
+        Off off[N], from[N];
+        if (left >= N && tile.kk <= tile.taps) {   // few scalar instructions
+#pragma unroll
+            for (int t = 0; t < N; ++t) {
+                off[t] = table[tap * 64];
+                from[t] = channel;
+                const bool turn = tap + 1 == tile.kk;
+                channel += turn ? step : Off(0);   // at most one past the last
+                tap = turn ? 0 : tap + 1;
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < N; ++t) {
+                const bool in = t < left;
+                off[t] = table[(!in ? tile.taps : tile.kk <= tile.taps ? tap : slot + t) * 64];
+                from[t] = channel;
+                if (++tap == tile.kk) {
+                    tap = 0;
+                    if (t + 1 < left) channel += step;
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < N; ++t) v[t] = load(off[t], from[t]);
+        slot += N;
+        left -= N;
+    }
+};
+
+// Codes q [rows, kp] (zero past K) for a tile of 64 rows x CONV_CHUNK columns per block, with a
+// fixed per-column scale (FIXED) or per-(gr rows, gc columns) group scales [ceil(rows/gr), ncg].
+// Each wave quantizes CONV_CHUNK/4 columns of the 64 rows into LDS, 16 values in flight, their
+// addresses from the tap table; the block then writes whole row segments.
+// A code is rint(RN(v / s)), clamped.  With r = RN(1/s), |v*r - v/s| and |RN(v/s) - v/s| are below
+// 2^-16 up to |v/s| = 128 (the codes end at 127; beyond, both clamp), so where the exact v*r is
+// further than 2^-15 from a tie, one FMA with 1.5 * 2^23 rounds to the same code.  Words with a
+// value nearer a tie (1 value in 2^14), not finite, or of a scale without such an r divide.
+// Bound: instruction issue, 17 vector and 14 scalar instructions per code and 64 rows where
+// division, 64-bit taps and their branches took about 50 and 80.  200704 patches of 576 columns:
+// 86 us, 187 before (reading and writing its 167 MB: 33 us).
 constexpr int CONV_CHUNK = CONV_CHUNK_COLS;
 constexpr int CONV_PITCH = CONV_CHUNK / 4 + 1;   // dwords per LDS row (odd: no conflicts)
 
+template <typename Off, bool FIXED>
 __global__ __launch_bounds__(256) void k_conv_codes(const float *x, const mf_conv_geometry g,
                                                     i64 K, i64 kp, const float *scale, i64 gr,
                                                     i64 gc, i64 ncg, float lower, float upper,
                                                     u32 mask, u8 *q, int vec, u32 *status,
                                                     u32 flag) {
+    extern __shared__ u64 conv_table[];
     __shared__ u32 tile[64 * CONV_PITCH];
+    const float MAGIC = 12582912.0f, CLEAR = 0.5f - 1.0f / 32768.0f;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 rows = g.n * g.out_height * g.out_width;
+    const i64 r0 = i64(blockIdx.x) * 64;
+    const bool live = r0 + lane < rows;
+    const u32 row = u32(live ? r0 + lane : r0);
+    ConvTile<Off> rows64(x, g, u32(r0), reinterpret_cast<Off *>(conv_table));
+    const bool one_table = rows64.kk <= rows64.taps;
+    if (one_table) rows64.fill(g, u32(r0), row, live, 0);
+    constexpr int CPW = CONV_CHUNK / 4, BATCH = 16;   // columns per wave, values in flight
+    bool finite = true;
+    const float lo = MAGIC + lower, hi = MAGIC + upper;
+    const u32 mask4 = mask * 0x01010101u;
+    const float *group = FIXED ? scale : scale + (i64(row) / gr) * ncg;
+    for (i64 kc = i64(blockIdx.y) * CONV_CHUNK; kc < kp; kc += i64(gridDim.y) * CONV_CHUNK) {
+        if (!one_table) rows64.fill(g, u32(r0), row, live, int(kc % rows64.kk));
+        __syncthreads();   // the table; the previous tile is written
+        const i64 k0 = kc + wave * CPW;
+        ConvWalk<Off> walk(rows64, K, kc, k0);
+        float column_scale = 1.0f, column_r = 1.0f;   // FIXED: of column k0 + lane
+        if (FIXED && lane < CPW && k0 + lane < K) {
+            column_scale = scale[k0 + lane];
+            column_r = 1.0f / column_scale;
+        }
+        i64 cg = FIXED ? 0 : k0 / gc, cr = FIXED ? 0 : k0 - cg * gc;
+        float s_now = 1.0f, r_now = 1.0f;
+#pragma unroll 1
+        for (int t0 = 0; t0 < CPW; t0 += BATCH) {
+            u32 *words = tile + lane * CONV_PITCH + (wave * CPW + t0) / 4;
+            if (k0 + t0 >= K) {
+#pragma unroll
+                for (int e = 0; e < BATCH / 4; ++e) words[e] = 0u;
+                continue;
+            }
+            float v[BATCH], s[BATCH];
+            u32 fresh = t0 == 0;   // bit t: column t begins a group of scales
+            walk.values(v);
+#pragma unroll
+            for (int t = 0; t < BATCH; ++t) {
+                if constexpr (!FIXED) {
+                    if (cr == gc) {
+                        cr = 0;
+                        ++cg;
+                        fresh |= 1u << t;
+                    }
+                    if (fresh >> t & 1u) s_now = k0 + t0 + t < K ? group[cg] : 1.0f;
+                    s[t] = s_now;
+                    ++cr;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < BATCH / 4; ++e) {
+                u32 y[4];
+                bool near = false;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const int t = e * 4 + b;
+                    float r;
+                    if constexpr (FIXED) {
+                        r = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(column_r), t0 + t));
+                    } else {
+                        if (fresh >> t & 1u) r_now = 1.0f / s[t];
+                        r = r_now;
+                    }
+                    const float code = fmaf(v[t], r, MAGIC);
+                    const float off = fmaf(v[t], r, -(code - MAGIC));
+                    near = near || !(fabsf(off) <= CLEAR);
+                    y[b] = __float_as_uint(__builtin_amdgcn_fmed3f(code, lo, hi));
+                }
+                u32 word = (__builtin_amdgcn_perm(y[1], y[0], 0x0C0C0400u) |
+                            __builtin_amdgcn_perm(y[3], y[2], 0x04000C0Cu)) & mask4;
+                if (__ballot(near)) {
+                    word = 0u;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const int t = e * 4 + b;
+                        const float sc = FIXED ? __uint_as_float(__builtin_amdgcn_readlane(
+                                                     __float_as_uint(column_scale), t0 + t))
+                                               : s[t];
+                        finite = finite && fabsf(v[t]) <= FLT_MAX;
+                        word |= u32(quantize_code(v[t], sc, lower, upper, mask)) << (8 * b);
+                    }
+                }
+                words[e] = word;
+            }
+        }
+        __syncthreads();
+        // Row trow of the tile: 4 threads x CONV_CHUNK/4 bytes.
+        const int trow = threadIdx.x >> 2, part = threadIdx.x & 3;
+        constexpr int WORDS = CONV_CHUNK / 16;
+        const i64 col = kc + part * (CONV_CHUNK / 4);
+        if (r0 + trow >= rows || col >= kp) continue;
+        u32 w[WORDS];
+#pragma unroll
+        for (int e = 0; e < WORDS; ++e) w[e] = tile[trow * CONV_PITCH + part * WORDS + e];
+        u8 *dst = q + (r0 + trow) * kp + col;
+        if (vec) {   // kp and q 16-byte aligned: whole 16-byte pieces below kp
+#pragma unroll
+            for (int e = 0; e < WORDS; e += 4)
+                if (col + 4 * e < kp)
+                    *reinterpret_cast<uint4 *>(dst + 4 * e) =
+                        make_uint4(w[e], w[e + 1], w[e + 2], w[e + 3]);
+        } else {
+            const int count = int(kp - col < CONV_CHUNK / 4 ? kp - col : CONV_CHUNK / 4);
+            for (int t = 0; t < count; ++t) dst[t] = u8(w[t >> 2] >> (8 * (t & 3)));
+        }
+    }
+    if (!finite && status) atomicOr(status, flag);
+}
+
+// Group maxima |x| of the patch matrix for groups of gr rows and gc columns into work
+// [ceil(rows/gr), ncg] (cleared; float bits: a NaN is above every number).  The tiles of
+// k_conv_codes; a wave flushes its lanes' running maxima at column-group boundaries and at the end
+// of its columns, as one where its rows share a group.  8192 patches of 288 columns: below 12 us;
+// 65 when a wave walked all columns, one load at a time.
+template <typename Off>
+__global__ __launch_bounds__(256) void k_conv_group_max(const float *x, const mf_conv_geometry g,
+                                                        i64 K, i64 gr, i64 gc, i64 ncg, u32 *work,
+                                                        u32 *status, u32 flag) {
+    extern __shared__ u64 conv_table[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const i64 rows = g.n * g.out_height * g.out_width;
     const i64 r0 = i64(blockIdx.x) * 64;
     const i64 kc = i64(blockIdx.y) * CONV_CHUNK;
     const bool live = r0 + lane < rows;
-    const ConvLane me = conv_lane(g, u32(live ? r0 + lane : r0));
-    const int k0 = int(kc) + wave * (CONV_CHUNK / 4);
-    bool finite = true;
-    constexpr int CPW = CONV_CHUNK / 4;   // columns per wave
-    if (k0 < K) {
-        // Gather every value (and scale) first, so the loads are all in flight
-        // before the first one is needed.
-        float v[CPW], sc[CPW];
-        ConvTap tap;
-        tap.start(g, k0);
-        const i64 rg = gc ? ((live ? r0 + lane : r0) / gr) * ncg : 0;
-        i64 cg = gc ? k0 / gc : 0, cr = gc ? k0 - cg * gc : 0;
-#pragma unroll
-        for (int t = 0; t < CPW; ++t) {
-            v[t] = 0.0f;
-            sc[t] = 1.0f;
-            if (k0 + t < K) {
-                v[t] = conv_load(x, g, me, live, tap);
-                sc[t] = gc ? scale[rg + cg] : scale[k0 + t];
-                tap.next(g);
-                if (gc && ++cr == gc) {
-                    cr = 0;
-                    ++cg;
-                }
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < CPW / 4; ++e) {
-            u32 word = 0;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int t = e * 4 + b;
-                if (k0 + t < K) {
-                    finite = finite && fabsf(v[t]) <= FLT_MAX;
-                    word |= u32(quantize_code(v[t], sc[t], lower, upper, mask)) << (8 * b);
-                }
-            }
-            tile[lane * CONV_PITCH + wave * (CPW / 4) + e] = word;
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < CPW / 4; ++e) tile[lane * CONV_PITCH + wave * (CPW / 4) + e] = 0;
-    }
-    if (!finite && status) atomicOr(status, flag);
+    const u32 row = u32(live ? r0 + lane : r0);
+    ConvTile<Off> rows64(x, g, u32(r0), reinterpret_cast<Off *>(conv_table));
+    rows64.fill(g, u32(r0), row, live,
+                rows64.kk <= rows64.taps ? 0 : int(kc % rows64.kk));
     __syncthreads();
-    // Row `row` of the tile: 4 threads x CONV_CHUNK/4 bytes.
-    const int row = threadIdx.x >> 2, part = threadIdx.x & 3;
-    constexpr int WORDS = CONV_CHUNK / 16;
-    if (r0 + row >= rows) return;
-    const i64 col = kc + part * (CONV_CHUNK / 4);
-    if (col >= kp) return;
-    u32 w[WORDS];
+    constexpr int CPW = CONV_CHUNK / 4, BATCH = 16;
+    const i64 k0 = kc + wave * CPW;
+    if (k0 >= K) return;
+    const i64 last = r0 + 63 < rows ? r0 + 63 : rows - 1;
+    const bool shared = r0 / gr == last / gr;   // one row group for all lanes
+    ConvWalk<Off> walk(rows64, K, kc, k0);
+    i64 cg = k0 / gc, cr = k0 - cg * gc;
+    u32 *target = work + (i64(row) / gr) * ncg + cg;
+    u32 peak = 0u, top = 0u;
+#pragma unroll 1
+    for (int t0 = 0; t0 < CPW && k0 + t0 < K; t0 += BATCH) {
+        float v[BATCH];
+        walk.values(v);
 #pragma unroll
-    for (int e = 0; e < WORDS; ++e) w[e] = tile[row * CONV_PITCH + part * WORDS + e];
-    u8 *dst = q + (r0 + row) * kp + col;
-    if (vec) {   // kp and q 16-byte aligned: whole 16-byte pieces below kp
-#pragma unroll
-        for (int e = 0; e < WORDS; e += 4)
-            if (col + 4 * e < kp)
-                *reinterpret_cast<uint4 *>(dst + 4 * e) =
-                    make_uint4(w[e], w[e + 1], w[e + 2], w[e + 3]);
-    } else {
-        const int count = int(kp - col < CONV_CHUNK / 4 ? kp - col : CONV_CHUNK / 4);
-        for (int t = 0; t < count; ++t) dst[t] = u8(w[t >> 2] >> (8 * (t & 3)));
+        for (int t = 0; t < BATCH; ++t) {
+            const u32 bits = __float_as_uint(fabsf(v[t]));
+            peak = peak > bits ? peak : bits;
+            if (++cr == gc || t0 + t + 1 == CPW || k0 + t0 + t + 1 == K) {
+                top = top > peak ? top : peak;
+                if (shared)
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const u32 other = __shfl_xor(peak, o, 64);
+                        peak = peak > other ? peak : other;
+                    }
+                if (peak && (shared ? lane == 0 : live)) atomicMax(target, peak);
+                if (k0 + t0 + t + 1 >= K) break;   // past the patch: nothing to add
+                if (cr == gc) {
+                    ++target;
+                    cr = 0;
+                }
+                peak = 0u;
+            }
+        }
     }
+    if (top > 0x7F7FFFFFu && status) atomicOr(status, flag);
 }
 
-// Group maxima |x| of the patch matrix for groups of gr rows and gc columns into
-// work [ceil(rows/gr), ncg] (cleared; float bits).  A wave owns 64 rows and walks all
-// K columns, flushing each lane's running maximum at column-group boundaries.
-__global__ __launch_bounds__(256) void k_conv_group_max(const float *x, const mf_conv_geometry g,
-                                                        i64 K, i64 gr, i64 gc, i64 ncg, u32 *work,
-                                                        u32 *status, u32 flag) {
-    const int lane = threadIdx.x & 63;
-    const i64 rows = g.n * g.out_height * g.out_width;
-    const i64 r0 = (i64(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 64;
-    if (r0 >= rows) return;
-    const bool live = r0 + lane < rows;
-    const ConvLane me = conv_lane(g, u32(live ? r0 + lane : r0));
-    u32 *target = work + ((live ? r0 + lane : r0) / gr) * ncg;
-    ConvTap tap;
-    tap.start(g, 0);
-    bool finite = true;
-    float peak = 0.0f;
-    i64 cr = 0;
-#pragma unroll 1
-    for (i64 k = 0; k < K; ++k) {
-        const float v = fabsf(conv_load(x, g, me, live, tap));
-        finite = finite && v <= FLT_MAX;
-        peak = v > peak || v != v ? v : peak;
-        tap.next(g);
-        if (++cr == gc || k + 1 == K) {
-            if (live && __float_as_uint(peak)) atomicMax(target, __float_as_uint(peak));
-            ++target;
-            cr = 0;
-            peak = 0.0f;
-        }
-    }
-    if (!finite && status) atomicOr(status, flag);
-}
+#define MF_CONV_INST(Off)                                                                         \
+    template __global__ void k_conv_codes<Off, false>(const float *, const mf_conv_geometry, i64, \
+                                                      i64, const float *, i64, i64, i64, float,   \
+                                                      float, u32, u8 *, int, u32 *, u32);         \
+    template __global__ void k_conv_codes<Off, true>(const float *, const mf_conv_geometry, i64,  \
+                                                     i64, const float *, i64, i64, i64, float,    \
+                                                     float, u32, u8 *, int, u32 *, u32);          \
+    template __global__ void k_conv_group_max<Off>(const float *, const mf_conv_geometry, i64,    \
+                                                   i64, i64, i64, u32 *, u32 *, u32);
+MF_CONV_INST(u32)
+MF_CONV_INST(u64)
+#undef MF_CONV_INST
 
 // xscale [n, m*Gr]: scale of the read's first physical row, replicate-padded.
 __global__ void k_input_scales(i64 n, i64 k, i64 groups, int R, int P, int Gr,
