@@ -301,6 +301,19 @@ int mf_narrow_output(const double *in, int64_t n, int64_t cols, int64_t ld, floa
 int mf_bias_add(float *out, int64_t n, int64_t o, int64_t ldo, const float *bias,
                 uint32_t *status, void *stream);
 
+/* Dequantized operands of a narrow configuration (memfast/nn/training.py:62-72), one FP32
+ * product code * scale each: out [n, k] of the codes q [n, m, R] and read scales xscale
+ * [n, m*Gr], and out [k, o] of the codes packed [m, p, R, C] (two's complement unless
+ * !weight_signed) and read scales wscale [m*Gr, p*C]. */
+int mf_dequantize_inputs(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n,
+                         int64_t k, float *out, void *stream);
+int mf_dequantize_program(const mf_config *cfg, const uint8_t *packed, const float *wscale,
+                          int64_t k, int64_t o, int32_t weight_signed, float *out, void *stream);
+
+/* Sets `flag` in status when one of the count values of x is not finite. */
+int mf_flag_nonfinite(const float *x, int64_t count, uint32_t flag, uint32_t *status,
+                      void *stream);
+
 /* Geometry of one convolution group for mf_conv_input_tiles: NCHW input
  * [n, channels, height, width], this group's channels [c0, c0 + group_channels),
  * output [out_height, out_width] and the kernel's size, stride, zero padding

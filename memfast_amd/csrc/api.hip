@@ -2096,6 +2096,43 @@ int mf_mm_totals(const mf_config *cfg, const uint8_t *q, int64_t n, int64_t m,
                         static_cast<hipStream_t>(stream));
 }
 
+int mf_dequantize_inputs(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n,
+                         int64_t k, float *out, void *stream) {
+    const int status = check_narrow(cfg);
+    if (status) return status;
+    if (!q || !xscale || !out || n < 1 || k < 1 || k > 0x7FFFFFFF)
+        return fail(MF_E_INVALID, "invalid dequantize arguments");
+    const i64 m = (k + cfg->rows - 1) / cfg->rows;
+    const dim3 grid(unsigned((k + 255) / 256), unsigned(std::min<i64>(n, 4096)));
+    hipLaunchKernelGGL(k_dequantize_inputs, grid, dim3(256), 0, static_cast<hipStream_t>(stream), q,
+                       xscale, n, k, cfg->rows, cfg->read_rows, cfg->reads, m,
+                       1u << (cfg->activation_bits - 1), out);
+    return check_launch("dequantize inputs");
+}
+
+int mf_dequantize_program(const mf_config *cfg, const uint8_t *packed, const float *wscale,
+                          int64_t k, int64_t o, int32_t weight_signed, float *out, void *stream) {
+    const int status = check_narrow(cfg);
+    if (status) return status;
+    if (!packed || !wscale || !out || k < 1 || o < 1 || k > 0x7FFFFFFF || o > 0x7FFFFFFF)
+        return fail(MF_E_INVALID, "invalid dequantize arguments");
+    const i64 p = (o + cfg->cols - 1) / cfg->cols;
+    const dim3 grid(unsigned((o + 255) / 256), unsigned(std::min<i64>(k, 4096)));
+    hipLaunchKernelGGL(k_dequantize_program, grid, dim3(256), 0, static_cast<hipStream_t>(stream),
+                       packed, wscale, k, o, cfg->rows, cfg->cols, cfg->read_rows, cfg->reads, p,
+                       (1u << cfg->weight_bits) - 1u,
+                       weight_signed ? 1u << (cfg->weight_bits - 1) : 0u, out);
+    return check_launch("dequantize program");
+}
+
+int mf_flag_nonfinite(const float *x, int64_t count, uint32_t flag, uint32_t *status,
+                      void *stream) {
+    if (!x || !status || count < 1) return fail(MF_E_INVALID, "invalid finiteness arguments");
+    hipLaunchKernelGGL(k_flag_nonfinite, dim3(unsigned(std::min<i64>((count + 255) / 256, 1024))),
+                       dim3(256), 0, static_cast<hipStream_t>(stream), x, count, flag, status);
+    return check_launch("finiteness check");
+}
+
 int mf_bias_add(float *out, int64_t n, int64_t o, int64_t ldo, const float *bias,
                 uint32_t *status, void *stream) {
     if (!out || !bias || n < 1 || o < 1 || ldo < o) return fail(MF_E_INVALID, "invalid bias arguments");

@@ -12,6 +12,47 @@
 
 namespace mf {
 
+// Dequantized operands of the training surrogate: code * scale of the row's read, FP32.  Rows in
+// grid y, columns in grid x.  784 x 512 weights: 4.1 us in one launch (2 MB, launch-bound); index
+// tables, integer widening, sign extension, gathers and the product took more than ten.
+__device__ __forceinline__ float signed_code(u32 code, u32 mask, u32 sign) {
+    return float(int((code & mask) ^ sign) - int(sign));
+}
+
+__global__ void k_dequantize_inputs(const u8 *q, const float *xscale, i64 n, i64 k, int R, int P,
+                                    int Gr, i64 m, u32 sign, float *out) {
+    const u32 mask = 2u * sign - 1u;
+    for (i64 c = i64(blockIdx.x) * blockDim.x + threadIdx.x; c < k; c += i64(gridDim.x) * blockDim.x) {
+        const u32 array = u32(c) / u32(R), r = u32(c) - array * u32(R);
+        const i64 read = i64(array) * Gr + r / u32(P);
+        for (i64 row = blockIdx.y; row < n; row += gridDim.y)
+            out[row * k + c] =
+                signed_code(q[row * m * R + c], mask, sign) * xscale[row * m * Gr + read];
+    }
+}
+
+__global__ void k_dequantize_program(const u8 *packed, const float *wscale, i64 k, i64 o, int R,
+                                     int C, int P, int Gr, i64 p, u32 mask, u32 sign, float *out) {
+    for (i64 c = i64(blockIdx.x) * blockDim.x + threadIdx.x; c < o; c += i64(gridDim.x) * blockDim.x) {
+        const u32 t = u32(c) / u32(C), cc = u32(c) - t * u32(C);
+        for (i64 row = blockIdx.y; row < k; row += gridDim.y) {
+            const u32 array = u32(row) / u32(R), r = u32(row) - array * u32(R);
+            const i64 read = i64(array) * Gr + r / u32(P);
+            const u32 code = packed[((array * p + t) * R + r) * C + cc];
+            out[row * o + c] = signed_code(code, mask, sign) * wscale[read * p * C + c];
+        }
+    }
+}
+
+// The finiteness check of a small operand beside others that set the same status word.
+__global__ void k_flag_nonfinite(const float *x, i64 count, u32 flag, u32 *status) {
+    bool finite = true;
+    for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < count;
+         i += i64(gridDim.x) * blockDim.x)
+        finite = finite && fabsf(x[i]) <= FLT_MAX;
+    if (!finite) atomicOr(status, flag);
+}
+
 // out[v, c] += bias[c] (one FP32 add, as torch's broadcast add), flagging a
 // non-finite sum in the status word.
 __global__ void k_bias_add(float *out, i64 n, i64 o, i64 ldo, const float *bias, u32 *status,

@@ -156,6 +156,9 @@ SIGNATURES = {
                       ct.c_uint64, _P, _I64, _I32, _P, _P], ct.c_int),
     "mf_mm_totals": ([_CFG, _P, _I64, _I64, _P, _I64, _P, ct.c_uint32, ct.c_uint64, _P, _P, _I64,
                       _P], ct.c_int),
+    "mf_dequantize_inputs": ([_P, _P, _P, _I64, _I64, _P, _P], ct.c_int),
+    "mf_dequantize_program": ([_P, _P, _P, _I64, _I64, ct.c_int32, _P, _P], ct.c_int),
+    "mf_flag_nonfinite": ([_P, _I64, ct.c_uint32, _P, _P], ct.c_int),
     "mf_bias_add": ([_P, _I64, _I64, _I64, _P, _P, _P], ct.c_int),
     "mf_gru_gates": ([_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P], ct.c_int),
     "mf_gru_sequence": ([_CFG, _I64, _I32, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64, _P,
@@ -945,6 +948,55 @@ def _workspace(config, n, m, p, device, variant=0):
     """Device scratch for the MFMA reads (mf_mm_workspace bytes, 256-byte aligned)."""
     return torch.empty(max(1, mm_workspace_bytes(config, n, m, p, variant)), dtype=torch.uint8,
                        device=device)
+
+
+def dequantize_inputs(q, xscale, config, k):
+    """quantization.dequantize_inputs of a narrow configuration's input tiles, in one kernel."""
+    require_device(q)
+    n, m, rows = q.shape
+    if (config.wide or q.dtype != torch.uint8 or xscale.dtype != torch.float32
+            or not (q.is_contiguous() and xscale.is_contiguous())
+            or rows != config.array_size[0] or m != math.ceil(k / rows)
+            or xscale.shape != (n, m * config.reads_per_array)):
+        raise ValueError("dequantize_inputs takes the input tiles of a narrow configuration")
+    out = torch.empty((n, k), dtype=torch.float32, device=q.device)
+    if n:
+        with _on(q.device):
+            check(library().mf_dequantize_inputs(
+                ct.byref(descriptor(config)), _ptr(q), _ptr(xscale), n, k, _ptr(out),
+                _stream(q.device)), "dequantize inputs")
+    return out
+
+
+def dequantize_program(packed, weight_scale, config, k, o):
+    """quantization.dequantize_program of a narrow configuration's program, in one kernel."""
+    require_device(packed)
+    r, c = config.array_size
+    m, p = math.ceil(k / r), math.ceil(o / c)
+    if (config.wide or packed.dtype != torch.uint8 or weight_scale.dtype != torch.float32
+            or not (packed.is_contiguous() and weight_scale.is_contiguous())
+            or packed.shape != (m, p, r, c)
+            or weight_scale.numel() != m * config.reads_per_array * p * c
+            or weight_scale.device != packed.device):
+        raise ValueError("dequantize_program takes the program of a narrow configuration")
+    out = torch.empty((k, o), dtype=torch.float32, device=packed.device)
+    with _on(packed.device):
+        check(library().mf_dequantize_program(
+            ct.byref(descriptor(config)), _ptr(packed), _ptr(weight_scale), k, o,
+            int(bool(config.weight_signed)), _ptr(out), _stream(packed.device)),
+            "dequantize program")
+    return out
+
+
+def flag_nonfinite(tensor, status, flag):
+    """Sets ``flag`` in ``status`` when a contiguous FP32 ``tensor`` is not finite."""
+    require_device(tensor)
+    if tensor.dtype != torch.float32 or not tensor.is_contiguous():
+        raise ValueError("flag_nonfinite takes a contiguous FP32 tensor")
+    if tensor.numel():
+        with _on(tensor.device):
+            check(library().mf_flag_nonfinite(_ptr(tensor), tensor.numel(), flag, _ptr(status),
+                                              _stream(tensor.device)), "finiteness check")
 
 
 def bias_add(out, bias, status=None):

@@ -63,14 +63,26 @@ def _dequantized_inputs(flat, config):
     quantizer's codes and read scales."""
     if flat.numel() == 0:
         return flat.float()
-    q, xscale = hip.input_tiles(flat.detach(), config)
-    return dequantize_inputs(q, xscale, config, flat.shape[1])
+    if config.wide:
+        q, xscale = hip.input_tiles(flat.detach(), config)
+        return dequantize_inputs(q, xscale, config, flat.shape[1])
+    # The finiteness check is the quantizer's, read once the values are queued.
+    status = hip.status_word(flat.device)
+    q, xscale = hip.input_tiles(flat.detach(), config, status=status)
+    values = hip.dequantize_inputs(q, xscale, config, flat.shape[1])
+    if int(status.item()) & hip.STATUS_INPUT:
+        raise ValueError(hip.input_error(config))
+    return values
 
 
 @torch.no_grad()
 def _dequantized_weights(matrix):
     """FP32 physical [K, O] weights of ``matrix``'s current program."""
-    return dequantize_program(matrix.packed, matrix.weight_scale, matrix.config,
+    native = (not matrix.config.wide and matrix.packed.dtype == torch.uint8
+              and matrix.packed.is_contiguous() and matrix.weight_scale.dtype == torch.float32
+              and matrix.weight_scale.is_contiguous())
+    dequantize = hip.dequantize_program if native else dequantize_program
+    return dequantize(matrix.packed, matrix.weight_scale, matrix.config,
                               matrix.in_features, matrix.out_features)
 
 

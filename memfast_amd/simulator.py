@@ -571,6 +571,8 @@ class AnalogMatrix(nn.Module):
         """A new program of floating [O,K] weights (and bias) for ``_commit``, with the
         checks of programming a fresh matrix (memfast/nn/training.py:40-47); nothing of
         this matrix changes."""
+        if self._checked_by_kernels(weight, bias):
+            return self._prepare_checked(weight, bias)
         if not bool(torch.isfinite(weight).all()):
             raise ValueError("weights must be finite")
         if not weight.is_floating_point():
@@ -580,6 +582,33 @@ class AnalogMatrix(nn.Module):
         dtype = torch.float64 if self.config.wide else torch.float32
         return packed, column_codes, table, _bias_buffer(bias, self.out_features,
                                                          self.packed.device, dtype)
+
+    def _checked_by_kernels(self, weight, bias):
+        """Whether the checks of ``_prepare`` are those of the quantizer and a kernel over the
+        bias buffer: operands that FP32 holds exactly and biases of the matrix's shape."""
+        exact = (torch.float32, torch.bfloat16, torch.float16)
+        return (not self.config.wide and weight.dtype in exact and weight.numel() > 0
+                and weight.device == self.packed.device
+                and (bias is None or (bias.dtype in exact and bias.device == weight.device
+                                      and tuple(bias.shape) == (self.out_features,))))
+
+    def _prepare_checked(self, weight, bias):
+        """``_prepare`` with one status read: what each operand's own scans would raise, in
+        their order."""
+        status = hip.status_word(weight.device)
+        packed, column_codes, table = hip.weight_tiles(weight.detach(), self.config, status=status)
+        stored = None
+        if bias is not None:
+            stored = bias.detach().to(torch.float32, copy=True).contiguous()
+            hip.flag_nonfinite(stored, status, hip.STATUS_INPUT)   # no input has this word
+        flags = int(status.item())
+        if flags & hip.STATUS_WEIGHT:
+            raise ValueError("weights must be finite")
+        if flags & hip.STATUS_NEGATIVE_WEIGHT:
+            raise ValueError(hip.UNSIGNED_MESSAGE)
+        if flags & hip.STATUS_INPUT:
+            raise ValueError("bias must be finite and match out_features")
+        return packed, column_codes, table, stored
 
     @torch.no_grad()
     def _commit(self, prepared):
