@@ -2096,6 +2096,23 @@ int mf_mm_totals(const mf_config *cfg, const uint8_t *q, int64_t n, int64_t m,
                         static_cast<hipStream_t>(stream));
 }
 
+int mf_unfold_rows(const float *x, const mf_conv_geometry *geom, float *out, void *stream) {
+    if (!x || !geom || !out) return fail(MF_E_INVALID, "invalid unfold arguments");
+    const mf_conv_geometry g = *geom;
+    const int status = check_conv_geometry(g);
+    if (status) return status;
+    const i64 rows = g.n * g.out_height * g.out_width, K = g.group_channels * g.kh * g.kw;
+    if (rows > 0x7FFFFFFF || K > 0x7FFFFFFF)
+        return fail(MF_E_UNSUPPORTED, "too many patches or patch columns");
+    // Up to 8192 workgroups (four per wave slot of the chip); a wave then takes several rows.
+    const i64 columns = (K + 63) / 64, blocks = (rows + 3) / 4;
+    const i64 most = std::max<i64>(1, 8192 / columns);
+    const dim3 grid(unsigned(columns), unsigned(std::min<i64>(std::min(blocks, most), 65535)));
+    hipLaunchKernelGGL(k_unfold_rows, grid, dim3(256), 0, static_cast<hipStream_t>(stream), x, g,
+                       rows, u32(K), out);
+    return check_launch("unfold");
+}
+
 int mf_dequantize_inputs(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n,
                          int64_t k, float *out, void *stream) {
     const int status = check_narrow(cfg);

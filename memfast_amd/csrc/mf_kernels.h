@@ -319,6 +319,8 @@ __global__ void k_fill_u32(u32 *p, i64 count, u32 value);
 __global__ void k_gru_gates(const float *inputs, i64 ldi, const float *hidden, i64 ldh,
                             const float *hx, i64 ldx, float *out, i64 ldo, i64 n, i64 width,
                             const float *bias, u32 *status, u32 flag);
+__global__ void k_unfold_rows(const float *x, const mf_conv_geometry g, i64 rows, u32 K,
+                              float *out);
 __global__ void k_dequantize_inputs(const u8 *q, const float *xscale, i64 n, i64 k, int R, int P,
                                     int Gr, i64 m, u32 sign, float *out);
 __global__ void k_dequantize_program(const u8 *packed, const float *wscale, i64 k, i64 o, int R,

@@ -156,6 +156,7 @@ SIGNATURES = {
                       ct.c_uint64, _P, _I64, _I32, _P, _P], ct.c_int),
     "mf_mm_totals": ([_CFG, _P, _I64, _I64, _P, _I64, _P, ct.c_uint32, ct.c_uint64, _P, _P, _I64,
                       _P], ct.c_int),
+    "mf_unfold_rows": ([_P, ct.POINTER(MFConvGeometry), _P, _P], ct.c_int),
     "mf_dequantize_inputs": ([_P, _P, _P, _I64, _I64, _P, _P], ct.c_int),
     "mf_dequantize_program": ([_P, _P, _P, _I64, _I64, ct.c_int32, _P, _P], ct.c_int),
     "mf_flag_nonfinite": ([_P, _I64, ct.c_uint32, _P, _P], ct.c_int),
@@ -951,6 +952,28 @@ def _workspace(config, n, m, p, device, variant=0):
 
 
 def dequantize_inputs(q, xscale, config, k):
+def unfold_rows(x, kernel, dilation, padding, stride):
+    """F.unfold(x, ...).transpose(1, 2) of FP32 NCHW ``x`` as a contiguous [N, L, K], in one
+    kernel (no autograd)."""
+    require_device(x)
+    if x.dtype != torch.float32 or x.ndim != 4 or not x.numel():
+        raise ValueError("unfold_rows takes an FP32 NCHW image")
+    value = x.contiguous()
+    n, channels, height, width = value.shape
+    out_size = [(size + 2 * pad - dil * (k - 1) - 1) // step + 1 for size, pad, dil, k, step in
+                zip((height, width), padding, dilation, kernel, stride)]
+    if min(out_size) < 1:
+        raise ValueError("unfold_rows needs a non-empty output")
+    out = torch.empty((n, out_size[0] * out_size[1], channels * kernel[0] * kernel[1]),
+                      dtype=torch.float32, device=x.device)
+    geom = MFConvGeometry(n, channels, height, width, 0, channels, *out_size, *kernel, *stride,
+                          *padding, *dilation)
+    with _on(x.device):
+        check(library().mf_unfold_rows(_ptr(value), ct.byref(geom), _ptr(out), _stream(x.device)),
+              "unfold")
+    return out
+
+
     """quantization.dequantize_inputs of a narrow configuration's input tiles, in one kernel."""
     require_device(q)
     n, m, rows = q.shape

@@ -27,7 +27,7 @@ from torch.nn import functional as F
 
 from .. import hip
 from ..quantization import dequantize_inputs, dequantize_program
-from .convolution import AnalogConv2d
+from .convolution import AnalogConv2d, _output_size
 
 GRADIENT_MODES = ("quantized", "digital")
 
@@ -50,6 +50,20 @@ class _SurrogateGradient(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         return None, grad_output.to(ctx.surrogate_dtype)
+
+
+class _PatchRows(torch.autograd.Function):
+    """``F.unfold(x, ...).transpose(1, 2)`` of an FP32 image, laid out [N, L, K]; backward is
+    F.unfold's own (F.fold)."""
+
+    @staticmethod
+    def forward(ctx, x, kernel, dilation, padding, stride):
+        ctx.size, ctx.geometry = x.shape[-2:], (kernel, dilation, padding, stride)
+        return hip.unfold_rows(x, kernel, dilation, padding, stride)
+
+    @staticmethod
+    def backward(ctx, grad_rows):
+        return F.fold(grad_rows.transpose(1, 2), ctx.size, *ctx.geometry), None, None, None, None
 
 
 def _through(value, replacement):
@@ -198,17 +212,17 @@ class TrainableAnalogConv2d(_HardwareAware):
 
     def _quantized_surrogate(self, x):
         source, padding = self._padded(x)
-        patches = F.unfold(source, self.kernel_size, self.dilation, padding, self.stride)
+        spatial = _output_size(x.shape[-2:], self.padding, self.dilation, self.kernel_size,
+                               self.stride)
+        geometry = (self.kernel_size, self.dilation, padding, self.stride)
+        if self.analog._gathers(source, spatial):   # the read took its patches the same way
+            rows = _PatchRows.apply(source, *geometry)
+        else:
+            rows = F.unfold(source, *geometry).transpose(1, 2)
         size = self.weight[0].numel()
-        pieces = [
-            _linear_surrogate(patches[:, g * size:(g + 1) * size].transpose(1, 2), weight, bias,
-                              matrix)
-            for g, (matrix, weight, bias) in enumerate(self._programs())
-        ]
+        pieces = [_linear_surrogate(rows[..., g * size:(g + 1) * size], weight, bias, matrix)
+                  for g, (matrix, weight, bias) in enumerate(self._programs())]
         merged = torch.cat(pieces, dim=-1).transpose(1, 2)
-        spatial = [(extent + 2 * pad - dil * (k - 1) - 1) // step + 1
-                   for extent, pad, dil, k, step in zip(x.shape[-2:], self.padding, self.dilation,
-                                                        self.kernel_size, self.stride)]
         return merged.reshape(x.shape[0], self.out_channels, *spatial)
 
     def _digital_surrogate(self, x):
