@@ -301,6 +301,11 @@ int mf_narrow_output(const double *in, int64_t n, int64_t cols, int64_t ld, floa
 int mf_bias_add(float *out, int64_t n, int64_t o, int64_t ldo, const float *bias,
                 uint32_t *status, void *stream);
 
+/* The same from `in` [n, o] (row stride ldi, e.g. a read's padded output) to `out` (row stride
+ * ldo); in == out takes one stride. */
+int mf_bias_output(const float *in, int64_t n, int64_t o, int64_t ldi, const float *bias, float *out,
+                   int64_t ldo, uint32_t *status, void *stream);
+
 /* Dequantized operands of a narrow configuration (memfast/nn/training.py:62-72), one FP32
  * product code * scale each: out [n, k] of the codes q [n, m, R] and read scales xscale
  * [n, m*Gr], and out [k, o] of the codes packed [m, p, R, C] (two's complement unless

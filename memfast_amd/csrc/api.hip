@@ -2150,13 +2150,32 @@ int mf_flag_nonfinite(const float *x, int64_t count, uint32_t flag, uint32_t *st
     return check_launch("finiteness check");
 }
 
+int mf_bias_output(const float *in, int64_t n, int64_t o, int64_t ldi, const float *bias, float *out,
+                   int64_t ldo, uint32_t *status, void *stream) {
+    if (!in || !out || !bias || n < 1 || o < 1 || ldi < o || ldo < o || (in == out && ldi != ldo))
+        return fail(MF_E_INVALID, "invalid bias arguments");
+    const bool vec = o % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 && aligned(in, 16) &&
+                     aligned(out, 16) && aligned(bias, 16);
+    const i64 units = vec ? o / 4 : o;
+    int lanes = 0;
+    while (lanes < 8 && (i64(1) << lanes) < units) ++lanes;
+    const i64 gy = std::min<i64>((units + 255) / 256, 65535);
+    const i64 per_block = 256 >> lanes;
+    const i64 gx = std::min<i64>((n + per_block - 1) / per_block, std::max<i64>(1, 8192 / gy));
+    const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (vec)
+        hipLaunchKernelGGL(k_bias_output<4>, grid, dim3(256), 0, s, in, n, o, ldi, bias, out, ldo,
+                           lanes, status, u32(MF_STATUS_OUTPUT));
+    else
+        hipLaunchKernelGGL(k_bias_output<1>, grid, dim3(256), 0, s, in, n, o, ldi, bias, out, ldo,
+                           lanes, status, u32(MF_STATUS_OUTPUT));
+    return check_launch("bias add");
+}
+
 int mf_bias_add(float *out, int64_t n, int64_t o, int64_t ldo, const float *bias,
                 uint32_t *status, void *stream) {
-    if (!out || !bias || n < 1 || o < 1 || ldo < o) return fail(MF_E_INVALID, "invalid bias arguments");
-    hipLaunchKernelGGL(k_bias_add, dim3(grid_for(n * o)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), out, n, o, ldo, bias, status,
-                       u32(MF_STATUS_OUTPUT));
-    return check_launch("bias add");
+    return mf_bias_output(out, n, o, ldo, bias, out, ldo, status, stream);
 }
 
 int mf_narrow_output(const double *in, int64_t n, int64_t cols, int64_t ld, float *out,

@@ -326,8 +326,9 @@ __global__ void k_dequantize_inputs(const u8 *q, const float *xscale, i64 n, i64
 __global__ void k_dequantize_program(const u8 *packed, const float *wscale, i64 k, i64 o, int R,
                                      int C, int P, int Gr, i64 p, u32 mask, u32 sign, float *out);
 __global__ void k_flag_nonfinite(const float *x, i64 count, u32 flag, u32 *status);
-__global__ void k_bias_add(float *out, i64 n, i64 o, i64 ldo, const float *bias, u32 *status,
-                           u32 flag);
+template <int V>
+__global__ void k_bias_output(const float *in, i64 n, i64 o, i64 ldi, const float *bias, float *out,
+                              i64 ldo, int lanes, u32 *status, u32 flag);
 __global__ void k_narrow_f64(const double *in, i64 n, i64 cols, i64 ld, float *out, u32 *status,
                              u32 flag);
 

@@ -79,20 +79,35 @@ __global__ void k_flag_nonfinite(const float *x, i64 count, u32 flag, u32 *statu
     if (!finite) atomicOr(status, flag);
 }
 
-// out[v, c] += bias[c] (one FP32 add, as torch's broadcast add), flagging a
-// non-finite sum in the status word.
-__global__ void k_bias_add(float *out, i64 n, i64 o, i64 ldo, const float *bias, u32 *status,
-                           u32 flag) {
+// out[v, c] = in[v, c] + bias[c] (one FP32 add, as torch's broadcast add; in place where
+// out == in), flagging a non-finite sum in the status word.  V columns per lane (4: 16-byte
+// accesses), 2^lanes lanes per row, which keep their bias over the block's rows; no division.
+// HBM-bound: 200704 x 64 outputs of 256-column arrays (103 MB) 18.6 us, 5.5 TB/s; a copy (18.4 us)
+// and an add in place with a 64-bit division per element (28.7 us) before.
+template <int V>
+__global__ __launch_bounds__(256) void k_bias_output(const float *in, i64 n, i64 o, i64 ldi,
+                                                     const float *bias, float *out, i64 ldo,
+                                                     int lanes, u32 *status, u32 flag) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const i64 per_block = 256 >> lanes, lane = threadIdx.x & ((1 << lanes) - 1);
+    const i64 first = i64(blockIdx.x) * per_block + (threadIdx.x >> lanes);
     bool finite = true;
-    for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < n * o;
-         i += i64(gridDim.x) * blockDim.x) {
-        const i64 v = i / o, c = i - v * o;
-        const float s = out[v * ldo + c] + bias[c];
-        out[v * ldo + c] = s;
-        finite = finite && fabsf(s) <= FLT_MAX;
+    for (i64 c = ((i64(blockIdx.y) << lanes) + lane) * V; c < o; c += (i64(gridDim.y) << lanes) * V) {
+        const vec b = *reinterpret_cast<const vec *>(bias + c);
+#pragma unroll 4
+        for (i64 v = first; v < n; v += gridDim.x * per_block) {
+            const vec s = *reinterpret_cast<const vec *>(in + v * ldi + c) + b;
+            *reinterpret_cast<vec *>(out + v * ldo + c) = s;
+#pragma unroll
+            for (int e = 0; e < V; ++e) finite = finite && fabsf(s[e]) <= FLT_MAX;
+        }
     }
     if (!finite && status) atomicOr(status, flag);
 }
+template __global__ void k_bias_output<1>(const float *, i64, i64, i64, const float *, float *, i64,
+                                          int, u32 *, u32);
+template __global__ void k_bias_output<4>(const float *, i64, i64, i64, const float *, float *, i64,
+                                          int, u32 *, u32);
 
 // out[v, c] = float(in[v * ld + c]) for c < cols (round to nearest even, as torch's cast
 // of an FP64 tensor to FP32), flagging a non-finite result in the status word.

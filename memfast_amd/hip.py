@@ -160,6 +160,7 @@ SIGNATURES = {
     "mf_dequantize_inputs": ([_P, _P, _P, _I64, _I64, _P, _P], ct.c_int),
     "mf_dequantize_program": ([_P, _P, _P, _I64, _I64, ct.c_int32, _P, _P], ct.c_int),
     "mf_flag_nonfinite": ([_P, _I64, ct.c_uint32, _P, _P], ct.c_int),
+    "mf_bias_output": ([_P, _I64, _I64, _I64, _P, _P, _I64, _P, _P], ct.c_int),
     "mf_bias_add": ([_P, _I64, _I64, _I64, _P, _P, _P], ct.c_int),
     "mf_gru_gates": ([_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P], ct.c_int),
     "mf_gru_sequence": ([_CFG, _I64, _I32, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64, _P,
@@ -951,7 +952,6 @@ def _workspace(config, n, m, p, device, variant=0):
                        device=device)
 
 
-def dequantize_inputs(q, xscale, config, k):
 def unfold_rows(x, kernel, dilation, padding, stride):
     """F.unfold(x, ...).transpose(1, 2) of FP32 NCHW ``x`` as a contiguous [N, L, K], in one
     kernel (no autograd)."""
@@ -974,6 +974,7 @@ def unfold_rows(x, kernel, dilation, padding, stride):
     return out
 
 
+def dequantize_inputs(q, xscale, config, k):
     """quantization.dequantize_inputs of a narrow configuration's input tiles, in one kernel."""
     require_device(q)
     n, m, rows = q.shape
@@ -1032,6 +1033,23 @@ def bias_add(out, bias, status=None):
     with _on(out.device):
         check(library().mf_bias_add(_ptr(out), out.shape[0], out.shape[1], out.stride(0),
                                     _ptr(bias), _ptr(status), _stream(out.device)), "bias add")
+    return out
+
+
+def bias_output(output, bias, status=None):
+    """A contiguous ``output + bias`` (as bias_add): in place, or where ``output`` is a column
+    block of a wider tensor into a new one."""
+    require_device(output)
+    if output.is_contiguous():
+        return bias_add(output, bias, status)
+    if output.dtype != torch.float32 or output.stride(1) != 1 or bias.shape != (output.shape[1],):
+        raise ValueError("bias_output takes an FP32 row-major output and a matching bias")
+    bias = bias.to(device=output.device, dtype=torch.float32).contiguous()
+    n, o = output.shape
+    out = torch.empty((n, o), dtype=torch.float32, device=output.device)
+    with _on(output.device):
+        check(library().mf_bias_output(_ptr(output), n, o, output.stride(0), _ptr(bias), _ptr(out),
+                                       o, _ptr(status), _stream(output.device)), "bias add")
     return out
 
 

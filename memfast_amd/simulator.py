@@ -759,18 +759,21 @@ class AnalogMatrix(nn.Module):
                             out_cols=self.out_features, k_rows=self.in_features)
             if source is not None:
                 self._terms_source = source
-        output = output[:, :self.out_features].contiguous()
-        if self.zero_correction is not None:
-            output = output + self._zero_point_term(q, xscale, stable).to(output.dtype)
-        # An FP32 read's bias goes through a kernel that also flags non-finite sums.
+        # An FP32 read's bias goes through a kernel that also flags non-finite sums and drops
+        # the array columns past the layer's.
         checked_bias = (self.bias is not None and self.zero_correction is None
                         and not config.wide and not stable)
+        output = output[:, :self.out_features]
+        if not checked_bias:
+            output = output.contiguous()
+        if self.zero_correction is not None:
+            output = output + self._zero_point_term(q, xscale, stable).to(output.dtype)
         if self.bias is not None and not checked_bias:
             output = output + self.bias
         if stable:
             return output, False
         if checked_bias:
-            hip.bias_add(output, self.bias, status)
+            output = hip.bias_output(output, self.bias, status)
         if defer:
             return output, True
         narrowed = narrow and config.wide
