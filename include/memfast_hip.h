@@ -343,15 +343,15 @@ int mf_conv_input_tiles(const mf_config *cfg, const float *x, const mf_conv_geom
                         const float *fixed_scale, int64_t gr, int64_t gc, uint32_t *work,
                         float *scale, uint8_t *q, float *xscale, uint32_t *status, void *stream);
 
+/* The patch matrix of mf_conv_input_tiles (group channels [c0, c0 + group_channels)) itself: out
+ * FP32 [n*L, K], the rows of F.unfold(x)'s transpose (memfast/nn/training.py:104-119). */
+int mf_unfold_rows(const float *x, const mf_conv_geometry *geom, float *out, void *stream);
+
 /* GRU gates over the two projections of one step (memfast/nn/recurrent.py
  * `AnalogGRUCell`, PyTorch's gate equations): with inputs and hidden [n, 3H]
  * (chunks r, z, n) and hx [n, H],
  *   out = (1 - z) * tanh(in + r * hn) + z * hx,  r|z = sigmoid(i + h),
  * every operation rounded to FP32 as PyTorch's separate elementwise ops are.
-/* The patch matrix of mf_conv_input_tiles (group channels [c0, c0 + group_channels)) itself: out
- * FP32 [n*L, K], the rows of F.unfold(x)'s transpose (memfast/nn/training.py:104-119). */
-int mf_unfold_rows(const float *x, const mf_conv_geometry *geom, float *out, void *stream);
-
  * Leading dimensions in elements. */
 int mf_gru_gates(const float *inputs, int64_t ldi, const float *hidden, int64_t ldh,
                  const float *hx, int64_t ldx, float *out, int64_t ldo, int64_t n, int64_t width,
