@@ -56,16 +56,26 @@ __device__ __forceinline__ v16i mfma(v4i a, v4i b, v16i c) {
 
 // Per-read digit sums, maximized over blocks of `block` (32 or 64) rows, then
 // tested against the slot thresholds: out[rb][g] = mask of proven slots.
-// Workgroup = 64 reads (one per lane, so a wave loads 64 consecutive P-byte
-// runs of a row) x 16 waves that split the block's rows; LDS combines the
+// Workgroup = LANES reads (one per lane, so a row's lanes load LANES consecutive P-byte
+// runs) x 64 / LANES rows per wave x 16 waves; LDS combines the
 // partial maxima.  Digit sums use SWAR: (word >> shift) & mask per byte, then
 // v_sad_u8 adds the four bytes.  Requires P in {32, 64} and reads that start
 // at g * P (R a multiple of P).
-template <int P>
+//
+// The combining is spread over the waves too: a wave takes one slice's maxima, then every
+// wave tests four of the 64 slots (one wave that did both walked 120 LDS reads and up to
+// 64 slots, each two scalar loads and an LDS read, one after another).  With 16 reads
+// per workgroup a lane sums one or no row instead of four and there are four times the workgroups,
+// which is what a matrix of few reads needs: 777 vectors and 1111 columns of 24 reads, 64 slots:
+// 7.9 us, 22.3 before; 2048 and 2048 of 32: 8.0, 21.4; 512 and 512 of 128 reads of 32 rows, 25
+// slots: 5.2, 8.6.  Bound: the digit sums (a shift, a mask and a sum per four digits and slice).
+template <int P, int LANES>
 __global__ __launch_bounds__(64 * DIGIT_WAVES) void k_digit_bits(
     const DigitJob a, const DigitJob b, i64 first_blocks, i64 kp, i64 G) {
     constexpr int CHUNKS = P / 16;
-    __shared__ int partial[DIGIT_WAVES][8][64];
+    constexpr int SUB = 64 / LANES;   // rows side by side in a wave
+    __shared__ int partial[DIGIT_WAVES][8][LANES];
+    __shared__ int maxima[8][LANES];
     const bool second = i64(blockIdx.y) >= first_blocks;
     const DigitJob &job = second ? b : a;
     const u8 *codes = job.codes;
@@ -74,23 +84,24 @@ __global__ __launch_bounds__(64 * DIGIT_WAVES) void k_digit_bits(
     const SliceLayout &layout = job.layout;
     const SlotTests &tests = job.tests;
     uint64_t *out = job.out;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const i64 g = i64(blockIdx.x) * 64 + lane;
+    const int lane = threadIdx.x & (LANES - 1), sub = (threadIdx.x & 63) / LANES;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 g = i64(blockIdx.x) * LANES + lane;
     const i64 rb = second ? i64(blockIdx.y) - first_blocks : i64(blockIdx.y);
     const int S = layout.count;
-    const int per = block / DIGIT_WAVES;
     int best[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     u32 masks[8];
 #pragma unroll
     for (int sl = 0; sl < 8; ++sl) masks[sl] = sl < S ? u32(layout.mask[sl]) * 0x01010101u : 0u;
     // Every row's loads are issued before the first digit sum.
-    constexpr int MAX_PER = 64 / DIGIT_WAVES;
+    constexpr int MAX_PER = 64 / (DIGIT_WAVES * SUB);
     uint4 chunk[MAX_PER][CHUNKS];
     bool live[MAX_PER];
 #pragma unroll
     for (int i = 0; i < MAX_PER; ++i) {
-        const i64 row = rb * block + wave * per + i;
-        live[i] = g < G && i < per && row < rows;
+        const int r = (i * DIGIT_WAVES + wave) * SUB + sub;
+        const i64 row = rb * block + r;
+        live[i] = g < G && r < block && row < rows;
         const uint4 *src = reinterpret_cast<const uint4 *>(codes + row * kp + g * P);
 #pragma unroll
         for (int c = 0; c < CHUNKS; ++c)
@@ -116,24 +127,36 @@ __global__ __launch_bounds__(64 * DIGIT_WAVES) void k_digit_bits(
         }
     }
 #pragma unroll
-    for (int sl = 0; sl < 8; ++sl) partial[wave][sl][lane] = best[sl];
-    __syncthreads();
-    if (wave > 0 || g >= G || rb * block >= rows) return;
-#pragma unroll
     for (int sl = 0; sl < 8; ++sl) {
-        if (sl >= S) break;
-        int m = best[sl];
-        for (int w = 1; w < DIGIT_WAVES; ++w) m = max(m, partial[w][sl][lane]);
-        partial[0][sl][lane] = m;
+#pragma unroll
+        for (int d = LANES; d < 64; d *= 2) best[sl] = max(best[sl], __shfl_xor(best[sl], d));
+        if (sub == 0) partial[wave][sl][lane] = best[sl];
     }
-    // Only this lane reads back its own words: no barrier needed.
+    __syncthreads();
+    if (wave < S && sub == 0) {
+        int m = 0;
+#pragma unroll
+        for (int w = 0; w < DIGIT_WAVES; ++w) m = max(m, partial[w][wave][lane]);
+        maxima[wave][lane] = m;
+    }
+    __syncthreads();
+    constexpr int SLOTS = 64 / DIGIT_WAVES;
+    u32 proven = 0;
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        const int slot = wave * SLOTS + i;
+        // (the slice of a slot that does not exist is not read as an index)
+        const bool exists = (tests.exists >> slot) & 1u;
+        const int sl = exists ? tests.slice[slot] : 0;
+        if (exists && maxima[sl][lane] <= tests.thr[slot]) proven |= 1u << i;
+    }
+    if (sub == 0) partial[wave][0][lane] = int(proven);   // (its maxima are read: the barrier)
+    __syncthreads();
+    if (wave > 0 || sub > 0 || g >= G) return;
     uint64_t bits = 0;
-    uint64_t slots = tests.exists;
-    while (slots) {
-        const int slot = __builtin_ctzll(slots);
-        slots &= slots - 1;
-        if (partial[0][tests.slice[slot]][lane] <= tests.thr[slot]) bits |= uint64_t(1) << slot;
-    }
+#pragma unroll
+    for (int w = 0; w < DIGIT_WAVES; ++w)
+        bits |= uint64_t(u32(partial[w][0][lane])) << (w * SLOTS);
     out[rb * G + g] = bits;
 }
 
@@ -424,8 +447,9 @@ __global__ __launch_bounds__(256, TN == 1 && KS == 1 ? 5 : 2) void k_ideal(const
         publish_status(args.status, args.mailbox);
 }
 
-template __global__ void k_digit_bits<32>(const DigitJob, const DigitJob, i64, i64, i64);
-template __global__ void k_digit_bits<64>(const DigitJob, const DigitJob, i64, i64, i64);
+template __global__ void k_digit_bits<32, 16>(const DigitJob, const DigitJob, i64, i64, i64);
+template __global__ void k_digit_bits<32, 64>(const DigitJob, const DigitJob, i64, i64, i64);
+template __global__ void k_digit_bits<64, 16>(const DigitJob, const DigitJob, i64, i64, i64);
 
 #define MF_IDEAL_INST(TN, KS) template __global__ void k_ideal<TN, KS>(const IdealPlan, const IdealArgs);
 MF_IDEAL_INST(2, 1)

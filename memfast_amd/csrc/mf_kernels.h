@@ -124,7 +124,7 @@ struct DigitJob {
     SlotTests tests;
     uint64_t *out;     // [ceil(rows / block), G]
 };
-template <int P>
+template <int P, int LANES>
 __global__ void k_digit_bits(const DigitJob a, const DigitJob b, i64 first_blocks, i64 kp, i64 G);
 
 // The same masks produced by the quantizers that wrote the codes (k_read_groups).
