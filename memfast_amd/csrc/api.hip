@@ -803,6 +803,16 @@ i64 wide_small_bytes(const mf_config *cfg, i64 n, i64 m, i64 p) {
     return align256(n * m * cfg->reads * p * cfg->cols * 4);
 }
 
+// Reads that k_wide_block takes: digit operands and one plane of terms, unless a tuned schedule's
+// LDS tier asks for k_noisy_wide, and tiles of 32 vectors by 128 columns for one round of four
+// workgroups per CU.  Nine by three slices of 64 rows, both with their sampling: 2048 x 4096 ->
+// 4096 (2048 tiles) 3.15 against 3.44 ms, sixteen by four 2048^3 (1024 tiles) 1.71 / 1.77; but 256 x
+// 4096 -> 4096 (256 tiles) 0.99 / 0.95, 4096 x 4096 -> 100 (128 tiles) 0.78 / 0.76.
+bool wide_block(const mf_config *cfg, i64 n, i64 cols, int tier_request) {
+    return !cfg->has_vnoise && wide_term_planes(cfg) == 1 && tier_request == 0 &&
+           (n + 31) / 32 * ((cols + 127) / 128) >= 1024;
+}
+
 // Batches that k_wide_small reads: no per-vector or per-slice noise (a tuned schedule's LDS tier
 // asks for k_noisy_wide), totals that fit where the terms would be, and where its time is the
 // lesser.  Both sample every cell once (2.8 ps per cell and weight slice).  Beside that, per read
@@ -908,6 +918,22 @@ int launch_noisy_wide(const mf_config *cfg, const NoisyWidePlan &plan, int ks,
         args.c_begin = c_begin;
         args.totals = totals;
         args.volt = volt;
+        args.CB = CB;
+        if (wide_block(cfg, n, cols, tier_request)) {
+            const dim3 tiles{unsigned((n + 31) / 32), unsigned((CB + 3) / 4), 1u};
+            const unsigned lds = unsigned(cfg->n_in * ks * 1024);
+#define MF_WIDE_BLOCK(KS, NL) \
+    hipLaunchKernelGGL((k_wide_block<KS, NL>), tiles, dim3(256), lds, s, plan, args)
+            if (ks == 4) {
+                if (cfg->has_nonlinear) MF_WIDE_BLOCK(4, true);
+                else MF_WIDE_BLOCK(4, false);
+            } else {
+                if (cfg->has_nonlinear) MF_WIDE_BLOCK(2, true);
+                else MF_WIDE_BLOCK(2, false);
+            }
+#undef MF_WIDE_BLOCK
+            continue;
+        }
         const dim3 grid{unsigned(CB), unsigned((n + 127) / 128), 1u};
         const bool nl = cfg->has_nonlinear != 0;
         // slice_pair read noise: a plane of terms per (weight, input) slice pair, staged in
@@ -2735,12 +2761,20 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                   : tier == 1 ? MF_WIDE_FN(2, WIDE_FRAGS_SMALL) : MF_WIDE_FN(2, WIDE_FRAGS_TINY);
 #undef MF_WIDE_FN
 #undef MF_WIDE_FN2
-        // (the matrix is not known here: one of 64 x 64 arrays)
+        // (the matrix is not known here: one of 64 x 64 arrays; without a batch, the tiers')
+        if (n > 0 && wide_block(cfg, n, 64 * i64(cfg->cols), variant_tier(variant))) {
+            fn = ks4 ? (nl ? reinterpret_cast<const void *>(&k_wide_block<4, true>)
+                           : reinterpret_cast<const void *>(&k_wide_block<4, false>))
+                     : (nl ? reinterpret_cast<const void *>(&k_wide_block<2, true>)
+                           : reinterpret_cast<const void *>(&k_wide_block<2, false>));
+            dynamic_lds = cfg->n_in * (ks4 ? 4 : 2) * 1024;
+        }
         if (n > 0 && wide_small(cfg, n, 64, 64, variant_tier(variant))) {
             fn = ks4 ? (nl ? reinterpret_cast<const void *>(&k_wide_small<4, true>)
                            : reinterpret_cast<const void *>(&k_wide_small<4, false>))
                      : (nl ? reinterpret_cast<const void *>(&k_wide_small<2, true>)
                            : reinterpret_cast<const void *>(&k_wide_small<2, false>));
+            dynamic_lds = 0;
             threads = 64 * cfg->n_w;
         }
     } else if (kernel_id == 0) {

@@ -270,6 +270,7 @@ struct NoisyWideArgs {
     double *out;           // fused: [n, ldo]; totals: [n, G, ldo]
     u32 *status;           // optional: MF_STATUS_OUTPUT for a non-finite fused output
     i64 n, kp, G, ldo, ldws, ncols, c_begin;
+    i64 CB;                // 32-column blocks of the chunk
     int totals;
     // Voltage variation: input operands [2][A][ceil(n/32)][kp/8][32] uint4 of 8 fp16 (hi,
     // lo) of digit * (1 + vv*z) from k_voltage_terms<u32>, read instead of the digits.
@@ -281,6 +282,10 @@ template <int KS>
 __global__ void k_split_wide(const mf_config cfg, const u32 *packed, const float *g_in, i64 m,
                              i64 p, i64 ncols, u32 seed, u64 event, i64 c_begin, i64 CB,
                              const NoisyWidePlan plan, uint4 *gs);
+// The wide read without voltage variation and slice_pair noise (grid: 32-vector tiles, 128-column
+// tiles; dynamic LDS n_in * KS KiB).
+template <int KS, bool NONLINEAR>
+__global__ void k_wide_block(const NoisyWidePlan plan, const NoisyWideArgs args);
 // The wide read of small batches, conductances sampled in place: integer totals [n, G, ncols]
 // (grid: 32-column blocks, reads; one wave per weight slice), and their FP64 restore and sum.
 template <int KS, bool NONLINEAR>

@@ -340,6 +340,149 @@ __global__ __launch_bounds__(256) void k_restore_sum_wide(const int *totals, i64
     if (!(fabs(s) <= DBL_MAX) && status) atomicOr(status, u32(MF_STATUS_OUTPUT));
 }
 
+// The read of digit operands under one plane of terms per weight slice (shared read noise or
+// none).  k_noisy_block's arrangement: four waves read the same 32 vectors through 32 columns each;
+// the digits of those vectors, every input slice of one read, are built once in LDS in MFMA operand
+// order, and a wave keeps one weight slice's terms in registers while it walks the input slices.
+// k_noisy_wide builds each digit in every wave (a quarter of its VALU work at nine by three
+// slices) and holds two chains of currents, for three waves per SIMD; here it is four.  The
+// order of the MFMAs within a pair, the converter and the sums are k_noisy_wide's: same bits.
+// 2048 x 4096 -> 4096, nine by three slices of 64 rows with their sampling: 3.15 ms, k_noisy_wide
+// 3.44 (S-curve 5.1 / 5.8; 32-row reads 4.3 / 4.7).  Bound: the two pipes' overlap (1.9e12 slice
+// operations in two terms take 1.5 ms of MFMA issue, the converter as much of the VALU's).
+template <int KS, bool NONLINEAR>
+__global__ __launch_bounds__(256, NONLINEAR ? 3 : 4) void k_wide_block(const NoisyWidePlan plan,
+                                                                       const NoisyWideArgs args) {
+    constexpr int P = 16 * KS;
+    extern __shared__ __align__(16) uint4 wide_digits[];   // [A][KS][64 lanes]
+    const float MAGIC = 12582912.0f;                        // 1.5 * 2^23
+    const u32 magic16 = 0x64006400u;                        // fp16 1024 in both halves
+    const int A = plan.n_in, W = plan.n_w;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lrow = lane & 31, lhalf = lane >> 5;
+
+    u32 vtile, ctile;
+    xcd_tile(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x, gridDim.y, vtile, ctile);
+    const i64 cb = i64(ctile) * 4 + wave;   // chunk-relative 32-column block
+    const i64 v0 = i64(vtile) * 32;
+    const int G = int(args.G);
+    const i64 kp = args.kp;
+    const bool live = cb < args.CB;   // the last workgroup may hold waves past the chunk
+    const i64 col_tile = args.c_begin + cb * 32;
+    const i64 n_out = v0 + lrow;
+    const bool live_n = n_out < args.n;
+    const uint4 *frag_base = args.gs + cb * i64(G) * W * NOISY_TERMS * KS * 64 + lane;
+
+    // Wave w builds the digits of 16-row step w % KS, every 4 / KS-th input slice; its codes are
+    // loaded a read ahead (rows past n read as zero).
+    const i64 vrows = (args.n - v0) < 32 ? (args.n - v0) : 32;
+    const __amdgpu_buffer_rsrc_t qbuf = wide_buffer(args.q16 + v0 * kp, vrows * kp * 2);
+    const int step = wave % KS, first = wave / KS;
+    const int q_off = (lrow * int(kp) + lhalf * 8 + step * 16) * 2;
+    uint4 qc = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qbuf, q_off, 0, 0));
+
+    double acc0[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc0[r] = 0.0;
+
+    for (int g = 0; g < G; ++g) {
+        __syncthreads();   // every wave is done with the previous read's digits
+        for (int a = first; a < A; a += 4 / KS)
+            wide_digits[(a * KS + step) * 64 + lane] = __builtin_bit_cast(
+                uint4, digits_magic(qc, plan.in_shift[a], plan.in_mask2[a], magic16));
+        __syncthreads();
+        if (g + 1 < G)
+            qc = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               qbuf, q_off + (g + 1) * P * 2, 0, 0));
+        if (!live) continue;
+
+        u32 T[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) T[r] = plan.bias;
+        for (int w = 0; w < W; ++w) {
+            v8h_w F[NOISY_TERMS][KS];
+            const uint4 *frag = frag_base + (i64(g) * W + w) * NOISY_TERMS * KS * 64;
+#pragma unroll
+            for (int term = 0; term < NOISY_TERMS; ++term)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    F[term][ks] = __builtin_bit_cast(v8h_w, frag[(term * KS + ks) * 64]);
+            const float top = MAGIC + plan.top[w], alpha = plan.alpha[w];
+            for (int a = 0; a < A; ++a) {
+                v8h_w D[KS];
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    D[ks] = __builtin_bit_cast(v8h_w, wide_digits[(a * KS + ks) * 64 + lane]);
+                v16f_w I = {};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int term = 0; term < NOISY_TERMS; ++term)
+                        I = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[term][ks], D[ks], I, 0, 0, 0);
+                const int f = plan.fa[a] * plan.fw[w];   // |fa*fw| < 2^23
+                const u32 f24 = u32(int(u32(f) << 8) >> 8);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float y = (NONLINEAR ? scurve(I[r], alpha) : I[r]) + MAGIC;
+                    y = __builtin_amdgcn_fmed3f(y, MAGIC, top);
+                    T[r] += u32(int(__float_as_uint(y) << 8) >> 8) * f24;
+                }
+            }
+        }
+
+        // FP64 restore and torch's cascade over reads (level step 16; level 1 is kept in `out`,
+        // reads < 256).
+        if (args.totals) {
+            if (live_n) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const i64 c = col_tile + (r >> 2) * 8 + lhalf * 4 + (r & 3);
+                    if (c < args.ncols)
+                        args.out[(n_out * G + g) * args.ldo + c] = double(int(T[r]));
+                }
+            }
+            continue;
+        }
+        const double xs = live_n ? args.xscale[n_out * G + g] : 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const i64 c = col_tile + (r >> 2) * 8 + lhalf * 4 + (r & 3);
+            const double ws = c < args.ncols ? args.wscale[i64(g) * args.ldws + c] : 0.0;
+            acc0[r] = acc0[r] + restore_fast(int(T[r]), xs, ws);
+        }
+        if (((g + 1) & 15) == 0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const i64 c = col_tile + (r >> 2) * 8 + lhalf * 4 + (r & 3);
+                if (live_n && c < args.ncols) {
+                    double *dst = args.out + n_out * args.ldo + c;
+                    *dst = g + 1 == 16 ? acc0[r] : *dst + acc0[r];
+                }
+                acc0[r] = 0.0;
+            }
+        }
+    }
+    if (args.totals || !live || !live_n) return;
+
+    bool finite = true;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const i64 c = col_tile + (r >> 2) * 8 + lhalf * 4 + (r & 3);
+        if (c >= args.ncols) continue;
+        double *dst = args.out + n_out * args.ldo + c;
+        const double s = acc0[r] + (G >= 16 ? *dst : 0.0);
+        *dst = s;
+        finite = finite && fabs(s) <= DBL_MAX;
+    }
+    if (!finite && args.status) atomicOr(args.status, u32(MF_STATUS_OUTPUT));
+}
+
+template __global__ void k_wide_block<2, false>(const NoisyWidePlan, const NoisyWideArgs);
+template __global__ void k_wide_block<2, true>(const NoisyWidePlan, const NoisyWideArgs);
+template __global__ void k_wide_block<4, false>(const NoisyWidePlan, const NoisyWideArgs);
+template __global__ void k_wide_block<4, true>(const NoisyWidePlan, const NoisyWideArgs);
+
 template <int KS, bool NONLINEAR, int FRMAX, bool VNOISE, bool SLICE>
 __global__ __launch_bounds__(256, wide_blocks_per_cu(FRMAX, NONLINEAR)) void k_noisy_wide(
     const NoisyWidePlan plan,
