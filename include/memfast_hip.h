@@ -220,6 +220,22 @@ int mf_mm(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n
           float *out, int64_t ldo, void *workspace, int64_t workspace_bytes, int32_t variant,
           uint32_t *status, void *stream);
 
+/* mf_mm (without g) with the noisy-device MFMA read's conductance terms in a buffer of their own,
+ * for callers that keep a program's terms between reads: `terms` (256-byte aligned, at least
+ * mf_mm_terms_bytes()) receives the terms of every column, or with MF_MM_REUSE_TERMS still holds
+ * them, and is only read then.  `workspace` (mf_mm_workspace() less mf_mm_terms_bytes(); NULL where
+ * that is 0) belongs to this call alone: reads of one program on several streams share the terms,
+ * once they are written, and take a workspace each.  Other read kernels ignore `terms`. */
+int mf_mm_kept(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n, int64_t m,
+               const uint8_t *packed, const uint8_t *packed_t, const float *wscale, int64_t p,
+               int64_t out_cols, int64_t k_rows, uint32_t seed, uint64_t event, float *out,
+               int64_t ldo, void *terms, int64_t terms_bytes, void *workspace,
+               int64_t workspace_bytes, int32_t variant, uint32_t *status, void *stream);
+
+/* Bytes of `terms` of mf_mm_kept and mf_gru_sequence_kept for m x p arrays; 0 where the noisy
+ * MFMA read does not apply or its terms depend on the read event (read noise). */
+int mf_mm_terms_bytes(const mf_config *cfg, int64_t m, int64_t p, int64_t *bytes);
+
 /* Both quantizations and the ideal read in two launches (memfast/functional.py:130-136:
  * the RHS program of Simulator._matrix_for, memfast/simulator.py:133-171 with
  * quantization.py:82-137, read by AnalogMatrix.forward, :618-646): x [n, k] FP32 (leading
@@ -380,6 +396,17 @@ int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_
                     int64_t ld_hidden, void *workspace, int64_t workspace_bytes, int32_t variant,
                     float *out, int64_t out_step, int64_t out_row, uint32_t *status,
                     void *stream);
+
+/* mf_gru_sequence with the hidden program's conductance terms in `terms`, as mf_mm_kept. */
+int mf_gru_sequence_kept(const mf_config *cfg, int64_t steps, int32_t reverse, int64_t batch,
+                         int64_t width, const float *projected, int64_t proj_step,
+                         int64_t proj_row, const float *h0, int64_t ld_h0, int64_t gr, int64_t gc,
+                         uint32_t *work, float *scale, uint8_t *q, float *xscale,
+                         const uint8_t *packed, const uint8_t *packed_t, const float *wscale,
+                         int64_t m, int64_t p, const float *bias, uint32_t seed, uint64_t event0,
+                         float *hidden, int64_t ld_hidden, void *terms, int64_t terms_bytes,
+                         void *workspace, int64_t workspace_bytes, int32_t variant, float *out,
+                         int64_t out_step, int64_t out_row, uint32_t *status, void *stream);
 
 /* Overflow-safe FP64 restore and read sum of one chunk of `width` tiles
  * (memfast/simulator.py:57-66 restore_scales and :578-585, the wide/retry path

@@ -544,12 +544,15 @@ bool terms_event_independent(const mf_config *cfg) { return !cfg->has_read; }
 // for every column (a previous call with the same codes, seed and config).
 // ocols, g_run: output columns computed and reads executed (the logical matrix;
 // columns past ocols are left unwritten, reads past g_run hold only padding).
+// terms: optional buffer of noisy_terms_bytes that the terms of every column go to (or are in)
+// instead of the workspace, which then holds the split's totals and the voltage operands alone.
 int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *q,
                  const float *xscale, i64 n, i64 m, const u8 *packed_t, const float *wscale, i64 p,
                  const float *g, u32 seed, u64 event, float *out, i64 ldo, void *workspace,
                  i64 bytes, int totals, u32 *status, hipStream_t s, bool reuse = false,
                  i64 ocols = -1, i64 g_run = -1, int split_request = 0,
-                 const float **split_totals = nullptr, bool *split_restored = nullptr) {
+                 const float **split_totals = nullptr, bool *split_restored = nullptr,
+                 void *terms = nullptr) {
     const i64 kp = m * cfg->rows, ncols = p * cfg->cols, G = m * cfg->reads;
     if (ocols < 0) ocols = ncols;
     if (g_run < 0) g_run = G;
@@ -572,17 +575,18 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
     const i64 split = totals ? 1 : noisy_split(cfg, n, m, p, split_request);
     const i64 full = noisy_terms_bytes(cfg, m, p);
     const i64 scratch = noisy_scratch_bytes(cfg, n, m, p, split_request);
-    const bool use_split = split > 1 && bytes >= full + scratch;
+    const i64 held = terms ? 0 : full;   // bytes of the workspace that the terms take
+    const bool use_split = split > 1 && bytes >= held + scratch;
     if (split > 1 && split_request > 1 && !use_split)
         return fail(MF_E_RESOURCE,
                     "workspace of %lld bytes below the %lld a %lld-way read split needs",
-                    static_cast<long long>(bytes), static_cast<long long>(full + scratch),
+                    static_cast<long long>(bytes), static_cast<long long>(held + scratch),
                     static_cast<long long>(split));
-    const i64 max_cb = use_split ? full / per_block : (bytes / per_block) / 2 * 2;
+    const i64 max_cb = use_split || terms ? full / per_block : (bytes / per_block) / 2 * 2;
     if (max_cb < 2) return fail(MF_E_RESOURCE, "workspace below one 64-column chunk");
     reuse = reuse && g == nullptr && terms_event_independent(cfg) && max_cb * 32 >= ocols;
-    uint4 *gs = static_cast<uint4 *>(workspace);
-    float *partial = use_split ? reinterpret_cast<float *>(static_cast<char *>(workspace) + full)
+    uint4 *gs = static_cast<uint4 *>(terms ? terms : workspace);
+    float *partial = use_split ? reinterpret_cast<float *>(static_cast<char *>(workspace) + held)
                                : nullptr;
     for (i64 c_begin = 0; c_begin < ocols; c_begin += max_cb * 32) {
         const i64 cols = (ocols - c_begin) < max_cb * 32 ? (ocols - c_begin) : max_cb * 32;
@@ -1774,7 +1778,7 @@ static i64 reads_with_rows(const mf_config *cfg, i64 m, i64 k_rows) {
     return used < G ? used : G;
 }
 
-// mf_mm; with `split_totals` a noisy MFMA read split across blocks leaves its totals to the
+// mf_mm (with `terms`, mf_mm_kept); with `split_totals` a noisy MFMA read split across blocks leaves its totals to the
 // caller (*split_totals, [n, G, p*C]) instead of restoring them into `out` (null otherwise);
 // *split_restored says whether they are already restored ((float(T) * xs) * ws).
 static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n,
@@ -1782,7 +1786,8 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
                    int64_t p, int64_t out_cols, int64_t k_rows, const void *g, uint32_t seed,
                    uint64_t event, float *out, int64_t ldo, void *workspace,
                    int64_t workspace_bytes, int32_t variant, uint32_t *status, void *stream,
-                   const float **split_totals, bool *split_restored = nullptr) {
+                   const float **split_totals, bool *split_restored = nullptr,
+                   void *terms = nullptr, i64 terms_bytes = 0) {
     if (split_totals) *split_totals = nullptr;
     const int valid = check_narrow(cfg);
     if (valid) return valid;
@@ -1833,13 +1838,19 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
                             out_cols, g_run, out, ldo, variant, status, s);
     }
     NoisyPlan noisy;
-    if (!g && packed_t && aligned && workspace && ideal_extent_ok(cfg, n, m, p) &&
-        noisy_extent_ok(n, m, cfg) && build_noisy_plan(cfg, m, p, &noisy, &ks, &why) &&
-        workspace_bytes >= noisy_voltage_bytes(cfg, n, m) + 2 * noisy_block_bytes(cfg, m)) {
-        return launch_noisy(cfg, noisy, ks, q, xscale, n, m, packed_t, wscale, p, nullptr, seed,
-                            event, out, ldo, workspace, workspace_bytes, 0, status, s,
-                            (variant & MF_MM_REUSE_TERMS) != 0, out_cols, g_run,
-                            variant_split(variant), split_totals, split_restored);
+    if (!g && packed_t && aligned && (workspace || terms) && ideal_extent_ok(cfg, n, m, p) &&
+        noisy_extent_ok(n, m, cfg) && build_noisy_plan(cfg, m, p, &noisy, &ks, &why)) {
+        const i64 full = noisy_terms_bytes(cfg, m, p);
+        if (terms && (terms_bytes < full || reinterpret_cast<uintptr_t>(terms) % 256))
+            return fail(MF_E_INVALID, "kept terms need %lld bytes, 256-byte aligned",
+                        static_cast<long long>(full));
+        if (!workspace) workspace_bytes = 0;
+        if (workspace_bytes >=
+            noisy_voltage_bytes(cfg, n, m) + (terms ? 0 : 2 * noisy_block_bytes(cfg, m)))
+            return launch_noisy(cfg, noisy, ks, q, xscale, n, m, packed_t, wscale, p, nullptr,
+                                seed, event, out, ldo, workspace, workspace_bytes, 0, status, s,
+                                (variant & MF_MM_REUSE_TERMS) != 0, out_cols, g_run,
+                                variant_split(variant), split_totals, split_restored, terms);
     }
     if (!g && needs_conductances(cfg))
         return fail(MF_E_INVALID, "device noise needs restored conductances (g)");
@@ -1882,6 +1893,30 @@ int mf_mm(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n
           uint32_t *status, void *stream) {
     return mm_read(cfg, q, xscale, n, m, packed, packed_t, wscale, p, out_cols, k_rows, g, seed,
                    event, out, ldo, workspace, workspace_bytes, variant, status, stream, nullptr);
+}
+
+int mf_mm_terms_bytes(const mf_config *cfg, int64_t m, int64_t p, int64_t *bytes) {
+    const int status = check_narrow(cfg);
+    if (status) return status;
+    if (!bytes || m < 1 || p < 1) return fail(MF_E_INVALID, "invalid terms query");
+    NoisyPlan noisy;
+    int ks = 0;
+    const char *why = "";
+    *bytes = terms_event_independent(cfg) && build_noisy_plan(cfg, m, p, &noisy, &ks, &why)
+                 ? noisy_terms_bytes(cfg, m, p)
+                 : 0;
+    return MF_OK;
+}
+
+int mf_mm_kept(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n, int64_t m,
+               const uint8_t *packed, const uint8_t *packed_t, const float *wscale, int64_t p,
+               int64_t out_cols, int64_t k_rows, uint32_t seed, uint64_t event, float *out,
+               int64_t ldo, void *terms, int64_t terms_bytes, void *workspace,
+               int64_t workspace_bytes, int32_t variant, uint32_t *status, void *stream) {
+    if (!terms) return fail(MF_E_INVALID, "mf_mm_kept takes a terms buffer");
+    return mm_read(cfg, q, xscale, n, m, packed, packed_t, wscale, p, out_cols, k_rows, nullptr,
+                   seed, event, out, ldo, workspace, workspace_bytes, variant, status, stream,
+                   nullptr, nullptr, terms, terms_bytes);
 }
 
 int mf_mm_from_float(const mf_config *cfg, const float *x, int64_t n, int64_t k, int64_t ldx,
@@ -2231,15 +2266,15 @@ int mf_gru_gates(const float *inputs, int64_t ldi, const float *hidden, int64_t 
     return check_launch("GRU gates");
 }
 
-int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_t batch,
-                    int64_t width, const float *projected, int64_t proj_step, int64_t proj_row,
-                    const float *h0, int64_t ld_h0, int64_t gr, int64_t gc, uint32_t *work,
-                    float *scale, uint8_t *q, float *xscale, const uint8_t *packed,
-                    const uint8_t *packed_t, const float *wscale, int64_t m, int64_t p,
-                    const float *bias, uint32_t seed, uint64_t event0, float *hidden,
-                    int64_t ld_hidden, void *workspace, int64_t workspace_bytes, int32_t variant,
-                    float *out, int64_t out_step, int64_t out_row, uint32_t *status,
-                    void *stream) {
+static int gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_t batch,
+                        int64_t width, const float *projected, int64_t proj_step, int64_t proj_row,
+                        const float *h0, int64_t ld_h0, int64_t gr, int64_t gc, uint32_t *work,
+                        float *scale, uint8_t *q, float *xscale, const uint8_t *packed,
+                        const uint8_t *packed_t, const float *wscale, int64_t m, int64_t p,
+                        const float *bias, uint32_t seed, uint64_t event0, float *hidden,
+                        int64_t ld_hidden, void *terms, int64_t terms_bytes, void *workspace,
+                        int64_t workspace_bytes, int32_t variant, float *out, int64_t out_step,
+                        int64_t out_row, uint32_t *status, void *stream) {
     const int valid = check_narrow(cfg);
     if (valid) return valid;
     if (!projected || !h0 || !q || !xscale || !scale || !packed || !wscale || !hidden || !out ||
@@ -2270,7 +2305,7 @@ int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_
             if (rc) return rc;
         }
         // The first read writes the program's event-independent conductance terms
-        // into the workspace (unless the caller's variant says they are there);
+        // into the workspace or `terms` (unless the caller's variant says they are there);
         // later reads of the same program reuse them.
         const int32_t v = i == 0 ? variant : (variant | MF_MM_REUSE_TERMS);
         const float *totals = nullptr;
@@ -2278,7 +2313,7 @@ int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_
         rc = mm_read(cfg, q, xscale, batch, m, packed, packed_t, wscale, p, 3 * width, width,
                      nullptr, seed, event0 + uint64_t(i), hidden, ld_hidden, workspace,
                      workspace_bytes, v, status, stream, fused ? &totals : nullptr,
-                     fused ? &restored : nullptr);
+                     fused ? &restored : nullptr, terms, terms_bytes);
         if (rc) return rc;
         if (fused) {
             GruStepArgs a{};
@@ -2322,6 +2357,37 @@ int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_
         if (rc) return rc;
     }
     return MF_OK;
+}
+
+int mf_gru_sequence(const mf_config *cfg, int64_t steps, int32_t reverse, int64_t batch,
+                    int64_t width, const float *projected, int64_t proj_step, int64_t proj_row,
+                    const float *h0, int64_t ld_h0, int64_t gr, int64_t gc, uint32_t *work,
+                    float *scale, uint8_t *q, float *xscale, const uint8_t *packed,
+                    const uint8_t *packed_t, const float *wscale, int64_t m, int64_t p,
+                    const float *bias, uint32_t seed, uint64_t event0, float *hidden,
+                    int64_t ld_hidden, void *workspace, int64_t workspace_bytes, int32_t variant,
+                    float *out, int64_t out_step, int64_t out_row, uint32_t *status,
+                    void *stream) {
+    return gru_sequence(cfg, steps, reverse, batch, width, projected, proj_step, proj_row, h0,
+                        ld_h0, gr, gc, work, scale, q, xscale, packed, packed_t, wscale, m, p,
+                        bias, seed, event0, hidden, ld_hidden, nullptr, 0, workspace,
+                        workspace_bytes, variant, out, out_step, out_row, status, stream);
+}
+
+int mf_gru_sequence_kept(const mf_config *cfg, int64_t steps, int32_t reverse, int64_t batch,
+                         int64_t width, const float *projected, int64_t proj_step,
+                         int64_t proj_row, const float *h0, int64_t ld_h0, int64_t gr, int64_t gc,
+                         uint32_t *work, float *scale, uint8_t *q, float *xscale,
+                         const uint8_t *packed, const uint8_t *packed_t, const float *wscale,
+                         int64_t m, int64_t p, const float *bias, uint32_t seed, uint64_t event0,
+                         float *hidden, int64_t ld_hidden, void *terms, int64_t terms_bytes,
+                         void *workspace, int64_t workspace_bytes, int32_t variant, float *out,
+                         int64_t out_step, int64_t out_row, uint32_t *status, void *stream) {
+    if (!terms) return fail(MF_E_INVALID, "mf_gru_sequence_kept takes a terms buffer");
+    return gru_sequence(cfg, steps, reverse, batch, width, projected, proj_step, proj_row, h0,
+                        ld_h0, gr, gc, work, scale, q, xscale, packed, packed_t, wscale, m, p,
+                        bias, seed, event0, hidden, ld_hidden, terms, terms_bytes, workspace,
+                        workspace_bytes, variant, out, out_step, out_row, status, stream);
 }
 
 int mf_stable_sum(const mf_config *cfg, const float *totals, int64_t n, int64_t G, int64_t width,

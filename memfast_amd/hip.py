@@ -188,6 +188,13 @@ SIGNATURES = {
                            _P, _I64, _P], ct.c_int),
     "mf_profile_kernels": ([_I32], ct.c_int),
     "mf_profile_collect": ([ct.POINTER(_I64), ct.POINTER(ct.c_double)], ct.c_int),
+    "mf_mm_kept": ([_CFG, _P, _P, _I64, _I64, _P, _P, _P, _I64, _I64, _I64, ct.c_uint32,
+                    ct.c_uint64, _P, _I64, _P, _I64, _P, _I64, _I32, _P, _P], ct.c_int),
+    "mf_mm_terms_bytes": ([_CFG, _I64, _I64, ct.POINTER(_I64)], ct.c_int),
+    "mf_gru_sequence_kept": ([_CFG, _I64, _I32, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64,
+                              _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _P, ct.c_uint32,
+                              ct.c_uint64, _P, _I64, _P, _I64, _P, _I64, _I32, _P, _I64, _I64,
+                              _P, _P], ct.c_int),
     "mf_mm_workspace": ([_CFG, _I64, _I64, _I64, _I32, ct.POINTER(_I64)], ct.c_int),
     "mf_mm_kernel": ([_CFG, _I64, _I64, _I64, _I32, ct.POINTER(_I32)], ct.c_int),
     "mf_resources_query": ([_CFG, _I32, _I64, _I32, ct.POINTER(MFResources)], ct.c_int),
@@ -835,8 +842,8 @@ def terms_event_independent(config):
 
 
 def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=None, out=None,
-       variant=0, status=None, workspace=None, reuse_terms=False, out_cols=None, k_rows=None,
-       split_budget=None):
+       variant=0, status=None, workspace=None, terms=None, reuse_terms=False, out_cols=None,
+       k_rows=None, split_budget=None):
     """Fused read + scale restore: [N, p*C] FP32, summed over reads in torch's order.
 
     Wide configurations: ``packed_t`` is the uint32 kernel copy of the codes
@@ -844,7 +851,8 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
     ``workspace`` (optional, at least ``mm_workspace_bytes``) is the MFMA
     kernels' scratch; with ``reuse_terms`` it still holds the conductance terms
     a previous call of this program sampled (honoured when they do not depend
-    on the read event).  ``out_cols``/``k_rows`` (default: all) are the logical
+    on the read event).  ``terms`` (optional, at least ``mm_terms_bytes``) takes those
+    terms instead, and the workspace is this call's own.  ``out_cols``/``k_rows`` (default: all) are the logical
     output columns and input rows; the MFMA kernels leave columns past
     ``out_cols`` unwritten and skip reads wholly past row ``k_rows``.  ``split_budget``
     (optional) bounds the bytes of totals that a general read may be split through.
@@ -870,9 +878,14 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
         packed_t = None
     if out is None:
         out = torch.empty((n, p * c), dtype=torch.float32, device=q.device)
+    if packed_t is None or kernel != 2:
+        terms = None
     if packed_t is not None and kernel:
         size = mm_workspace_bytes(config, n, m, p, variant & ~REUSE_TERMS)
-        if workspace is None:
+        if terms is not None:
+            size -= mm_terms_bytes(config, m, p)
+            workspace = torch.empty(max(1, size), dtype=torch.uint8, device=q.device)
+        elif workspace is None:
             workspace = torch.empty(max(1, size), dtype=torch.uint8, device=q.device)
             reuse_terms = False
         elif workspace.numel() < size or workspace.device != q.device:
@@ -888,18 +901,19 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
     # temporary could be handed to the next conversion by the caching allocator).
     q, xscale = q.contiguous(), xscale.contiguous()
     packed, wscale = packed.contiguous(), wscale.contiguous()
+    lib = library()
+    operands = (ct.byref(descriptor(config)), _ptr(q), _ptr(xscale), n, m, _ptr(packed),
+                _ptr(packed_t), _ptr(wscale), p, p * c if out_cols is None else out_cols,
+                m * r if k_rows is None else k_rows)
+    scratch = (_ptr(workspace), 0 if workspace is None else workspace.numel(), variant,
+               _ptr(status), _stream(q.device))
     with _on(q.device):
-        check(
-            library().mf_mm(
-                ct.byref(descriptor(config)), _ptr(q), _ptr(xscale), n,
-                m, _ptr(packed), _ptr(packed_t), _ptr(wscale), p,
-                p * c if out_cols is None else out_cols, m * r if k_rows is None else k_rows,
-                _ptr(g), seed, event, _ptr(out), out.stride(0), _ptr(workspace),
-                0 if workspace is None else workspace.numel(), variant, _ptr(status),
-                _stream(q.device),
-            ),
-            "mm",
-        )
+        if terms is not None:
+            check(lib.mf_mm_kept(*operands, seed, event, _ptr(out), out.stride(0), _ptr(terms),
+                                 terms.numel(), *scratch), "mm")
+        else:
+            check(lib.mf_mm(*operands, _ptr(g), seed, event, _ptr(out), out.stride(0), *scratch),
+                  "mm")
     return out
 
 
@@ -943,6 +957,16 @@ def mm_workspace_bytes(config, n, m, p, variant=0):
     size = ct.c_int64()
     check(library().mf_mm_workspace(ct.byref(descriptor(config)), n, m, p, variant,
                                     ct.byref(size)), "workspace size")
+    return size.value
+
+
+@lru_cache(maxsize=4096)
+def mm_terms_bytes(config, m, p):
+    """Bytes of the conductance terms that reads of one program can share (``mm``'s ``terms``);
+    0 where the read has none or samples them anew on every read event."""
+    size = ct.c_int64()
+    check(library().mf_mm_terms_bytes(ct.byref(descriptor(config)), m, p, ct.byref(size)),
+          "terms size")
     return size.value
 
 
@@ -1071,12 +1095,12 @@ def gru_gates(inputs, hidden, hx):
 
 
 def gru_sequence(config, projected, h0, packed, packed_t, wscale, bias, seed, event, *, reverse,
-                 status, workspace, reuse_terms=False):
+                 status, workspace=None, terms=None, reuse_terms=False):
     """One GRU direction's hidden reads and gates (``mf_gru_sequence``): ``projected``
     [T, B, 3H] FP32 input projections, ``h0`` [B, H] FP32; the hidden program's packed
     codes, kernel codes ``packed_t``, read scales ``wscale`` [G, p*C], FP32 ``bias`` [3H]
-    or None and ``seed``; step i reads at event ``event + i``.  Returns the states
-    [T, B, H] in time order.  Non-finite values set bits of ``status``, which is not read."""
+    or None and ``seed``; step i reads at event ``event + i``.  ``workspace``, ``terms``
+    and ``reuse_terms`` are ``mm``'s.  Returns the states [T, B, H] in time order.  Non-finite values set bits of ``status``, which is not read."""
     supported(config)
     require_device(projected)
     if config.wide:
@@ -1093,10 +1117,16 @@ def gru_sequence(config, projected, h0, packed, packed_t, wscale, bias, seed, ev
     if not shapes_ok:
         raise ValueError("gru_sequence takes FP32 [T, B, 3H] projections, [B, H] states and a "
                          "matching hidden program")
-    size = mm_workspace_bytes(config, batch, m, p, 0)
-    if workspace.numel() < size or workspace.device != projected.device:
-        raise ValueError(f"gru_sequence workspace needs {size} bytes on {projected.device}")
     device = projected.device
+    size = mm_workspace_bytes(config, batch, m, p, 0)
+    if terms is not None:
+        size -= mm_terms_bytes(config, m, p)
+        workspace = None
+    if workspace is None:
+        workspace = torch.empty(max(1, size), dtype=torch.uint8, device=device)
+        reuse_terms = reuse_terms and terms is not None
+    elif workspace.numel() < size or workspace.device != device:
+        raise ValueError(f"gru_sequence workspace needs {size} bytes on {device}")
     q = torch.empty((batch, m, r), dtype=torch.uint8, device=device)
     xscale = torch.empty((batch, m * config.reads_per_array), dtype=torch.float32, device=device)
     gr, gc = _group_dims((batch, width), config.input_quant_gran)
@@ -1108,18 +1138,16 @@ def gru_sequence(config, projected, h0, packed, packed_t, wscale, bias, seed, ev
     hidden = torch.empty((batch, p * c), dtype=torch.float32, device=device)
     out = torch.empty((steps, batch, width), dtype=torch.float32, device=device)
     wscale = wscale.contiguous()
-    with _on(device):
-        check(
-            library().mf_gru_sequence(
-                ct.byref(descriptor(config)), steps, int(reverse), batch, width, _ptr(projected),
+    operands = (ct.byref(descriptor(config)), steps, int(reverse), batch, width, _ptr(projected),
                 batch * three, three, _ptr(h0), h0.stride(0), gr, gc, work, scale, _ptr(q),
                 _ptr(xscale), _ptr(packed), _ptr(packed_t), _ptr(wscale), m, p, _ptr(bias), seed,
-                event, _ptr(hidden), p * c, _ptr(workspace), workspace.numel(),
-                REUSE_TERMS if reuse_terms else 0, _ptr(out), batch * width, width, _ptr(status),
-                _stream(device),
-            ),
-            "GRU sequence",
-        )
+                event, _ptr(hidden), p * c)
+    kept = () if terms is None else (_ptr(terms), terms.numel())
+    entry = library().mf_gru_sequence if terms is None else library().mf_gru_sequence_kept
+    with _on(device):
+        check(entry(*operands, *kept, _ptr(workspace), workspace.numel(),
+                    REUSE_TERMS if reuse_terms else 0, _ptr(out), batch * width, width,
+                    _ptr(status), _stream(device)), "GRU sequence")
     return out
 
 

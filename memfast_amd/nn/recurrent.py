@@ -379,22 +379,21 @@ def _native_steps(cell, projected, order, hidden):
     config = matrix.config
     batch = hidden.shape[0]
     arrays = -(-matrix.in_features // config.array_size[0])
-    codes_t = matrix._column_codes()
-    source = None
-    if hip.mm_kernel(config, batch, arrays, matrix.p) == 2 and hip.terms_event_independent(config):
-        workspace, reuse, source = matrix._terms_workspace(batch, arrays, hidden.device, codes_t)
-    else:
-        workspace = hip._workspace(config, batch, arrays, matrix.p, hidden.device)
-        reuse = False
+    keeps = (hip.mm_kernel(config, batch, arrays, matrix.p) == 2
+             and hip.terms_event_independent(config))
     status = hip.status_word(hidden.device)
     bias = None if matrix.bias is None else matrix.bias.contiguous()
     columns = matrix.p * config.array_size[1]
-    states = hip.gru_sequence(config, projected.contiguous(), hidden.contiguous(), matrix.packed,
-                              codes_t, matrix.weight_scale.reshape(-1, columns), bias,
-                              matrix.seed, matrix._event, reverse=order[0] > order[-1],
-                              status=status, workspace=workspace, reuse_terms=reuse)
-    if source is not None:
-        matrix._terms_source = source
+    with matrix._kept.lock:
+        codes_t = matrix._column_codes()
+        terms, reuse, source = (matrix._terms(arrays, hidden.device, codes_t) if keeps
+                                else (None, False, None))
+        states = hip.gru_sequence(config, projected.contiguous(), hidden.contiguous(),
+                                  matrix.packed, codes_t, matrix.weight_scale.reshape(-1, columns),
+                                  bias, matrix.seed, matrix._event, reverse=order[0] > order[-1],
+                                  status=status, terms=terms, reuse_terms=reuse)
+        if keeps and not reuse:
+            matrix._kept.queued(source)
     if int(status.item()):
         return None
     matrix._event += len(order)

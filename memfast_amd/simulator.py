@@ -29,6 +29,7 @@ from torch import nn
 
 from . import checkpoint, hip, host_order, tuning
 from .config import Config
+from .kept import KeptTerms
 from .quantization import (_signed, check_read_scales, expanded_parameter, pack_weight,
                            read_starts, row_reads)
 from .tuning import default_schedule, schedule_grid
@@ -528,8 +529,7 @@ class AnalogMatrix(nn.Module):
         self.seed = self.config.seed ^ _name_tag(name)
         self._prepared = {}          # tuned schedules by (input shape, dtype)
         self._kernel_codes = None    # (codes key, the kernels' copy of the codes)
-        self._workspace = None       # noisy MFMA scratch kept across reads
-        self._terms_source = None    # (kernel codes, version, seed) of the terms it holds
+        self._kept = KeptTerms()     # conductance terms kept across reads
         if column_codes is not None:
             self._kernel_codes = (self._codes_key(), column_codes)
 
@@ -540,10 +540,14 @@ class AnalogMatrix(nn.Module):
 
     def _column_codes(self):
         """The kernels' copy of the codes (hip.kernel_codes), refreshed on change."""
-        key = self._codes_key()
-        if self._kernel_codes is None or self._kernel_codes[0] != key:
-            self._kernel_codes = (key, hip.kernel_codes(self.packed, self.config))
-        return self._kernel_codes[1]
+        with self._kept.lock:
+            key = self._codes_key()
+            if self._kernel_codes is None or self._kernel_codes[0] != key:
+                self._kernel_codes = (key, hip.kernel_codes(self.packed, self.config))
+                self._kept.built(self._kernel_codes[1])
+            codes = self._kernel_codes[1]
+            self._kept.order_codes(codes)
+            return codes
 
     def _accepts(self, tiles):
         """Whether freshly quantized ``tiles`` can replace this program's in place."""
@@ -738,7 +742,6 @@ class AnalogMatrix(nn.Module):
         else:
             budget = (self.simulator.workspace_bytes if self.simulator.mode == "tuned" else None)
             kernel = tuning.read_kernel(config, q.shape[0], q.shape[1], self.p, budget)
-            codes_t = self._column_codes() if config.wide or kernel else None
             status = hip.status_word(q.device) if status is None else status
             if not defer and self._output_bounded(q.shape[1]):
                 # The quantizer's bits are the only ones this read can leave: publish them
@@ -746,19 +749,20 @@ class AnalogMatrix(nn.Module):
                 box = self.simulator._layer_mailbox()
                 hip.status_publish(status, box)
             variant = tuning.schedule_variant(schedule)
-            workspace, reuse, source = None, False, None
-            if kernel == 2 and hip.terms_event_independent(config):
-                workspace, reuse, source = self._terms_workspace(q.shape[0], q.shape[1], q.device,
-                                                                 codes_t, variant)
             # A tuned read's totals stay within the budget its schedule was admitted under.
             left = (None if budget is None else budget - tuning.workspace_need(
                 config, q.shape[0], q.shape[1], self.p, schedule, budget))
-            output = hip.mm(q, xscale, packed, codes_t, self.weight_scale.reshape(-1, columns),
-                            config, self.seed, event, variant=variant, status=status,
-                            workspace=workspace, reuse_terms=reuse, split_budget=left,
-                            out_cols=self.out_features, k_rows=self.in_features)
-            if source is not None:
-                self._terms_source = source
+            with self._kept.lock:
+                codes_t = self._column_codes() if config.wide or kernel else None
+                keeps = kernel == 2 and hip.terms_event_independent(config)
+                terms, reuse, source = (self._terms(q.shape[1], q.device, codes_t) if keeps
+                                        else (None, False, None))
+                output = hip.mm(q, xscale, packed, codes_t, self.weight_scale.reshape(-1, columns),
+                                config, self.seed, event, variant=variant, status=status,
+                                terms=terms, reuse_terms=reuse, split_budget=left,
+                                out_cols=self.out_features, k_rows=self.in_features)
+                if keeps and not reuse:
+                    self._kept.queued(source)
         # An FP32 read's bias goes through a kernel that also flags non-finite sums and drops
         # the array columns past the layer's.
         checked_bias = (self.bias is not None and self.zero_correction is None
@@ -827,23 +831,21 @@ class AnalogMatrix(nn.Module):
         bound = reads * self.config.reconstruction_bound * xs * ws * 1.07 + bias
         return math.isfinite(bound) and bound < torch.finfo(torch.float32).max / 2
 
-    def _terms_workspace(self, rows, arrays, device, codes_t, variant=tuning.DEFAULT_VARIANT):
-        """Workspace of the noisy MFMA read kept across calls, and whether it still holds
-        this program's conductance terms (same kernel codes object and version, seed).
+    @property
+    def _terms_source(self):
+        """(kernel codes, version, seed) of the conductance terms kept, or None."""
+        return self._kept.source
+
+    def _terms(self, arrays, device, codes_t):
+        """(buffer of this program's conductance terms kept across reads, whether it holds
+        them, what they are sampled from), under the lock of ``_kept``.
 
         Write variation, drift and stuck-at faults do not depend on the read event
         (memfast/reference.py:36-46), so those samples are identical on every read
         of a programmed matrix and need not be drawn again."""
-        need = hip.mm_workspace_bytes(self.config, rows, arrays, self.p, variant)
-        workspace = self._workspace
-        if workspace is None or workspace.numel() < need or workspace.device != device:
-            workspace = torch.empty(max(1, need), dtype=torch.uint8, device=device)
-            self._workspace, self._terms_source = workspace, None
         source = (codes_t, codes_t._version, self.seed)
-        held = self._terms_source
-        reuse = held is not None and held[0] is codes_t and held[1:] == source[1:]
-        self._terms_source = None     # set again once the call has been queued
-        return workspace, reuse, source
+        need = hip.mm_terms_bytes(self.config, arrays, self.p)
+        return *self._kept.take(need, device, source), source
 
     def _execute_stable(self, q, xscale, packed, event):
         """FP64 overflow-safe restore of the slice totals (non-finite FP32 retry).
