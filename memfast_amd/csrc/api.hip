@@ -459,22 +459,31 @@ bool pairs_read(const mf_config *cfg, i64 n, i64 m, i64 p) {
 // Waves per workgroup of k_noisy_block: 32 columns each, four where there are as many.
 int block_waves(i64 cols) { return cols > 96 ? 4 : int((cols + 31) / 32); }
 
-// Read chunks of k_noisy_block.  A tile's read (32 x 32 outputs of one read, one wave) takes one
-// unit of a SIMD's time where another wave fills its gaps and 1.6 units alone, so a chunk of s
-// reads takes s * max(1.6, waves per SIMD).  Splitting writes and reads back 8 bytes per output
-// and read: 2e-4 units per tile for eight by eight slices of 64 rows (10 us), more for less work.
-i64 block_split(const mf_config *cfg, i64 n, i64 G, i64 cols) {
+// 32 x 32 tiles of n vectors by cols columns.
+i64 block_tiles(i64 n, i64 cols) { return (cols + 31) / 32 * ((n + 31) / 32); }
+
+// What k_noisy_block takes for `tiles` split into z chunks of reads.  A tile's read (32 x 32 outputs
+// of one read, one wave) takes one unit of a SIMD's time where another wave fills its gaps and 1.6
+// units alone, so a chunk of s reads takes s * max(1.6, waves per SIMD).  Splitting writes and reads
+// back 8 bytes per output and read: 2e-4 units per tile for eight by eight slices of 64 rows
+// (10 us), more for less work.
+double block_cost(const mf_config *cfg, i64 tiles, i64 G, i64 z) {
     constexpr i64 SIMDS = 1024;
-    const i64 tiles = (cols + 31) / 32 * ((n + 31) / 32);
+    const double waves = double((tiles * z + SIMDS - 1) / SIMDS);
     const double traffic = 2e-4 * double(tiles) * double(G) * 256.0 /
                            (double(cfg->n_in) * cfg->n_w * (cfg->read_rows / 16));
+    return double((G + z - 1) / z) * std::max(1.6, waves) + (z > 1 ? traffic : 0.0);
+}
+
+// The number of chunks of least cost: of those with the same reads per chunk, the fewest.
+i64 block_chunks(const mf_config *cfg, i64 tiles, i64 G) {
     i64 best = 1;
-    double least = 0.0;
-    for (i64 z = 1; z <= G; ++z) {
-        const double waves = double((tiles * z + SIMDS - 1) / SIMDS);
-        const double cost =
-            double((G + z - 1) / z) * std::max(1.6, waves) + (z > 1 ? traffic : 0.0);
-        if (z == 1 || cost < least) {
+    double least = block_cost(cfg, tiles, G, 1);
+    for (i64 step = G; step > 1;) {
+        const i64 z = (G + step - 2) / (step - 1);   // the fewest chunks of step - 1 reads
+        step = (G + z - 1) / z;
+        const double cost = block_cost(cfg, tiles, G, z);
+        if (cost < least) {
             least = cost;
             best = z;
         }
@@ -482,30 +491,61 @@ i64 block_split(const mf_config *cfg, i64 n, i64 G, i64 cols) {
     return best;
 }
 
-// Read chunks of a split read (1: not split).  `requested` (the variant's
-// split field) overrides the automatic choice: 1 never splits, s >= 2 splits
-// into s chunks (at most one per read).
-i64 noisy_split(const mf_config *cfg, i64 n, i64 m, i64 p, int requested = 0) {
-    const i64 G = m * cfg->reads;
+// How a noisy read is split: z chunks of reads (1: not split), passes of `rows` vectors by `cols`
+// columns.
+struct NoisySplit {
+    i64 z, rows, cols;
+};
+
+// Passes of a split block read: its totals are one FP32 per output and read, however many chunks,
+// so a pass takes as many outputs as 1 GiB holds (a Simulator's default workspace budget).  That
+// is 256 (tile, read) units per SIMD and 65536 sums or more, so passes do not idle the chip: 2048 x
+// 11008 -> 1088 takes 5.28 ms in two, 5.22 with 1.5 GiB at once (at 256 MiB, 100 x 200000 -> 640 took
+// 6.7 ms instead of 4.5, its sums over 3125 reads short of threads).
+NoisySplit block_passes(i64 n, i64 G, i64 ncols) {
+    const i64 most = (i64(1) << 30) / 4 / G;   // outputs; G < 4096
+    if (n * ncols <= most) return {1, n, ncols};
+    const i64 fit = std::max<i64>(1, most / ncols / 32) * 32;   // vectors in multiples of 32
+    const i64 passes = (n + fit - 1) / fit;
+    const i64 rows = ((n + passes - 1) / passes + 31) / 32 * 32;
+    const i64 taken = std::min(rows, n);
+    if (taken * ncols <= most) return {1, taken, ncols};
+    return {1, taken, std::max<i64>(64, most / taken / 64 * 64)};
+}
+
+// The split of a noisy read.  `requested` (the variant's split field) overrides the automatic
+// choice of chunks: 1 never splits, s >= 2 splits into s chunks (at most one per read).
+NoisySplit noisy_split(const mf_config *cfg, i64 n, i64 m, i64 p, int requested = 0) {
+    const i64 G = m * cfg->reads, ncols = p * cfg->cols;
+    NoisySplit split{1, n, ncols};
+    if (requested == 1 || G < 2) return split;
+    if (block_read(cfg)) split = block_passes(n, G, ncols);
     i64 z;
     if (requested > 0) {
         z = requested;
+    } else if (block_read(cfg) && pairs_read(cfg, n, m, p)) {
+        z = G;
     } else if (block_read(cfg)) {
-        z = pairs_read(cfg, n, m, p) ? G : block_split(cfg, n, G, p * cfg->cols);
+        const i64 tiles = block_tiles(split.rows, split.cols);
+        const i64 passes = ((n + split.rows - 1) / split.rows) * ((ncols + split.cols - 1) / split.cols);
+        z = block_chunks(cfg, tiles, G);
+        if (passes > 1 && double(passes) * block_cost(cfg, tiles, G, z) >=
+                              block_cost(cfg, block_tiles(n, ncols), G, 1))
+            z = 1;
     } else {
-        const i64 blocks = (p * cfg->cols + 63) / 64 * ((n + 63) / 64);
-        if (G < 2 || blocks >= NOISY_SPLIT_BELOW) return 1;
-        z = (NOISY_SPLIT_BELOW + blocks - 1) / blocks;
+        const i64 blocks = (ncols + 63) / 64 * ((n + 63) / 64);
+        z = blocks >= NOISY_SPLIT_BELOW ? 1 : (NOISY_SPLIT_BELOW + blocks - 1) / blocks;
     }
     if (z > G) z = G;
-    if (z < 2) return 1;
+    if (z < 2) return {1, n, ncols};
     const i64 step = (G + z - 1) / z;
-    return (G + step - 1) / step;
+    split.z = (G + step - 1) / step;
+    return split;
 }
 
-i64 noisy_scratch_bytes(const mf_config *cfg, i64 n, i64 m, i64 p, int requested = 0) {
-    if (noisy_split(cfg, n, m, p, requested) < 2) return 0;
-    return align256(n * m * cfg->reads * p * cfg->cols * 4);
+// Totals of a split read (one pass of it).
+i64 noisy_scratch_bytes(const mf_config *cfg, const NoisySplit &split, i64 m) {
+    return split.z < 2 ? 0 : align256(split.rows * m * cfg->reads * split.cols * 4);
 }
 
 // Operand terms per input value with voltage variation: x hi and lo, and with output-mode
@@ -572,22 +612,26 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
     }
     const i64 per_block = noisy_block_bytes(cfg, m);
     // Split read (fused output only, when the whole program's terms fit).
-    const i64 split = totals ? 1 : noisy_split(cfg, n, m, p, split_request);
+    const NoisySplit split = totals ? NoisySplit{1, n, ncols}
+                                    : noisy_split(cfg, n, m, p, split_request);
     const i64 full = noisy_terms_bytes(cfg, m, p);
-    const i64 scratch = noisy_scratch_bytes(cfg, n, m, p, split_request);
+    const i64 scratch = noisy_scratch_bytes(cfg, split, m);
     const i64 held = terms ? 0 : full;   // bytes of the workspace that the terms take
-    const bool use_split = split > 1 && bytes >= held + scratch;
-    if (split > 1 && split_request > 1 && !use_split)
+    const bool use_split = split.z > 1 && bytes >= held + scratch;
+    if (split.z > 1 && split_request > 1 && !use_split)
         return fail(MF_E_RESOURCE,
                     "workspace of %lld bytes below the %lld a %lld-way read split needs",
                     static_cast<long long>(bytes), static_cast<long long>(held + scratch),
-                    static_cast<long long>(split));
+                    static_cast<long long>(split.z));
     const i64 max_cb = use_split || terms ? full / per_block : (bytes / per_block) / 2 * 2;
     if (max_cb < 2) return fail(MF_E_RESOURCE, "workspace below one 64-column chunk");
     reuse = reuse && g == nullptr && terms_event_independent(cfg) && max_cb * 32 >= ocols;
     uint4 *gs = static_cast<uint4 *>(terms ? terms : workspace);
     float *partial = use_split ? reinterpret_cast<float *>(static_cast<char *>(workspace) + held)
                                : nullptr;
+    const bool one_pass = split.rows >= n && split.cols >= ncols;
+    // A small split read runs k_noisy_pairs: one read per workgroup, one wave per weight slice.
+    const bool pairs = use_split && pairs_read(cfg, n, m, p);
     for (i64 c_begin = 0; c_begin < ocols; c_begin += max_cb * 32) {
         const i64 cols = (ocols - c_begin) < max_cb * 32 ? (ocols - c_begin) : max_cb * 32;
         const i64 CB = (cols + 63) / 64 * 2;
@@ -620,6 +664,7 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
         args.ncols = ocols;
         args.c_begin = c_begin;
         args.CB = CB;
+        args.blocks = CB;
         args.totals = totals;
         args.g_begin = 0;
         args.g_end = g_run;
@@ -631,78 +676,100 @@ int launch_noisy(const mf_config *cfg, const NoisyPlan &plan, int ks, const u8 *
         if (use_split) {
             args.totals = 1;
             args.out = partial;
-            args.ldo = ncols;
-            args.g_step = (g_run + split - 1) / split;
+            args.ldo = split.cols;
+            args.g_step = (g_run + split.z - 1) / split.z;
             gz = unsigned((g_run + args.g_step - 1) / args.g_step);
         }
         const bool nl = cfg->has_nonlinear != 0;
         const bool slice = plan.planes > 1 && !plan.out_noise;
-        // A small split read runs k_noisy_pairs: one read per workgroup, one wave per weight
-        // slice.
-        const bool pairs = use_split && pairs_read(cfg, n, m, p);
-        const bool wide_block = block_read(cfg) && !pairs;
-        const int waves = block_waves(cols);
-        const dim3 grid = pairs ? dim3{unsigned(CB), unsigned((n + 31) / 32), unsigned(g_run)}
-                          : wide_block ? dim3{unsigned((n + 31) / 32),
-                                              unsigned((cols + 32 * waves - 1) / (32 * waves)), gz}
-                                       : dim3{unsigned((n + 63) / 64), unsigned(CB / 2), gz};
-        const dim3 block{pairs ? unsigned(64 * cfg->n_w) : wide_block ? unsigned(64 * waves) : 256u};
         if (pairs) {
             args.g_step = 1;
             args.restored = 1;   // the values (float(T) * xs) * ws; consumers only sum them
         }
-        // Benchmark timing brackets the read kernel alone (not the conductance split).
-        std::pair<hipEvent_t, hipEvent_t> timing{nullptr, nullptr};
-        if (profiling() && (timing = profile_pair()).first) hipEventRecord(timing.first, s);
+        // One pass (NoisySplit) of the read: args.n vectors by `columns`.
+        auto launch = [&](i64 columns) {
+            const i64 vectors = args.n;
+            const int waves = block_waves(columns);
+            const dim3 grid =
+                pairs ? dim3{unsigned(args.blocks), unsigned((vectors + 31) / 32), unsigned(g_run)}
+                : block_read(cfg) ? dim3{unsigned((vectors + 31) / 32),
+                                         unsigned((columns + 32 * waves - 1) / (32 * waves)), gz}
+                                  : dim3{unsigned((vectors + 63) / 64), unsigned(args.blocks / 2), gz};
+            const dim3 block{pairs ? unsigned(64 * cfg->n_w)
+                                   : block_read(cfg) ? unsigned(64 * waves) : 256u};
+            // Benchmark timing brackets the read kernel alone (not the conductance split).
+            std::pair<hipEvent_t, hipEvent_t> timing{nullptr, nullptr};
+            if (profiling() && (timing = profile_pair()).first) hipEventRecord(timing.first, s);
 #define MF_NOISY_LAUNCH1(KS, NA, NL, VN, SL, ON) \
-    hipLaunchKernelGGL((k_noisy<KS, NA, NL, VN, SL, ON>), grid, block, 0, s, plan, args)
+        hipLaunchKernelGGL((k_noisy<KS, NA, NL, VN, SL, ON>), grid, block, 0, s, plan, args)
 #define MF_NOISY_LAUNCH2(KS, NA, VN, SL, ON)                    \
-    {                                                          \
-        if (nl) MF_NOISY_LAUNCH1(KS, NA, true, VN, SL, ON);    \
-        else MF_NOISY_LAUNCH1(KS, NA, false, VN, SL, ON);      \
-    }
-#define MF_NOISY_LAUNCH(KS, NA)                                                                \
-    {                                                                                         \
-        if (pairs && nl)                                                                      \
-            hipLaunchKernelGGL((k_noisy_pairs<KS, NA, true>), grid, block, 0, s, plan, args);  \
-        else if (pairs)                                                                       \
-            hipLaunchKernelGGL((k_noisy_pairs<KS, NA, false>), grid, block, 0, s, plan, args); \
-        else if (plan.out_noise && volt) MF_NOISY_LAUNCH2(KS, NA, true, false, true)          \
-        else if (plan.out_noise) MF_NOISY_LAUNCH2(KS, NA, false, false, true)                 \
-        else if (volt && slice) MF_NOISY_LAUNCH2(KS, NA, true, true, false)                   \
-        else if (volt) MF_NOISY_LAUNCH2(KS, NA, true, false, false)                           \
-        else if (slice) MF_NOISY_LAUNCH2(KS, NA, false, true, false)                          \
-        else MF_NOISY_LAUNCH2(KS, NA, false, false, false)                                    \
-    }
-#define MF_BLOCK_LAUNCH(KS)                                                                     \
-    if (pairs) hipLaunchKernelGGL((k_noisy_pairs<KS, 8, false>), grid, block, 0, s, plan, args); \
-    else hipLaunchKernelGGL(k_noisy_block<KS>, grid, block, unsigned(cfg->n_in * KS * 1024), s,   \
-                            plan, args)
-        if (block_read(cfg)) {
-            if (ks == 8) { MF_BLOCK_LAUNCH(8); }
-            else { MF_BLOCK_LAUNCH(4); }
+        {                                                          \
+            if (nl) MF_NOISY_LAUNCH1(KS, NA, true, VN, SL, ON);    \
+            else MF_NOISY_LAUNCH1(KS, NA, false, VN, SL, ON);      \
         }
-        else if (ks == 4) MF_NOISY_LAUNCH(4, 5)
-        else if (cfg->n_in <= 5) MF_NOISY_LAUNCH(2, 5)
-        else MF_NOISY_LAUNCH(2, 8)
+#define MF_NOISY_LAUNCH(KS, NA)                                                                \
+        {                                                                                         \
+            if (pairs && nl)                                                                      \
+                hipLaunchKernelGGL((k_noisy_pairs<KS, NA, true>), grid, block, 0, s, plan, args);  \
+            else if (pairs)                                                                       \
+                hipLaunchKernelGGL((k_noisy_pairs<KS, NA, false>), grid, block, 0, s, plan, args); \
+            else if (plan.out_noise && volt) MF_NOISY_LAUNCH2(KS, NA, true, false, true)          \
+            else if (plan.out_noise) MF_NOISY_LAUNCH2(KS, NA, false, false, true)                 \
+            else if (volt && slice) MF_NOISY_LAUNCH2(KS, NA, true, true, false)                   \
+            else if (volt) MF_NOISY_LAUNCH2(KS, NA, true, false, false)                           \
+            else if (slice) MF_NOISY_LAUNCH2(KS, NA, false, true, false)                          \
+            else MF_NOISY_LAUNCH2(KS, NA, false, false, false)                                    \
+        }
+#define MF_BLOCK_LAUNCH(KS)                                                                     \
+        if (pairs) hipLaunchKernelGGL((k_noisy_pairs<KS, 8, false>), grid, block, 0, s, plan, args); \
+        else hipLaunchKernelGGL(k_noisy_block<KS>, grid, block, unsigned(cfg->n_in * KS * 1024), s,   \
+                                plan, args)
+            if (block_read(cfg)) {
+                if (ks == 8) { MF_BLOCK_LAUNCH(8); }
+                else { MF_BLOCK_LAUNCH(4); }
+            }
+            else if (ks == 4) MF_NOISY_LAUNCH(4, 5)
+            else if (cfg->n_in <= 5) MF_NOISY_LAUNCH(2, 5)
+            else MF_NOISY_LAUNCH(2, 8)
 #undef MF_BLOCK_LAUNCH
 #undef MF_NOISY_LAUNCH
 #undef MF_NOISY_LAUNCH2
 #undef MF_NOISY_LAUNCH1
-        if (timing.first) {
-            hipEventRecord(timing.second, s);
-            profile_push(timing);
+            if (timing.first) {
+                hipEventRecord(timing.second, s);
+                profile_push(timing);
+            }
+        };
+        if (!use_split || one_pass) {
+            launch(cols);
+            continue;
         }
+        for (i64 v0 = 0; v0 < n; v0 += split.rows)
+            for (i64 c0 = 0; c0 < ocols; c0 += split.cols) {   // (a split read's c_begin is 0)
+                const i64 pass_cols = std::min(split.cols, ocols - c0);
+                args.n = std::min(split.rows, n - v0);
+                args.blocks = (pass_cols + 63) / 64 * 2;
+                args.q = q + v0 * kp;
+                args.xscale = xscale + v0 * G;
+                args.gs = gs + c0 / 32 * G * NOISY_TERMS * ks * 64;
+                args.c_begin = c0;
+                args.ncols = c0 + pass_cols;
+                args.out = partial - c0;   // (columns are absolute)
+                launch(pass_cols);
+                hipLaunchKernelGGL(k_restore_sum_f32, dim3(grid_for(args.n * pass_cols)), dim3(256),
+                                   0, s, partial, args.n, G, g_run, split.cols, pass_cols,
+                                   args.xscale, wscale + c0, ncols, out + v0 * ldo + c0, ldo,
+                                   level_power(G), int(pairs), status);
+            }
     }
-    // With split_totals the caller restores and sums a split read's totals [n, G, ncols]
-    // itself (null when the read wrote `out`).
-    const bool restored = use_split && pairs_read(cfg, n, m, p);   // k_noisy_pairs restored
-    if (split_totals) *split_totals = use_split ? partial : nullptr;
-    if (split_restored) *split_restored = restored;
-    if (use_split && !split_totals)
+    // With split_totals the caller restores and sums the totals [n, G, ncols] of a read split in
+    // one pass itself (null when the read wrote `out`).
+    if (split_totals) *split_totals = use_split && one_pass ? partial : nullptr;
+    if (split_restored) *split_restored = pairs;   // k_noisy_pairs restored
+    if (use_split && one_pass && !split_totals)
         hipLaunchKernelGGL(k_restore_sum_f32, dim3(grid_for(n * ocols)), dim3(256), 0, s, partial, n,
                            G, g_run, ncols, ocols, xscale, wscale, ncols, out, ldo, level_power(G),
-                           int(restored), status);
+                           int(pairs), status);
     return check_launch("noisy MFMA read");
 }
 
@@ -1691,7 +1758,7 @@ int mf_mm_workspace(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32
         *bytes = xb + wb;
     } else if (build_noisy_plan(cfg, m, p, &noisy, &ks, &why)) {
         *bytes = noisy_terms_bytes(cfg, m, p) +
-                 noisy_scratch_bytes(cfg, n, m, p, variant_split(variant)) +
+                 noisy_scratch_bytes(cfg, noisy_split(cfg, n, m, p, variant_split(variant)), m) +
                  noisy_voltage_bytes(cfg, n, m);
     } else if (wide_plan_ok(cfg, n, m, p)) {
         // At least the two 32-column blocks the wide read's chunking needs, even for

@@ -201,6 +201,7 @@ struct NoisyArgs {
     float *out;           // fused: [n, ldo]; totals: [n, G, ldo]
     u32 *status;          // optional: MF_STATUS_OUTPUT for a non-finite fused output
     i64 n, kp, G, ldo, ldws, ncols, c_begin, CB;
+    i64 blocks;           // 32-column blocks of this launch, from c_begin on (at most CB)
     i64 g_begin, g_end;   // reads of this launch (blockIdx.z adds g_step)
     i64 g_step;
     int totals;

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256, 2) void k_noisy_block(const NoisyPlan plan,
     const i64 vrows = (args.n - v0) < 32 ? (args.n - v0) : 32;
     const __amdgpu_buffer_rsrc_t qbuf = noisy_buffer(args.q + v0 * kp, vrows * kp);
     const int q_off = lrow * int(kp) + lhalf * 8;
-    const bool live = c0 < args.CB * 32;   // the last workgroup may hold waves past the chunk
+    const bool live = c0 < args.blocks * 32;   // the last workgroup may hold waves past these
     const i64 col_tile = args.c_begin + c0;
     const i64 n_out = v0 + lrow;
     const i64 w_stride = args.CB * i64(G) * NOISY_TERMS * KS * 64;

@@ -97,6 +97,29 @@ def test_read_order_levels(hip_device, name, reads):
     assert torch.equal(fused.view(torch.int32), split.view(torch.int32))
 
 
+@pytest.mark.parametrize("name,n,reads,o", [
+    ("default", 700, 700, 600),          # passes of vectors
+    ("int4_faults", 45, 3300, 2600),     # and of columns, the last of 13 vectors and 104 columns
+    ("default", 32, 3300, 2600),         # one vector block on k_noisy_pairs
+])
+def test_splits_in_passes(hip_device, name, n, reads, o):
+    """A split read whose totals exceed 1 GiB runs in passes; each output is the unsplit read's."""
+    cfg = case(name)
+    gen = torch.Generator(device=hip_device).manual_seed(7)
+    k = reads * cfg.read_rows - 3
+    a = torch.randn(n, k, generator=gen, device=hip_device)
+    w = torch.randn(o, k, generator=gen, device=hip_device)
+    q, xs = hip.input_tiles(a, cfg)
+    packed, packed_t, ws = hip.weight_tiles(w, cfg)
+    p = packed.shape[1]
+    assert 4 * n * reads * p * cfg.array_size[1] > 1 << 30
+    outputs = [hip.mm(q, xs, packed, packed_t, ws.reshape(-1, p * cfg.array_size[1]), cfg, 11, 0,
+                      out_cols=o, k_rows=k, variant=hip.variant_word(split=z))[:, :o]
+               for z in (1, 0, 3)]
+    for output in outputs[1:]:
+        assert torch.equal(output.view(torch.int32), outputs[0].view(torch.int32))
+
+
 def test_tuned_read_without_samples_beyond_its_budget(hip_device, tmp_path):
     """Ideal devices need no sampled conductances: where the block read's terms exceed a tuned
     simulator's workspace budget, the general kernel reads the same counts."""

@@ -81,6 +81,22 @@ def test_workspace_need_prices_each_schedule():
     assert tuning.workspace_need(output, n, m, p, dict(split=1)) == 2 * terms + 4 * 5 * n * m * 128 * 2
 
 
+@pytest.mark.parametrize("n,k,o", [(2048, 4096, 1056), (512, 11008, 2240), (2048, 11008, 1088),
+                                   (256, 4096, 4096), (32, 262016, 4096), (33, 262016, 16384)])
+def test_split_totals_of_default_arrays_are_bounded(n, k, o):
+    """Reads of 64-row arrays with eight slices take their split in passes of at most 1 GiB of
+    totals, whatever the batch and the schedule's chunks."""
+    cfg = Config(nonidealities=Nonidealities(write_variation=0.02))
+    m, p = -(-k // 64), -(-o // 64)
+    terms = hip.mm_terms_bytes(cfg, m, p)
+    assert hip.block_read(cfg) and terms == 32 * m * 64 * p * 64
+    for split in (0, 1, 2, 15):
+        totals = hip.mm_workspace_bytes(cfg, n, m, p, hip.variant_word(split=split)) - terms
+        assert totals == 0 if split == 1 else 0 <= totals <= 1 << 30
+        if n * m * p * 64 * 4 <= 1 << 30 and split > 1:
+            assert totals == n * m * p * 64 * 4
+
+
 def test_unknown_variant_bits_are_refused():
     import ctypes as ct
 
