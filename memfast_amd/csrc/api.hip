@@ -1920,7 +1920,9 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
                                 variant_split(variant), split_totals, split_restored, terms);
     }
     if (!g && needs_conductances(cfg))
-        return fail(MF_E_INVALID, "device noise needs restored conductances (g)");
+        return fail(MF_E_INVALID, "device noise needs restored conductances (g)%s",
+                    aligned ? "" : ": the MFMA read that samples them takes 16-byte aligned q, "
+                                   "packed_t and out, and ldo in multiples of 4");
     GeneralArgs args{};
     args.q = q;
     args.packed = packed;

@@ -841,6 +841,13 @@ def terms_event_independent(config):
     return not config.nonidealities.read_variation
 
 
+def _mfma_aligned(q, packed_t, out):
+    """Whether the MFMA reads take these operands (the checks of mf_mm): 16-byte aligned codes
+    and output, output rows in multiples of 16 bytes."""
+    return ((q.data_ptr() | packed_t.data_ptr() | out.data_ptr()) % 16 == 0
+            and out.stride(0) % 4 == 0)
+
+
 def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=None, out=None,
        variant=0, status=None, workspace=None, terms=None, reuse_terms=False, out_cols=None,
        k_rows=None, split_budget=None):
@@ -869,6 +876,16 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
         raise ValueError("out_cols must be in [1, p*C]")
     if k_rows is not None and not 1 <= k_rows <= m * r:
         raise ValueError("k_rows must be in [1, m*R]")
+    if out is None:
+        out = torch.empty((n, p * c), dtype=torch.float32, device=q.device)
+    # Converted operands stay referenced until the launch is queued (a freed
+    # temporary could be handed to the next conversion by the caching allocator).
+    q, xscale = q.contiguous(), xscale.contiguous()
+    packed, wscale = packed.contiguous(), wscale.contiguous()
+    if packed_t is not None and not _mfma_aligned(q, packed_t, out):
+        if terms is not None:
+            raise ValueError("mm keeps terms for aligned operands only")
+        packed_t = None   # the general kernel takes any alignment
     g = conductance
     kernel = mm_kernel(config, n, m, p) if g is None and packed_t is not None else 0
     if g is None and kernel == 0 and needs_conductances(config):
@@ -876,8 +893,6 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
     if g is not None:
         g = _checked_conductance(g, config, m, p, r, c)
         packed_t = None
-    if out is None:
-        out = torch.empty((n, p * c), dtype=torch.float32, device=q.device)
     if packed_t is None or kernel != 2:
         terms = None
     if packed_t is not None and kernel:
@@ -897,10 +912,6 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
         size = mm_workspace_bytes(config, n, m, p, 0) if mm_kernel(config, n, m, p) == 0 else 0
         fits = size and (split_budget is None or size <= split_budget)
         workspace = torch.empty(size, dtype=torch.uint8, device=q.device) if fits else None
-    # Converted operands stay referenced until the launch is queued (a freed
-    # temporary could be handed to the next conversion by the caching allocator).
-    q, xscale = q.contiguous(), xscale.contiguous()
-    packed, wscale = packed.contiguous(), wscale.contiguous()
     lib = library()
     operands = (ct.byref(descriptor(config)), _ptr(q), _ptr(xscale), n, m, _ptr(packed),
                 _ptr(packed_t), _ptr(wscale), p, p * c if out_cols is None else out_cols,

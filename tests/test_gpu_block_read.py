@@ -77,6 +77,28 @@ def test_product_and_schedules(hip_device, name, n, k, o):
     check_product(cfg, got, a, b, hip_device, label=f"block read {name}")
 
 
+SLICED = Config(input_slice=(1, 1, 2, 2, 2), weight_slice=(1, 1, 2, 2, 2), array_size=(128, 128),
+                rows_per_read=32, adc_bits=7, nonidealities=Nonidealities(**WRITE))
+
+
+@pytest.mark.parametrize("cfg", [case("default"), case("rows128"), case("rows128_ideal"), SLICED],
+                         ids=["default", "rows128", "rows128_ideal", "sliced"])
+@pytest.mark.parametrize("offset,stride", [(0, 131), (1, 132), (2, 130)])
+def test_unaligned_output(hip_device, cfg, offset, stride):
+    """An output view that the MFMA reads do not take (row stride, first element) gets the general
+    kernel's read: the output for the conductances restored and passed in."""
+    n, k, o = 33, 200, 128
+    *_, q, xs, packed, packed_t, ws = programmed(cfg, n, k, o, hip_device, 9)
+    g = hip.restore(packed, cfg, 5, 2, 0, packed.shape[1])
+    expected = hip.mm(q, xs, packed, None, ws, cfg, 5, 2, conductance=g, k_rows=k)
+    flat = torch.full((n * stride + 4,), float("nan"), device=hip_device)
+    view = flat[offset:offset + n * stride].view(n, stride)
+    got = hip.mm(q, xs, packed, packed_t, ws, cfg, 5, 2, out=view, k_rows=k)
+    assert got is view
+    assert torch.equal(got[:, :o].contiguous().view(torch.int32), expected.view(torch.int32))
+    assert bool(got[:, o:].isnan().all()) and bool(flat[:offset].isnan().all())
+
+
 def test_reads_between_counts_keep_the_general_kernel():
     """Read noise, drift, nonlinear converters and voltage noise put converter arguments
     anywhere between two counts."""
