@@ -1711,6 +1711,20 @@ static bool ideal_extent_ok(const mf_config *cfg, i64 n, i64 m, i64 p) {
            (n + 63) / 64 + (ncols + 31) / 32 <= 65535;
 }
 
+// Whether a shape runs the ideal or the noisy MFMA read: its extents and its plan.
+static bool ideal_applies(const mf_config *cfg, i64 n, i64 m, i64 p, IdealPlan *plan, SlotTests *xt,
+                          SlotTests *wt, int *ks) {
+    const char *why = "";
+    return ideal_extent_ok(cfg, n, m, p) && build_ideal_plan(cfg, m, p, plan, xt, wt, ks, &why);
+}
+
+static bool noisy_applies(const mf_config *cfg, i64 n, i64 m, i64 p, NoisyPlan *plan, int *ks,
+                          const char **why) {
+    *why = "extents beyond 32-bit offsets or the grid";
+    return ideal_extent_ok(cfg, n, m, p) && noisy_extent_ok(n, m, cfg) &&
+           build_noisy_plan(cfg, m, p, plan, ks, why);
+}
+
 static bool wide_plan_ok(const mf_config *cfg, i64 n, i64 m, i64 p) {
     NoisyWidePlan plan;
     int ks = 0;
@@ -1728,11 +1742,9 @@ int mf_mm_kernel(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32_t 
     int ks = 0;
     const char *why = "";
     NoisyPlan noisy;
-    if (has_packed_t && ideal_extent_ok(cfg, n, m, p) &&
-        build_ideal_plan(cfg, m, p, &plan, &xt, &wt, &ks, &why))
+    if (has_packed_t && ideal_applies(cfg, n, m, p, &plan, &xt, &wt, &ks))
         *kernel_id = 1;
-    else if (has_packed_t && noisy_extent_ok(n, m, cfg) &&
-             build_noisy_plan(cfg, m, p, &noisy, &ks, &why))
+    else if (has_packed_t && noisy_applies(cfg, n, m, p, &noisy, &ks, &why))
         *kernel_id = 2;
     else if (wide_plan_ok(cfg, n, m, p))
         *kernel_id = 3;
@@ -1752,11 +1764,11 @@ int mf_mm_workspace(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32
     NoisyPlan noisy;
     int ks = 0;
     const char *why = "";
-    if (build_ideal_plan(cfg, m, p, &plan, &xt, &wt, &ks, &why)) {
+    if (ideal_applies(cfg, n, m, p, &plan, &xt, &wt, &ks)) {
         i64 xb, wb;
         ideal_workspace(cfg, n, m, p, &xb, &wb);
         *bytes = xb + wb;
-    } else if (build_noisy_plan(cfg, m, p, &noisy, &ks, &why)) {
+    } else if (noisy_applies(cfg, n, m, p, &noisy, &ks, &why)) {
         *bytes = noisy_terms_bytes(cfg, m, p) +
                  noisy_scratch_bytes(cfg, noisy_split(cfg, n, m, p, variant_split(variant)), m) +
                  noisy_voltage_bytes(cfg, n, m);
@@ -1878,8 +1890,8 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
     ideal_workspace(cfg, n, m, p, &xbytes, &wbytes);
     const bool room = workspace && workspace_bytes >= xbytes + wbytes;
     SlotTests xtests, wtests;
-    if (!g && packed_t && aligned && room && ideal_extent_ok(cfg, n, m, p) &&
-        build_ideal_plan(cfg, m, p, &plan, &xtests, &wtests, &ks, &why)) {
+    if (!g && packed_t && aligned && room &&
+        ideal_applies(cfg, n, m, p, &plan, &xtests, &wtests, &ks)) {
         uint64_t *xbits = static_cast<uint64_t *>(workspace);
         uint64_t *wbits = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + xbytes);
         const i64 kp = m * cfg->rows, ncols = p * cfg->cols;
@@ -1905,8 +1917,8 @@ static int mm_read(const mf_config *cfg, const uint8_t *q, const float *xscale, 
                             out_cols, g_run, out, ldo, variant, status, s);
     }
     NoisyPlan noisy;
-    if (!g && packed_t && aligned && (workspace || terms) && ideal_extent_ok(cfg, n, m, p) &&
-        noisy_extent_ok(n, m, cfg) && build_noisy_plan(cfg, m, p, &noisy, &ks, &why)) {
+    if (!g && packed_t && aligned && (workspace || terms) &&
+        noisy_applies(cfg, n, m, p, &noisy, &ks, &why)) {
         const i64 full = noisy_terms_bytes(cfg, m, p);
         if (terms && (terms_bytes < full || reinterpret_cast<uintptr_t>(terms) % 256))
             return fail(MF_E_INVALID, "kept terms need %lld bytes, 256-byte aligned",
@@ -2018,10 +2030,9 @@ int mf_mm_from_float(const mf_config *cfg, const float *x, int64_t n, int64_t k,
     IdealPlan plan;
     SlotTests xtests, wtests;
     int ks = 0;
-    const char *why = "";
     const i64 wgrid_x = o / 64, wblocks = wgrid_x * (m * R / 128), xblocks = (n + 63) / 64 * (G / 4);
-    if (!shapes || !aligned || !room || !ideal_extent_ok(cfg, n, m, p) ||
-        wblocks + xblocks > 0x7FFFFFFF || !build_ideal_plan(cfg, m, p, &plan, &xtests, &wtests, &ks, &why))
+    if (!shapes || !aligned || !room || wblocks + xblocks > 0x7FFFFFFF ||
+        !ideal_applies(cfg, n, m, p, &plan, &xtests, &wtests, &ks))
         return fail(MF_E_UNSUPPORTED, "mm_from_float not applicable");
     u32 *device_mailbox = nullptr;
     if (mailbox) {
@@ -2172,12 +2183,12 @@ int mf_mm_static(const mf_config *cfg, const uint8_t *q, const float *xscale, in
     NoisyPlan noisy;
     int ks = 0;
     const char *why = "";
-    if (!g && packed_t && build_ideal_plan(cfg, m, p, &plan, &xt, &wt, &ks, &why)) {
+    if (!g && packed_t && ideal_applies(cfg, n, m, p, &plan, &xt, &wt, &ks)) {
         i64 xb = 0, wb = 0;
         ideal_workspace(cfg, n, m, p, &xb, &wb);
         need = xb + wb;
         what = "digit masks of the ideal-device read";
-    } else if (!g && packed_t && build_noisy_plan(cfg, m, p, &noisy, &ks, &why)) {
+    } else if (!g && packed_t && noisy_applies(cfg, n, m, p, &noisy, &ks, &why)) {
         need = noisy_voltage_bytes(cfg, n, m) + 2 * noisy_block_bytes(cfg, m);
         what = cfg->has_vnoise ? "voltage-noise operands and one 64-column chunk of noisy "
                                  "conductance terms"
@@ -2222,8 +2233,7 @@ int mf_mm_totals(const mf_config *cfg, const uint8_t *q, int64_t n, int64_t m,
     NoisyPlan noisy;
     int ks = 0;
     const char *why = "";
-    if (!ideal_extent_ok(cfg, n, m, p) || !noisy_extent_ok(n, m, cfg) ||
-        !build_noisy_plan(cfg, m, p, &noisy, &ks, &why))
+    if (!noisy_applies(cfg, n, m, p, &noisy, &ks, &why))
         return fail(MF_E_UNSUPPORTED, "noisy MFMA read not applicable: %s", why);
     const i64 ncols = p * cfg->cols;
     return launch_noisy(cfg, noisy, ks, q, nullptr, n, m, packed_t, nullptr, p, g, seed, event,

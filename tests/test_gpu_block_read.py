@@ -99,6 +99,25 @@ def test_unaligned_output(hip_device, cfg, offset, stride):
     assert bool(got[:, o:].isnan().all()) and bool(flat[:offset].isnan().all())
 
 
+@pytest.mark.parametrize("cfg", [case("default"), SLICED], ids=["default", "sliced"])
+def test_batch_beyond_the_mfma_reads(hip_device, cfg):
+    """4.2 million vectors are more than the MFMA reads' grids take: a layer's read samples the
+    conductances for the general kernel."""
+    k, o = cfg.array_size[0] - 1, 30
+    n = (65535 - cfg.array_size[1] // 32) * 64 + 1
+    gen = torch.Generator(device=hip_device).manual_seed(10)
+    x = torch.randn(n, k, generator=gen, device=hip_device)
+    layer = Simulator(cfg, device=hip_device).map(
+        torch.randn(o, k, generator=gen, device=hip_device), name="layer")
+    assert hip.mm_kernel(cfg, n, 1, 1) == 0
+    got = layer(x)
+    q, xs = hip.input_tiles(x[-65:], cfg)
+    g = hip.restore(layer.packed, cfg, layer.seed, 0, 0, 1)
+    expected = hip.mm(q, xs, layer.packed, None, layer.weight_scale.reshape(-1, layer.p * cfg.array_size[1]),
+                      cfg, layer.seed, 0, conductance=g, k_rows=k)[:, :o]
+    assert torch.equal(got[-65:].view(torch.int32), expected.contiguous().view(torch.int32))
+
+
 def test_reads_between_counts_keep_the_general_kernel():
     """Read noise, drift, nonlinear converters and voltage noise put converter arguments
     anywhere between two counts."""

@@ -97,6 +97,20 @@ def test_split_totals_of_default_arrays_are_bounded(n, k, o):
             assert totals == n * m * p * 64 * 4
 
 
+def test_kernel_choice_has_the_extents_of_the_reads():
+    """Batches beyond the MFMA reads' extents (4.2 million vectors of one array) are the general
+    kernel's, which then gets restored conductances, and take none of their workspace."""
+    configs = [Config(nonidealities=Nonidealities(write_variation=0.02)),
+               Config(**INT8, nonidealities=Nonidealities(write_variation=0.02)),
+               Config(**INT8, nonidealities=Nonidealities(write_variation=0.0))]
+    for cfg, kernel in zip(configs, (2, 2, 1)):
+        blocks = -(-cfg.array_size[1] // 32)
+        most = (65535 - blocks) * 64
+        assert hip.mm_kernel(cfg, most, 1, 1) == kernel
+        assert hip.mm_kernel(cfg, most + 1, 1, 1) == 0
+        assert hip.mm_workspace_bytes(cfg, most + 1, 1, 1) == 0
+
+
 def test_unknown_variant_bits_are_refused():
     import ctypes as ct
 
