@@ -2824,9 +2824,15 @@ int mf_profile_collect(int64_t *launches, double *milliseconds) {
 
 int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32_t variant,
                        mf_resources *out) {
+    return mf_resources_shape(cfg, kernel_id, n, 0, 0, variant, out);
+}
+
+int mf_resources_shape(const mf_config *cfg, int32_t kernel_id, int64_t n, int64_t m, int64_t p,
+                       int32_t variant, mf_resources *out) {
     int status = check_config(cfg);
     if (status) return status;
     if (!out) return fail(MF_E_INVALID, "resources output is NULL");
+    if (m < 0 || p < 0 || (m > 0) != (p > 0)) return fail(MF_E_INVALID, "invalid matrix extents");
     if (!variant_valid(variant)) return fail(MF_E_INVALID, "unknown kernel variant 0x%x", variant);
     // The instance of the read kernel that mf_mm (mf_mm_wide) launches for this descriptor
     // and schedule (`variant`), chosen as launch_ideal, launch_noisy, launch_noisy_wide and
@@ -2842,8 +2848,7 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
         else if (variant_tile(variant) == 1) fn = reinterpret_cast<const void *>(&k_ideal<2, 1>);
         else fn = reinterpret_cast<const void *>(&k_ideal<1, 1>);
     } else if (kernel_id == 2) {
-        // ks index 0: KS 2 with up to 5 slices, 1: KS 2 with 8, 2: KS 4.  The read split
-        // does not change the instance.
+        // ks index 0: KS 2 with up to 5 slices, 1: KS 2 with 8, 2: KS 4.
 #define MF_NOISY_FN(KS, NA, NL, VN, SL, ON) \
     reinterpret_cast<const void *>(&k_noisy<KS, NA, NL, VN, SL, ON>)
 #define MF_NOISY_ROW(KS, NA)                                                                      \
@@ -2869,10 +2874,12 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                      : reinterpret_cast<const void *>(&k_noisy_block<8>);
             dynamic_lds = cfg->n_in * (ks4 ? 4 : 8) * 1024;
         }
-        if (n > 0 && noisy_small_tile(cfg, n) && variant_split(variant) != 1) {
-            // A split read of at most 32 vectors (the automatic split applies below 512
-            // four-wave blocks, 32768 output columns): k_noisy_pairs, one wave per weight
-            // slice.
+        // A small split read runs k_noisy_pairs, one wave per weight slice (launch_noisy).  Without
+        // the matrix, batches of at most 32 vectors are taken as split.
+        const bool small = m > 0 ? n > 0 && pairs_read(cfg, n, m, p) &&
+                                       noisy_split(cfg, n, m, p, variant_split(variant)).z > 1
+                                 : n > 0 && noisy_small_tile(cfg, n) && variant_split(variant) != 1;
+        if (small) {
             const void *pairs[3][2] = {
                 {reinterpret_cast<const void *>(&k_noisy_pairs<2, 5, false>),
                  reinterpret_cast<const void *>(&k_noisy_pairs<2, 5, true>)},
@@ -2906,15 +2913,15 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                   : tier == 1 ? MF_WIDE_FN(2, WIDE_FRAGS_SMALL) : MF_WIDE_FN(2, WIDE_FRAGS_TINY);
 #undef MF_WIDE_FN
 #undef MF_WIDE_FN2
-        // (the matrix is not known here: one of 64 x 64 arrays; without a batch, the tiers')
-        if (n > 0 && wide_block(cfg, n, 64 * i64(cfg->cols), variant_tier(variant))) {
+        // (without a batch or the matrix, the tiers' kernels)
+        if (n > 0 && m > 0 && wide_block(cfg, n, p * cfg->cols, variant_tier(variant))) {
             fn = ks4 ? (nl ? reinterpret_cast<const void *>(&k_wide_block<4, true>)
                            : reinterpret_cast<const void *>(&k_wide_block<4, false>))
                      : (nl ? reinterpret_cast<const void *>(&k_wide_block<2, true>)
                            : reinterpret_cast<const void *>(&k_wide_block<2, false>));
             dynamic_lds = cfg->n_in * (ks4 ? 4 : 2) * 1024;
         }
-        if (n > 0 && wide_small(cfg, n, 64, 64, variant_tier(variant))) {
+        if (n > 0 && m > 0 && wide_small(cfg, n, m, p, variant_tier(variant))) {
             fn = ks4 ? (nl ? reinterpret_cast<const void *>(&k_wide_small<4, true>)
                            : reinterpret_cast<const void *>(&k_wide_small<4, false>))
                      : (nl ? reinterpret_cast<const void *>(&k_wide_small<2, true>)
@@ -2935,7 +2942,7 @@ int mf_resources_query(const mf_config *cfg, int32_t kernel_id, int64_t n, int32
                          : reinterpret_cast<const void *>(&k_general<float, 8, false, WIDE>)))
         fn = cfg->wide ? MF_GENERAL_FN(true) : MF_GENERAL_FN(false);
 #undef MF_GENERAL_FN
-        if (fp32_mfma_ok(cfg, 1, 2)) {
+        if (m > 0 ? fp32_mfma_ok(cfg, m, p) : fp32_mfma_ok(cfg, 1, 2)) {
             const bool sl = restore_planes(cfg) > 1, vn = cfg->has_vnoise != 0;
 #define MF_MFMA32_FN(ROWS)                                                                       \
     (sl ? reinterpret_cast<const void *>(&k_general_mfma32<ROWS, true, false>)                   \

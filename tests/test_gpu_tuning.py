@@ -204,3 +204,33 @@ def test_resources_follow_the_schedule(hip_device):
     say("noisy small batch", small, "unsplit", unsplit, "large", large)
     assert small["threads"] == 64 * len(noisy.weight_layout)
     assert unsplit == large and large["threads"] == 256
+
+
+def test_resources_follow_the_matrix(hip_device):
+    """With the matrix the query answers for the kernel that its read launches: k_noisy_pairs (one
+    wave per weight slice) where a small read of default arrays is split, k_noisy_block (256
+    threads) elsewhere; k_wide_small, k_wide_block (its digits in LDS) or a tier of k_noisy_wide."""
+    from memfast_amd import hip
+
+    def ask(cfg, kernel, n, arrays, partitions, **fields):
+        return hip.program(cfg, 64, 64, hip_device.index).resources(
+            cfg, 64, 64, 0, kernel=kernel, batch=n, arrays=arrays, partitions=partitions,
+            variant=hip.variant_word(**fields))
+
+    write = Nonidealities(write_variation=0.02)
+    default = Config(nonidealities=write)
+    for n, arrays, partitions, fields, threads in (
+            (64, 16, 16, {}, 512), (128, 16, 16, {}, 256), (64, 16, 16, dict(split=1), 256),
+            (64, 16, 16, dict(split=2), 512), (32, 1, 4, {}, 256), (2048, 32, 32, {}, 256)):
+        assert ask(default, 2, n, arrays, partitions, **fields)["threads"] == threads
+    sliced = Config(**INT8, nonidealities=write)   # 32768 columns are not split
+    assert ask(sliced, 2, 32, 4, 8)["threads"] == 64 * 5
+    assert ask(sliced, 2, 32, 4, 256)["threads"] == 256
+    wide = Config(activation_bits=16, weight_bits=4, input_slice=(1, 1, 2, 2, 2, 2, 2, 2, 2),
+                  weight_slice=(1, 1, 2), bw_e=8, array_size=(64, 64), rows_per_read=64,
+                  adc_bits=(6, 6, 7), nonidealities=write)
+    assert ask(wide, 3, 4, 16, 16)["threads"] == 64 * 3
+    assert ask(wide, 3, 4, 16, 16, tier=1)["threads"] == 256
+    block = ask(wide, 3, 2048, 64, 64)
+    assert block["threads"] == 256 and block["shared"] == 9 * 4 * 1024
+    assert ask(wide, 3, 2048, 64, 64, tier=1)["shared"] != block["shared"]
