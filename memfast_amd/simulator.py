@@ -416,13 +416,13 @@ class Simulator:
         budget = self.workspace_bytes
         if tuning.workspace_need(c, n, arrays, matrix.p, schedule, budget) > budget:
             raise hip.ResourceError("workspace budget")
-        kernel = tuning.read_kernel(c, n, arrays, matrix.p, budget)
+        variant = tuning.schedule_variant(schedule)
+        kernel = tuning.read_kernel(c, n, arrays, matrix.p, budget, variant)
         with torch.cuda.device(self.device):
             resource = hip.program(c, schedule["vectors"], schedule["columns"],
                                    self.device.index).resources(
                 c, schedule["vectors"], schedule["columns"], schedule["workers"], kernel=kernel,
-                variant=tuning.schedule_variant(schedule), batch=n, arrays=arrays,
-                partitions=matrix.p)
+                variant=variant, batch=n, arrays=arrays, partitions=matrix.p)
         # The output-noise MFMA read at 32-row reads keeps part of its state in scratch by
         # design (three waves per SIMD with spills run faster than two without), and its
         # registers do not depend on the schedule; the policy refuses any other spill.
@@ -742,14 +742,14 @@ class AnalogMatrix(nn.Module):
             output = self._execute_stable(q, xscale, packed, event)
         else:
             budget = (self.simulator.workspace_bytes if self.simulator.mode == "tuned" else None)
-            kernel = tuning.read_kernel(config, q.shape[0], q.shape[1], self.p, budget)
+            variant = tuning.schedule_variant(schedule)
+            kernel = tuning.read_kernel(config, q.shape[0], q.shape[1], self.p, budget, variant)
             status = hip.status_word(q.device) if status is None else status
             if not defer and self._output_bounded(q.shape[1]):
                 # The quantizer's bits are the only ones this read can leave: publish them
                 # now, and the read runs on behind the caller's next work.
                 box = self.simulator._layer_mailbox()
                 hip.status_publish(status, box)
-            variant = tuning.schedule_variant(schedule)
             # A tuned read's totals stay within the budget its schedule was admitted under.
             left = (None if budget is None else budget - tuning.workspace_need(
                 config, q.shape[0], q.shape[1], self.p, schedule, budget))

@@ -50,15 +50,15 @@ def schedule_variant(schedule):
                             schedule.get("tier", 0))
 
 
-def read_kernel(config, n, arrays, partitions, budget=None):
+def read_kernel(config, n, arrays, partitions, budget=None, variant=0):
     """The read kernel (0-3) ``hip.mm`` launches for n vectors through m x p arrays.
 
-    A block read (``hip.block_read``) whose scratch exceeds ``budget`` bytes goes to the
-    general kernel where that needs no scratch of its own."""
+    A block read (``hip.block_read``) whose scratch under the schedule word ``variant`` exceeds
+    ``budget`` bytes goes to the general kernel where that needs no scratch of its own."""
     kernel = hip.mm_kernel(config, n, arrays, partitions)
     if (budget is not None and kernel == 2 and hip.block_read(config)
             and not hip.needs_conductances(config)
-            and hip.mm_workspace_bytes(config, n, arrays, partitions, 0) > budget):
+            and hip.mm_workspace_bytes(config, n, arrays, partitions, variant) > budget):
         return 0
     return kernel
 
@@ -85,9 +85,10 @@ def workspace_need(config, n, arrays, partitions, schedule, budget=None):
     """Device bytes a read under ``schedule`` allocates besides its inputs and output: the MFMA
     kernels' scratch (mf_mm_workspace for the schedule's variant) or, for the general kernel
     with device noise, the restored conductance tensor."""
-    kernel = read_kernel(config, n, arrays, partitions, budget)
+    variant = schedule_variant(schedule)
+    kernel = read_kernel(config, n, arrays, partitions, budget, variant)
     if kernel:
-        return hip.mm_workspace_bytes(config, n, arrays, partitions, schedule_variant(schedule))
+        return hip.mm_workspace_bytes(config, n, arrays, partitions, variant)
     if not hip.needs_conductances(config):
         return 0
     rows, cols = config.array_size
@@ -116,10 +117,15 @@ class ScheduleSearch:
         self.key, self.payload = simulator._key(matrix, x, self.grid)
         self.path = simulator.cache_dir / f"{self.key}.json"
         self.record = dict(key=self.key, layer=matrix.name, shape=list(x.shape),
-                           kernel=read_kernel(simulator.config, n, arrays, matrix.p),
+                           kernel=self._kernel(default_schedule(simulator.config)),
                            cache_hit=False, candidates=[], selected=None, complete=False)
 
     # -- helpers --------------------------------------------------------------
+    def _kernel(self, schedule):
+        """The read kernel of ``schedule`` within the simulator's workspace budget."""
+        return read_kernel(self.simulator.config, self.q.shape[0], self.q.shape[1], self.matrix.p,
+                           self.simulator.workspace_bytes, schedule_variant(schedule))
+
     def _read(self, schedule):
         return self.matrix._execute(self.q, self.xscale, schedule, self.event)
 
@@ -222,7 +228,7 @@ class ScheduleSearch:
         return winner
 
     def _finish(self, winner, **fields):
-        self.record.update(selected=winner, complete=True,
+        self.record.update(selected=winner, kernel=self._kernel(winner), complete=True,
                            preparation_seconds=time.perf_counter() - self.started, **fields)
         self.simulator._selections[self.key] = winner
 

@@ -172,3 +172,16 @@ def test_tuned_read_without_samples_beyond_its_budget(hip_device, tmp_path):
     expected = Simulator(cfg, device=hip_device).mm(a.to(hip_device), b.to(hip_device))
     assert torch.equal(got.view(torch.int32), expected.view(torch.int32))
     assert tuned.report()["selections"][0]["selected"] is not None
+    assert tuned.report()["selections"][0]["kernel"] == 0
+    # A budget that only the unsplit read's scratch fits: that schedule keeps the block read.
+    n, m, p = 40, 4, 4
+    need = {z: hip.mm_workspace_bytes(cfg, n, m, p, hip.variant_word(split=z)) for z in (0, 1)}
+    assert need[1] < need[0]
+    partly = Simulator(cfg, device=hip_device, mode="tuned", cache_dir=tmp_path / "partly",
+                       workspace_mb=need[1] / 1024**2)
+    got = partly.mm(a.to(hip_device), b.to(hip_device))
+    assert torch.equal(got.view(torch.int32), expected.view(torch.int32))
+    record = partly.report()["selections"][0]
+    unsplit = [c for c in record["candidates"] if c["schedule"]["split"] == 1][0]
+    assert unsplit["status"] == "accepted" and unsplit["resources"]["threads"] == 256
+    assert record["kernel"] == (2 if record["selected"]["split"] == 1 else 0)

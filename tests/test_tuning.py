@@ -97,6 +97,23 @@ def test_split_totals_of_default_arrays_are_bounded(n, k, o):
             assert totals == n * m * p * 64 * 4
 
 
+def test_read_kernel_within_a_budget_follows_the_schedule():
+    """An ideal 128-row read leaves the MFMA read only for the schedules whose own scratch
+    exceeds the budget."""
+    cfg = Config(array_size=(128, 64), adc_bits=7, nonidealities=Nonidealities(write_variation=0.0))
+    n, m, p = 100, 4, 4
+    need = {split: hip.mm_workspace_bytes(cfg, n, m, p, hip.variant_word(split=split))
+            for split in (0, 1, 2)}
+    assert need[1] < need[2] and need[1] < need[0]
+    for budget, kernels in ((need[1] - 1, (0, 0, 0)), (need[1], (0, 2, 0)),
+                            (max(need.values()), (2, 2, 2)), (None, (2, 2, 2))):
+        for split, kernel in enumerate(kernels):
+            variant = hip.variant_word(split=split)
+            assert tuning.read_kernel(cfg, n, m, p, budget, variant) == kernel
+            scratch = tuning.workspace_need(cfg, n, m, p, dict(split=split), budget)
+            assert scratch == (need[split] if kernel else 0)
+
+
 def test_kernel_choice_has_the_extents_of_the_reads():
     """Batches beyond the MFMA reads' extents (4.2 million vectors of one array) are the general
     kernel's, which then gets restored conductances, and take none of their workspace."""
