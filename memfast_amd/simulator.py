@@ -18,6 +18,7 @@ memfast_amd/checkpoint.py.
 
 import hashlib
 import math
+import threading
 import weakref
 from dataclasses import asdict
 from functools import lru_cache
@@ -144,6 +145,28 @@ class _ProgramCache(dict):
         self[key] = _CacheEntry(weakref.ref(owner, forget), _geometry(owner), program)
 
 
+class _Mailboxes:
+    """The pinned words that calls publish their quantizers' status bits to, one per use and
+    thread: a call waits for its word before it returns.  A copy of the simulator starts
+    without any (a copied tensor is not pinned)."""
+
+    def __init__(self):
+        self._boxes = {}
+
+    def __deepcopy__(self, memo):
+        return type(self)()
+
+    def __reduce__(self):
+        return type(self), ()
+
+    def box(self, use):
+        key = use, threading.get_ident()
+        box = self._boxes.get(key)
+        if box is None:
+            box = self._boxes[key] = hip.mailbox()
+        return box
+
+
 # Dtypes whose FP32 quantization keeps finiteness, so that the device-side check of the
 # single-pass product raises exactly where a host check would.
 _SINGLE_PASS = (torch.float16, torch.bfloat16, torch.float32)
@@ -182,19 +205,11 @@ class Simulator:
         self._next_id = 0
         self._matrix_cache = _ProgramCache(self)
         self._status = None   # _product's device status word; replaced once it holds flags
-        self._mailbox = None  # pinned host word the fused route publishes its status bits to
-        self._mailbox_layers = None   # the same for layer reads (_layer_mailbox)
+        self._mailboxes = _Mailboxes()
         self._from_float = {}   # (n, k, o) -> whether hip.mm_from_float applies
         # (shape, stream, (q, xscale, workspace)) of the last fused call, written again by the
         # next call of that shape on that stream.
         self._from_float_scratch = (None, None, None)
-
-    def _layer_mailbox(self):
-        """The pinned word that layer reads of this simulator publish their quantizers'
-        status bits to (one call at a time, as the device status words)."""
-        if self._mailbox_layers is None:
-            self._mailbox_layers = hip.mailbox()
-        return self._mailbox_layers
 
     def _next_name(self):
         name = f"matrix.{self._next_id}"
@@ -345,9 +360,7 @@ class Simulator:
             # they are published to the mailbox before the read runs.
             box = None
             if config.wide and x.dtype in (torch.float32, torch.float64):
-                if self._mailbox is None:
-                    self._mailbox = hip.mailbox()
-                box = self._mailbox
+                box = self._mailboxes.box("product")
                 hip.status_publish(status, box)
             output = hip.mm(q, xscale, packed, codes_t, wscale.reshape(-1, p * config.array_size[1]),
                             config, config.seed ^ _name_tag(name), event,
@@ -380,10 +393,9 @@ class Simulator:
         last_shape, last_stream, scratch = self._from_float_scratch
         stream = hip._stream(self.device).value
         reuse = last_shape == shape and last_stream == stream
-        if self._mailbox is None:
-            self._mailbox = hip.mailbox()
+        box = self._mailboxes.box("product")
         fused = hip.mm_from_float(flat, rhs, self.config, status=status,
-                                  scratch=scratch if reuse else None, mailbox=self._mailbox)
+                                  scratch=scratch if reuse else None, mailbox=box)
         if fused is None:
             self._from_float[shape] = False
             return None
@@ -396,7 +408,7 @@ class Simulator:
         # The read publishes the quantizers' status bits when it starts.  Unless a scale is
         # large enough for an FP32 output to overflow, they are every bit of the call, and
         # the read finishes behind the caller's next work on the stream.
-        flags = hip.status_wait(self._mailbox)
+        flags = hip.status_wait(box)
         if flags is None or flags & hip.STATUS_RANGE:
             flags = int(status.item())
         return flags, tiles, q, xscale, output, kept, True, event
@@ -748,7 +760,7 @@ class AnalogMatrix(nn.Module):
             if not defer and self._output_bounded(q.shape[1]):
                 # The quantizer's bits are the only ones this read can leave: publish them
                 # now, and the read runs on behind the caller's next work.
-                box = self.simulator._layer_mailbox()
+                box = self.simulator._mailboxes.box("layer")
                 hip.status_publish(status, box)
             # A tuned read's totals stay within the budget its schedule was admitted under.
             left = (None if budget is None else budget - tuning.workspace_need(

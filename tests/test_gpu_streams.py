@@ -1,6 +1,7 @@
 """One programmed layer read on several streams and from several threads: every output is that
 of reads one after another."""
 
+import copy
 import threading
 
 import pytest
@@ -116,6 +117,39 @@ def test_threads_read_one_layer(hip_device, own_stream):
         assert len(results[index]) == 8
         for got in results[index]:
             assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+def test_copies_and_threads_have_their_own_status_words(hip_device):
+    """Fixed-scale reads return on a pinned word: a copied model's is its own and pinned, and two
+    threads' reads of one simulator do not see each other's bits."""
+    layer = layer_of("default", hip_device, k=256, o=64)
+    x = torch.randn(40, 256, generator=torch.Generator().manual_seed(9)).to(hip_device)
+    expected = layer(x)
+    product = layer.simulator.mm(x, x.T.contiguous())
+    clone = copy.deepcopy(layer)
+    assert torch.equal(clone(x).view(torch.int32), expected.view(torch.int32))
+    assert clone.simulator.mm(x, x.T.contiguous()).shape == product.shape
+    bad = x.clone()
+    bad[39, 255] = float("nan")
+    wrong = []
+
+    def work(value, raises):
+        torch.cuda.set_device(hip_device)
+        for _ in range(200):
+            try:
+                layer(value)
+                raised = False
+            except ValueError:
+                raised = True
+            if raised != raises:
+                wrong.append(raises)
+
+    threads = [threading.Thread(target=work, args=args) for args in ((x, False), (bad, True))]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not wrong
 
 
 def test_recurrent_sequences_on_two_streams(hip_device):
