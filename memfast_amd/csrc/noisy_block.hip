@@ -11,7 +11,7 @@
 // and walks the input slices over them: 2*KS MFMAs, KS LDS reads and three VALU instructions
 // per output and pair of slices.
 //
-// Terms carry a power of two, plan.k1[w] = S_w * V*Mw/unit, chosen on the host as large as the
+// Each term is two fp16, 22 bits of the FP32 conductance's 24.  Terms carry a power of two, plan.k1[w] = S_w * V*Mw/unit, chosen on the host as large as the
 // fp16 range allows: small conductances keep their low term out of fp16's subnormals, and the
 // converter takes the scale for nothing (its rounding constant and its limit are scaled by the
 // same power, which is exact).  The low terms are accumulated first,

@@ -118,9 +118,52 @@ def test_batch_beyond_the_mfma_reads(hip_device, cfg):
     assert torch.equal(got[-65:].view(torch.int32), expected.contiguous().view(torch.int32))
 
 
+def totals_in_64_bits(cfg, q, g):
+    """Slice totals [N, G, p*C] of codes ``q`` [N, m, R] read through conductances ``g``
+    [m, p, W, R, C], every product, sum and conversion in FP64."""
+    n, m, r = q.shape
+    p, c, rows = g.shape[1], g.shape[4], cfg.read_rows
+    totals = torch.zeros(n, m * r // rows, p * c, dtype=torch.float64, device=q.device)
+    codes = q.long()
+    for read in range(totals.shape[1]):
+        i, first = divmod(read * rows, r)
+        for shift, mask, in_factor in cfg.input_layout:
+            digits = ((codes[:, i, first:first + rows] >> shift) & mask).double()
+            for w, (_, w_mask, w_factor) in enumerate(cfg.weight_layout):
+                level = g[i, :, w, first:first + rows].double() - cfg.low_conductance
+                current = digits @ level.permute(1, 0, 2).reshape(rows, p * c) * cfg.read_voltage
+                counts = (current * (w_mask / cfg.current_unit)).clamp(0, cfg.adc_maxima[w]).round()
+                totals[:, read] += counts * (in_factor * w_factor)
+    return totals
+
+
+@pytest.mark.parametrize("variation", [0.02, 0.1, 0.3])
+@pytest.mark.parametrize("name", ["default", "int4_faults", "six_slices", "rows128",
+                                  "rows128_sliced"])
+def test_closer_to_64_bits_than_the_general_read(hip_device, name, variation):
+    """Programming noise puts converter arguments anywhere between two counts, and the two reads
+    round the closest ones differently: the block read's totals miss the 64-bit ones no more often
+    than the general read's.  (Both counts are of rare independent events: four standard
+    deviations of their difference.)"""
+    kwargs, effects = CASES[name]
+    cfg = Config(**kwargs, nonidealities=Nonidealities(**(effects | dict(write_variation=variation))))
+    *_, q, _, packed, packed_t, _ = programmed(cfg, 256, 512, 256, hip_device, 12)
+    n, p = q.shape[0], packed.shape[1]
+    assert hip.mm_kernel(cfg, n, q.shape[1], p) == 2
+    g = hip.restore(packed, cfg, 21, 0, 0, p)
+    expected = totals_in_64_bits(cfg, q, g[0])
+    block = hip.mm_totals(q, packed_t, cfg, 21, 0, conductance=g[0]).double().reshape_as(expected)
+    general = hip.partial(q, packed, cfg, None, 21, 0, 0, p,
+                          conductance=g).double().reshape_as(expected)
+    missed, bound = int((block != expected).sum()), int((general != expected).sum())
+    print("[block read]", name, variation, "off 64 bits:", missed, "general:", bound, "of",
+          expected.numel() * len(cfg.input_layout) * len(cfg.weight_layout), flush=True)
+    assert missed <= bound + 4 * (missed + bound) ** 0.5
+
+
 def test_reads_between_counts_keep_the_general_kernel():
-    """Read noise, drift, nonlinear converters and voltage noise put converter arguments
-    anywhere between two counts."""
+    """Read noise, drift, nonlinear converters and voltage noise: reads that have only been
+    compared with 64 bits in the general kernel's order of sums."""
     for effects in (dict(read_variation=0.01), dict(adc_nonlinearity=0.1), dict(voltage_variation=0.01),
                     dict(drift_coefficient=0.05, drift_time=100.0)):
         cfg = Config(nonidealities=Nonidealities(**(WRITE | effects)))
