@@ -46,6 +46,37 @@ def test_same_codes_as_patches(hip_device, geometry, gran):
     compare(hip_device, x, kernel, padding, cfg, fixed)
 
 
+@pytest.mark.parametrize("gran", ["fixed", (1, None), (7, 48)], ids=str)
+def test_images_beyond_32_bit_offsets(hip_device, gran):
+    """One image of more than 2^29 elements, few patches of it: taps in its first and last rows and
+    channels, padding on every side."""
+    c, h, w, kernel, stride, padding = 4, 11601, 11603, (3, 5), (5800, 5801), (1, 2)
+    assert c * h * w > 0x1FFFFFFF
+    quant = {} if gran == "fixed" else dict(input_quant_gran=gran)
+    cfg = Config(array_size=(16, 32), nonidealities=Nonidealities(write_variation=0.0), **quant)
+    x = torch.empty(1, c, h, w, device=hip_device)
+    x.normal_(generator=torch.Generator(device=hip_device).manual_seed(1))
+    out = [(e + 2 * p - k) // s + 1 for e, p, k, s in zip((h, w), padding, kernel, stride)]
+    rows = [[i * stride[0] - padding[0] + t for t in range(kernel[0])] for i in range(out[0])]
+    columns = [[j * stride[1] - padding[1] + t for t in range(kernel[1])] for j in range(out[1])]
+    assert max(map(max, rows)) >= h - 1 and max(map(max, columns)) >= w - 1
+    patches = torch.zeros(out[0], out[1], c, *kernel, device=hip_device)
+    for i, ys in enumerate(rows):
+        for j, xs in enumerate(columns):
+            for a, y in enumerate(ys):
+                for b, xx in enumerate(xs):
+                    if 0 <= y < h and 0 <= xx < w:
+                        patches[i, j, :, a, b] = x[0, :, y, xx]
+    patches = patches.reshape(out[0] * out[1], -1)
+    fixed = None
+    if gran == "fixed":
+        fixed = (torch.rand(1, patches.shape[1]) * 0.05 + 0.005).to(hip_device)
+    got, got_scale = hip.conv_input_tiles(x, cfg, (0, c, kernel, stride, padding, (1, 1), out), fixed)
+    want, want_scale = hip.input_tiles(patches, cfg, fixed)
+    assert torch.equal(got, want)
+    assert torch.equal(got_scale.view(torch.int32), want_scale.view(torch.int32))
+
+
 @pytest.mark.parametrize("bits", [3, 8])
 @pytest.mark.parametrize("scale", [2.0**-7, 0.1, 3.0, 2.0**127, 2.0**-126, 2.0**-149, 1e-38])
 def test_ties_and_extreme_scales(hip_device, scale, bits):

@@ -58,22 +58,33 @@ def test_general_mfma_read(hip_device, name, n, k, o):
     if p > 1:   # a chunk of tiles away from the first
         part = hip.partial(q, packed, cfg, None, seed, event, 1, p)
         assert torch.equal(part.view(torch.int32), expected[:, :, 1:].contiguous().view(torch.int32))
-    fused = hip.mm(q, xs, packed, packed_t, ws.reshape(-1, p * c), cfg, seed, event, k_rows=k)
     restored = oracle.execute(q.cpu(), xs.cpu(), packed.cpu(), ws.cpu(), cfg, seed, event, p * c,
                               totals=expected.cpu())
-    assert torch.equal(fused.cpu().view(torch.int32), restored.view(torch.int32))
+    for budget in (0, None):   # unsplit, and split where the rule says so
+        fused = hip.mm(q, xs, packed, packed_t, ws.reshape(-1, p * c), cfg, seed, event, k_rows=k,
+                       split_budget=budget)
+        assert torch.equal(fused.cpu().view(torch.int32), restored.view(torch.int32)), budget
 
 
-def test_general_mfma_read_order_levels(hip_device):
-    """Over 16 and 256 reads the fused cascade is the reference epilogue of the totals."""
+@pytest.mark.parametrize("reads", [17, 256, 257, 531])
+@pytest.mark.parametrize("spare", [0, 20])
+def test_general_mfma_read_order_levels(hip_device, reads, spare):
+    """Over 16 and 256 reads the cascade in the kernel (no room for totals: unsplit) and that of the
+    split read's totals are the reference epilogue of the totals; ``spare`` reads hold padding
+    alone and are not run."""
     cfg = Config(array_size=(8, 32), adc_bits=4,
                  nonidealities=Nonidealities(write_variation=0.02, read_variation=0.01))
     gen = torch.Generator().manual_seed(18)
-    a, b = torch.randn(5, 8 * 531 - 3, generator=gen), torch.randn(8 * 531 - 3, 64, generator=gen)
+    k, k_rows = 8 * (reads + spare), 8 * reads - 3
+    a, b = torch.randn(5, k, generator=gen), torch.randn(k, 64, generator=gen)
+    a[:, k_rows:] = 0.0
     q, xs = hip.input_tiles(a.to(hip_device), cfg)
     packed, packed_t, ws = hip.weight_tiles(b.T.to(hip_device), cfg)
+    assert hip.mm_workspace_bytes(cfg, 5, reads + spare, 2) > 0
     totals = hip.partial(q, packed, cfg, None, 3, 0, 0, 2)
-    fused = hip.mm(q, xs, packed, packed_t, ws.reshape(-1, 64), cfg, 3, 0)
     restored = oracle.execute(q.cpu(), xs.cpu(), packed.cpu(), ws.cpu(), cfg, 3, 0, 64,
                               totals=totals.cpu())
-    assert torch.equal(fused.cpu().view(torch.int32), restored.view(torch.int32))
+    for budget in (0, None):
+        fused = hip.mm(q, xs, packed, packed_t, ws.reshape(-1, 64), cfg, 3, 0, k_rows=k_rows,
+                       split_budget=budget)
+        assert torch.equal(fused.cpu().view(torch.int32), restored.view(torch.int32)), budget

@@ -79,6 +79,23 @@ def test_static_scratch_read_equals_mm(hip_device, kind):
             kind, call, int((got[:, :o] != expected[:, :o]).sum()))
 
 
+def test_block_read_beyond_the_scratch_runs_unsampled_counts_on_the_general_kernel(hip_device):
+    """Ideal 128-row arrays with eight weight slices at K = 33024: a 64-column chunk of terms
+    (256*W*m*R = 67.6 MB) exceeds the array, and the general kernel needs none of it."""
+    cfg = Config(array_size=(128, 64), adc_bits=7, nonidealities=Nonidealities(write_variation=0.0))
+    n, k, o = 3, 33020, 70
+    q, xscale, packed, packed_t, wscale = _operands(cfg, n, k, o, hip_device, 8)
+    m, p = q.shape[1], packed.shape[1]
+    assert hip.block_read(cfg) and hip.mm_kernel(cfg, n, m, p) == 2
+    assert 256 * 8 * m * 128 > STATIC_SCRATCH_BYTES
+    expected = hip.mm(q, xscale, packed, packed_t, wscale.reshape(-1, p * 64), cfg, 5, 0,
+                      out_cols=o, k_rows=k)
+    got, status = mm_static(q, xscale, packed, packed_t, wscale, cfg, 5, 0, o, k)
+    torch.cuda.synchronize()
+    assert int(status.item()) == 0
+    assert torch.equal(got[:, :o].view(torch.int32), expected[:, :o].view(torch.int32))
+
+
 def test_static_scratch_rejects_reads_beyond_it(hip_device):
     """Binary weights on 128-row arrays at K = 40960: one 64-column chunk of conductance
     terms (256*W*m*R = 84 MB) exceeds the 64 MiB array, so the call fails before any
