@@ -7,8 +7,10 @@ workgroup, cascades of 16 and 256 reads, small batches on k_noisy_pairs.
 
 import pytest
 import torch
+from torch import nn
 
 from memfast_amd import Config, Nonidealities, Simulator, hip
+from memfast_amd.nn import AnalogGRU
 from oracle import oracle
 from parity import check_product
 
@@ -75,6 +77,24 @@ def test_product_and_schedules(hip_device, name, n, k, o):
         assert torch.equal(output.view(torch.int32), outputs[0].view(torch.int32))
     got = Simulator(cfg, device=hip_device).mm(a.to(hip_device), b.to(hip_device))
     check_product(cfg, got, a, b, hip_device, label=f"block read {name}")
+
+
+@pytest.mark.parametrize("batch,hidden", [(3, 70), (50, 768), (300, 768)])
+def test_recurrent_sequence(hip_device, batch, hidden):
+    """A GRU's native steps on default arrays equal its cells stepped one by one: hidden reads of
+    one wave per weight slice, split over reads with the totals left to the gate kernel, and whole."""
+    torch.manual_seed(13)
+    source = nn.GRU(20, hidden).to(hip_device)
+    layer, stepped = (AnalogGRU(source, Simulator(case("default"), device=hip_device), name="gru")
+                      for _ in range(2))
+    x = torch.randn(4, batch, 20, device=hip_device)
+    got, _ = layer(x)
+    state, states = torch.zeros(batch, hidden, device=hip_device), []
+    for step in x:
+        state = stepped.cells[0](step, state)
+        states.append(state)
+    assert torch.equal(got.view(torch.int32), torch.stack(states).view(torch.int32))
+    assert layer.cells[0].hidden._event == stepped.cells[0].hidden._event == 4
 
 
 SLICED = Config(input_slice=(1, 1, 2, 2, 2), weight_slice=(1, 1, 2, 2, 2), array_size=(128, 128),

@@ -66,6 +66,26 @@ def test_general_mfma_read(hip_device, name, n, k, o):
         assert torch.equal(fused.cpu().view(torch.int32), restored.view(torch.int32)), budget
 
 
+@pytest.mark.parametrize("name", ["read_scurve", "voltage", "rows128"])
+def test_conductances_beyond_finite_currents(hip_device, name):
+    """Injected infinities, NaN and conductances whose currents overflow convert as on k_general."""
+    kwargs, effects = CASES[name]
+    cfg = Config(**kwargs, nonidealities=Nonidealities(**effects))
+    p = 2
+    gen = torch.Generator().manual_seed(19)
+    k, o = 100, 2 * cfg.array_size[1]
+    q, _ = hip.input_tiles(torch.randn(40, k, generator=gen).to(hip_device), cfg)
+    packed, _, _ = hip.weight_tiles(torch.randn(o, k, generator=gen).to(hip_device), cfg)
+    g = hip.restore(packed, cfg, 6, 0, 0, p)
+    flat = g.view(-1)
+    strange = torch.tensor([float("inf"), float("-inf"), float("nan"), 3e38, -3e38, 1e30, 0.0, -1e-5])
+    at = torch.randperm(flat.numel(), generator=gen)[:flat.numel() // 50].to(hip_device)
+    flat[at] = strange.to(hip_device)[torch.arange(at.numel(), device=hip_device) % 8]
+    expected, _ = hip.partial(q, packed, cfg, None, 6, 0, 0, p, conductance=g, codes=True)
+    got = hip.partial(q, packed, cfg, None, 6, 0, 0, p, conductance=g)
+    assert torch.equal(got.view(torch.int32), expected.view(torch.int32))
+
+
 @pytest.mark.parametrize("reads", [17, 256, 257, 531])
 @pytest.mark.parametrize("spare", [0, 20])
 def test_general_mfma_read_order_levels(hip_device, reads, spare):
