@@ -294,7 +294,9 @@ int mf_status_wait(const uint32_t *mailbox, int64_t timeout_us, uint32_t *flags,
  *  - A read whose least scratch exceeds the array (the ideal-device read's digit
  *    masks, ceil(n/64)*G*8 + ceil(p*C/32)*G*8 bytes rounded up to 256; or one
  *    64-column chunk of noisy conductance terms, 256*W*m*R bytes) fails with
- *    MF_E_RESOURCE before launching anything. */
+ *    MF_E_RESOURCE before launching anything, except 128-row reads, and 64-row
+ *    reads of more than five input slices, whose conductances need no sampling:
+ *    they run on the general kernel, which takes none of the array. */
 #define MF_STATIC_SCRATCH_BYTES (64ll << 20)
 int mf_mm_static(const mf_config *cfg, const uint8_t *q, const float *xscale, int64_t n,
                  int64_t m, const uint8_t *packed, const uint8_t *packed_t, const float *wscale,
@@ -501,7 +503,8 @@ int mf_profile_collect(int64_t *launches, double *milliseconds);
  * the conductance terms of every column plus a split read's integer totals
  * (noisy devices; a smaller workspace of at least 64 columns' worth makes mf_mm
  * work in column chunks, unsplit), or 16-bit input codes and terms (wide
- * codes).  0 when the general kernel is used. */
+ * codes), or the totals through which the general kernel splits a small read over
+ * blocks (0 where it does not; mf_mm runs it unsplit without them). */
 int mf_mm_workspace(const mf_config *cfg, int64_t n, int64_t m, int64_t p, int32_t variant,
                     int64_t *bytes);
 

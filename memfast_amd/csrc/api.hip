@@ -292,8 +292,8 @@ bool plain_read(const mf_config *cfg) {
     return !cfg->has_vnoise && !(cfg->has_read && cfg->read_mode != MF_READ_SHARED);
 }
 // Reads that k_noisy_block (noisy_block.hip) takes: 64-row reads with more input slices than
-// k_noisy's registers hold, and 128-row reads, of linear converters under programming noise and
-// stuck-at faults alone (programming_only).  Its terms hold 22 bits where the general read
+// k_noisy's registers hold, and 128-row reads; of them, linear converters under programming noise
+// and stuck-at faults alone (programming_only).  Its terms hold 22 bits where the general read
 // multiplies 24, and it sums in another order, so the conversions closest to a tie round another
 // way.  Against 64 bits it is the closer of the two: it misses none of 6.7e7 conversions of the
 // default arrays at 2% programming noise (the general read none), 8.5e-7 of them at 10% (1.0e-6) and
@@ -1086,11 +1086,13 @@ int launch_general(const mf_config *cfg, const GeneralArgs &args, int out_kind, 
 }
 
 // FP32 currents run on FP32 MFMA (k_general_mfma32, the same bits) for narrow codes without
-// output-mode read noise (or slice_pair noise with voltage variation, which spills): reads of at most 128 rows, cascade columns, totals in 32 bits, and
-// products of voltage and conductance far from FP32's subnormals.  `p`: tiles of the matrix.
+// output-mode read noise (or slice_pair noise with voltage variation, which spills): reads of at
+// most 128 rows, cascade columns, totals in 32 bits, and products of voltage and conductance far
+// from FP32's subnormals.  `p`: tiles of the matrix.
 static bool fp32_mfma_ok(const mf_config *cfg, i64 m, i64 p) {
     return !cfg->wide && !cfg->precise && !(cfg->has_read && cfg->read_mode == MF_READ_OUTPUT) &&
-           !(cfg->has_vnoise && restore_planes(cfg) > 1) && cfg->read_rows <= 128 && cfg->n_in <= 8 && cfg->n_w <= 8 && m * cfg->reads < 4096 &&
+           !(cfg->has_vnoise && restore_planes(cfg) > 1) && cfg->read_rows <= 128 &&
+           cfg->n_in <= 8 && cfg->n_w <= 8 && m * cfg->reads < 4096 &&
            all_cascade_columns(cfg->cols, p) && totals_bound(cfg) < 2147483647.0 &&
            double(cfg->f_low) * double(cfg->f_voltage) > 1e-25 && largest_delta(cfg) < 1e18;
 }
@@ -1181,12 +1183,14 @@ static int launch_general_mfma64(const mf_config *cfg, const GeneralArgs &args, 
 // applies and no per-pair codes are asked for, else on k_general.
 static int launch_general_read(const mf_config *cfg, const GeneralArgs &args, int out_kind,
                                hipStream_t s, void *workspace = nullptr, i64 bytes = 0) {
-    const i64 scratch = out_kind == OUT_FUSED && workspace ? mfma32_scratch(cfg, args.n, args.m, args.p) : 0;
+    const i64 scratch =
+        out_kind == OUT_FUSED && workspace ? mfma32_scratch(cfg, args.n, args.m, args.p) : 0;
     if (scratch > 0 && scratch <= bytes) {
         // Chunks of reads write totals; the epilogue restores and sums them in torch's order.
         GeneralArgs part = args;
         part.out = workspace;
-        if (launch_general_mfma32(cfg, part, OUT_TOTALS, s, mfma32_split(cfg, args.n, args.m, args.p))) {
+        const i64 split = mfma32_split(cfg, args.n, args.m, args.p);
+        if (launch_general_mfma32(cfg, part, OUT_TOTALS, s, split)) {
             const i64 ncols = args.p * cfg->cols, G = args.m * cfg->reads;
             hipLaunchKernelGGL(k_restore_sum_f32, dim3(grid_for(args.n * ncols)), dim3(256), 0, s,
                                static_cast<const float *>(workspace), args.n, G, args.g_run, ncols,

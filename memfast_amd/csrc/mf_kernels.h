@@ -220,14 +220,14 @@ __global__ void k_split_conductances(const mf_config cfg, const u8 *packed_t, co
                                      i64 CB, const NoisyPlan plan, uint4 *gs);
 template <int KS, int NA, bool NONLINEAR, bool VNOISE, bool SLICE, bool OUTN>
 __global__ void k_noisy(const NoisyPlan plan, const NoisyArgs args);
-// Split read of batches of at most 32 vectors: block = one wave per weight slice on 32
-// vectors x 32 columns and one read (grid: column blocks, vector blocks, reads); writes
-// slice totals [n, G, ldo], or with args.restored the restored (float(T) * xs) * ws
-// (plain and S-curve reads).
 // The read of digits in LDS (noisy_block.hip): block = up to 4 waves on the same 32 vectors,
 // 32 columns per wave; n_in * KS KiB of dynamic LDS.
 template <int KS>
 __global__ void k_noisy_block(const NoisyPlan plan, const NoisyArgs args);
+// Small split reads (pairs_read in api.hip: at most 32 vectors, or few waves of k_noisy_block):
+// block = one wave per weight slice on 32 vectors x 32 columns and one read (grid: column
+// blocks, vector blocks, reads); writes slice totals [n, G, ldo], or with args.restored the
+// restored (float(T) * xs) * ws (plain and S-curve reads).
 template <int KS, int NA, bool NONLINEAR>
 __global__ void k_noisy_pairs(const NoisyPlan plan, const NoisyArgs args);
 // Input operands of a read with voltage variation (memfast/reference.py:77-82): per

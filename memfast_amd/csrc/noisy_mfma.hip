@@ -620,9 +620,9 @@ __device__ __forceinline__ void noisy_read(const NoisyPlan &plan, const NoisyArg
     if (!finite && args.status) atomicOr(args.status, u32(MF_STATUS_OUTPUT));
 }
 
-// Split reads of small batches (at most 32 vectors): one workgroup per (32-column block,
-// read) with one wave per weight slice, so a read's 25 pairs (config 3) run on five waves
-// at once instead of one after another.  Each wave loads its weight slice's terms once (a
+// Small split reads (pairs_read in api.hip): one workgroup per (32-column block, 32 vectors,
+// read) with one wave per weight slice, so a read's 25 pairs (five by five slices) run on five
+// waves at once instead of one after another.  Each wave loads its weight slice's terms once (a
 // block reads every term of its read once) and converts its pairs with every input slice,
 // whose digits it builds from the read's codes (fa*fw*(0x400000 + code) modulo 2^32, as
 // noisy_read); the waves add their words in LDS (integer sums: any order gives the same
