@@ -901,7 +901,7 @@ def mm(q, xscale, packed, packed_t, wscale, config, seed, event, *, conductance=
         size = mm_workspace_bytes(config, n, m, p, variant & ~REUSE_TERMS)
         if terms is not None:
             size -= mm_terms_bytes(config, m, p)
-            workspace = torch.empty(max(1, size), dtype=torch.uint8, device=q.device)
+            workspace = torch.empty(size, dtype=torch.uint8, device=q.device) if size else None
         elif workspace is None:
             workspace = torch.empty(max(1, size), dtype=torch.uint8, device=q.device)
             reuse_terms = False

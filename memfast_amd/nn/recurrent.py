@@ -392,9 +392,11 @@ def _native_steps(cell, projected, order, hidden):
                                   matrix.packed, codes_t, matrix.weight_scale.reshape(-1, columns),
                                   bias, matrix.seed, matrix._event, reverse=order[0] > order[-1],
                                   status=status, terms=terms, reuse_terms=reuse)
-        if keeps and not reuse:
-            matrix._kept.queued(source)
-    if int(status.item()):
+        sampled = matrix._kept.queued(source, waits=True) if keeps and not reuse else None
+    flags = int(status.item())
+    if sampled is not None:
+        matrix._kept.settled(sampled)
+    if flags:
         return None
     matrix._event += len(order)
     return states, states[order[-1]]

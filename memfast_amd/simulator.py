@@ -749,7 +749,7 @@ class AnalogMatrix(nn.Module):
         packed = self.packed
         if not config.wide and packed.dtype != torch.uint8:
             packed = packed.to(torch.uint8)
-        box = None
+        box = sampled = None
         if stable:
             output = self._execute_stable(q, xscale, packed, event)
         else:
@@ -775,7 +775,7 @@ class AnalogMatrix(nn.Module):
                                 terms=terms, reuse_terms=reuse, split_budget=left,
                                 out_cols=self.out_features, k_rows=self.in_features)
                 if keeps and not reuse:
-                    self._kept.queued(source)
+                    sampled = self._kept.queued(source, waits=box is None and not defer)
         # An FP32 read's bias goes through a kernel that also flags non-finite sums and drops
         # the array columns past the layer's.
         checked_bias = (self.bias is not None and self.zero_correction is None
@@ -803,6 +803,8 @@ class AnalogMatrix(nn.Module):
             if flags == 0:
                 return output, _BOUNDED
         flags = int(status.item())   # the one status read: deferred input check, then outputs
+        if sampled is not None:
+            self._kept.settled(sampled)
         if flags & hip.STATUS_INPUT:
             raise ValueError(input_error or "quantized values must be finite")
         flagged = bool(flags & hip.STATUS_OUTPUT)
@@ -857,8 +859,11 @@ class AnalogMatrix(nn.Module):
         (memfast/reference.py:36-46), so those samples are identical on every read
         of a programmed matrix and need not be drawn again."""
         source = (codes_t, codes_t._version, self.seed)
+        held = self._kept.held(device, source)
+        if held is not None:
+            return held, True, source
         need = hip.mm_terms_bytes(self.config, arrays, self.p)
-        return *self._kept.take(need, device, source), source
+        return self._kept.fresh(need, device), False, source
 
     def _execute_stable(self, q, xscale, packed, event):
         """FP64 overflow-safe restore of the slice totals (non-finite FP32 retry).

@@ -61,10 +61,14 @@ CPU = torch.device("cpu")
 
 
 def sampled(terms, codes, seed=1):
-    buffer, reuse = terms.take(64, CPU, (codes, codes._version, seed))
-    if not reuse:
-        terms.queued((codes, codes._version, seed))
-    return buffer, reuse
+    """(buffer, whether it held the terms) of a read, which samples them otherwise."""
+    source = (codes, codes._version, seed)
+    held = terms.held(CPU, source)
+    if held is not None:
+        return held, True
+    buffer = terms.fresh(64, CPU)
+    terms.queued(source, waits=False)
+    return buffer, False
 
 
 def test_another_stream_waits_for_the_samples(device):
@@ -108,11 +112,41 @@ def test_new_samples_leave_terms_in_use_alone(device):
 def test_terms_are_not_held_until_their_read_is_queued(device):
     terms, codes = kept.KeptTerms(), torch.zeros(4)
     source = (codes, codes._version, 1)
-    assert terms.take(64, CPU, source)[1] is False     # (its read raised)
-    assert terms.take(64, CPU, source)[1] is False
-    terms.queued(source)
-    assert terms.take(64, CPU, source)[1] is True
-    assert terms.take(64, CPU, (codes, codes._version, 2))[1] is False
+    assert terms.held(CPU, source) is None
+    buffer = terms.fresh(64, CPU)      # (the read that follows raises)
+    assert terms.held(CPU, source) is None and terms.fresh(64, CPU) is buffer
+    terms.queued(source, waits=False)
+    assert terms.held(CPU, source) is buffer
+    assert terms.held(CPU, (codes, codes._version, 2)) is None
+    assert terms.held(torch.device("meta"), source) is None
+
+
+def test_a_read_that_its_call_waits_for_is_recorded_only_in_between(device):
+    terms, codes = kept.KeptTerms(), torch.zeros(4)
+    source = (codes, codes._version, 1)
+    first = terms.fresh(64, CPU)
+    number = terms.queued(source, waits=True)
+    writer = device.stream()
+    assert terms._written._event is None
+    device.use(2)                      # another thread's read, before the call has waited
+    assert terms.held(CPU, source) is first
+    event = terms._written._event
+    assert event.recorded == [writer] and device.stream().waited == [event]
+    terms.settled(number)
+    device.use(3)
+    assert terms.held(CPU, source) is first and not device.stream().waited
+    device.use(1)
+    codes.add_(1)
+    source = (codes, codes._version, 1)
+    terms.fresh(64, CPU)
+    later = terms.queued(source, waits=True)
+    assert later != number
+    terms.settled(number)              # (the earlier call again)
+    device.use(4)
+    terms.held(CPU, source)
+    assert len(device.stream().waited) == 1
+    terms.settled(later)
+    del device.used[:]
 
 
 def test_codes_built_on_one_stream_are_waited_for_on_another(device):
