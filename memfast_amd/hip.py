@@ -242,7 +242,8 @@ def check(status, operation):
 
 
 def _ptr(tensor):
-    return ct.c_void_p(tensor.data_ptr()) if tensor is not None else None
+    """The tensor's device address for a c_void_p argument (None stays NULL)."""
+    return tensor.data_ptr() if tensor is not None else None
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
