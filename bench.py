@@ -38,7 +38,7 @@ HBM_PEAK_GBS = 8000.0
 # runs.  Summaries and commands: profiles/k_ideal_config2_pmc.md and
 # profiles/k_noisy_config2_noisy_pmc.md.  Only valid for the kernel sources they were
 # measured on (hash prefix below); otherwise the bench reports null.
-MEASURED_TRAFFIC = dict(kernels="99c076a9c35b3c25", ideal=298554125, noisy=2052971964)
+MEASURED_TRAFFIC = dict(kernels="444dba0d729dbbfd", ideal=298583144, noisy=2052131810)
 
 
 def measured_traffic(leg):

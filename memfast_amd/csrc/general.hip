@@ -276,17 +276,18 @@ __global__ __launch_bounds__(256) void k_general(const mf_config cfg, const Gene
 //
 // Block: 32 vectors x 32 columns, a wave per weight slice (two from five slices on where two
 // blocks then fit a CU: one's staging and converters run under the other's sums, 13.8 against
-// 14.9 ms at 2048^3 on one box).  Per read the block stages the voltages of every input slice in
+// 14.9 ms at 2048^3 on one card).  Per read the block stages the voltages of every input slice in
 // LDS in operand order (a lane's float4 is four steps of two rows; its digit's voltage comes from
-// a small table, computed once); a wave loads its slice's conductances from global memory eight rows ahead and holds
-// the currents of four input slices at a time, 16 registers each (eight at a time spilled).
+// a small table, computed once); a wave loads its slice's conductances from global memory eight
+// rows ahead and holds the currents of four input slices at a time, 16 registers each (eight at a
+// time spilled).
 // After the converters the waves' totals meet in LDS, and each restores and sums the outputs
 // r = wave, wave + waves, ..
 // Why: k_general spends an LDS read per two FMAs and reaches 4.2 TFMA/s.  Bound: FP32 MFMA
 // (69 TFMA/s measured back to back on this card), with the converters (5 VALU instructions per
 // output and pair, 11 with the S-curve) partly under it.  Default Config, 2048^3, read noise and
-// S-curve: 13.4-13.8 ms from box to box (41 TFMA/s), 134 ms on k_general; 600x900 inputs and 500 columns with
-// slice_pair noise: 1.1 ms against 22.5.
+// S-curve: 13.4-13.8 ms from card to card (41 TFMA/s), 134 ms on k_general; 600x900 inputs and
+// 500 columns with slice_pair noise: 1.1 ms against 22.5.
 typedef float v16fg __attribute__((ext_vector_type(16)));
 
 template <int ROWS, bool SLICE, bool VNOISE>
